@@ -22,12 +22,16 @@ struct cgd_ctx {
   int thomas = 0;  // column solve: 0 = cyclic reduction, 1 = serial Thomas (CGD_THOMAS=1)
   int ntr = 0;     // tracers (components 5..4+ntr of the state arrays, 0-based)
   int ncolor = 0;
-  std::vector<int> color_off;  // first element slot of each colour (elements are stored in colour order)
+  std::vector<int> color_off;  // first entry of each colour in the colour list
   int *d_glob = nullptr;       // [NF][NN] 0-based
-  int *d_slot = nullptr;       // element -> slot (colour order), set-up only
+  int *d_clist = nullptr;      // elements by colour, ascending within one
+  int *d_cpy = nullptr, *d_gcpy = nullptr;  // the copies of each element node / global node, colour order
+  double *d_e1 = nullptr, *d_e2 = nullptr;  // element copies of the pass-1 cache and of the tendency (5 each)
   double *d_met = nullptr, *d_met1 = nullptr, *d_ms = nullptr, *d_bwork = nullptr;
   double *d_metn = nullptr, *d_met1n = nullptr;  // compact metric layout: per element node
   int cm = 0;                                    // 1: compact metric layout
+  int reg = 0;                                   // 1: regular compact metric (k_fcn2r)
+  double *d_iMn = nullptr;                       // regular metric: 1/(M1+M2) per node
   int mixed = 0;                                 // 1: mixed-precision cgd_rw_step
   int smooth = 0;                                // 1: kink-smoothed upwind flux (SmoothW or SmoothC > 0)
   float *d_ims32 = nullptr;                      // 1/(M1+M2) in FP32 (mixed precision)
@@ -35,10 +39,10 @@ struct cgd_ctx {
   float *d_metp32 = nullptr;                     // compact per-point metric in FP32 (mixed precision)
   double *d_f4x = nullptr;     // [NF][NN][nchunk] chunk-bottom F4 terms
   int *d_nptr = nullptr, *d_ncopy = nullptr;  // global node -> element copies (colour order)
-  double *d_kvis = nullptr;    // [slot][3] hyperviscosity coefficients
-  // HorLimit: each slot's stencil (itself and the elements sharing a node,
-  // 13 slot numbers), the element bounds of the mixing ratios
-  // [tracer][slot][Nz], and the stage time step (dtauStage)
+  double *d_kvis = nullptr;    // [element][3] hyperviscosity coefficients
+  // HorLimit: each element's stencil (itself and the elements sharing a node,
+  // 13 element numbers), the element bounds of the mixing ratios
+  // [tracer][element][Nz], and the stage time step (dtauStage)
   int horlimit = 0;
   double dtau = 0.0;
   // the checkpoints that cgd_rw_forward_ckpt left in a work array, for the
@@ -61,11 +65,9 @@ struct cgd_ctx {
   int colw = 64, colblock = 256;
   int items1 = 1;  // pass-1 work items (element, level chunk) per workgroup: 1 or 2
   // one persistent launch per RW stage (k_stage_persist): on/off, its grid
-  // (workgroups resident at once), the colour offsets on the device, the
-  // grid barrier's state and wait bound
+  // (workgroups resident at once), the grid barrier's state and wait bound
   int persistent = 0;
   int pgrid = 0;
-  int *d_coff = nullptr;
   GridBar *d_bar = nullptr;
   long long bar_ticks = 0;
   // captured step graph (cgd_rw_graph_create)
@@ -99,6 +101,12 @@ template <typename R> static size_t lds_fcn2(const cgd_ctx *c) {
   const size_t base = sizeof(double) * (c->NN + c->NN * c->nzt);
   if (std::is_same<R, double>::value) return base + r;
   return base + (r + 7) / 8 * 8 + sizeof(double) * (c->NN + 3 * c->NN * c->nzt);
+}
+
+// k_fcn2r: D, DW, 12 tiles, four tiles with the level below, its sums, the
+// horizontal metric and 1/(2 M)
+static size_t lds_fcn2r(const cgd_ctx *c) {
+  return sizeof(double) * (2 * c->NN + 12 * c->NN * c->nzt + 4 * c->NN * (c->nzt + 1) + 7 * c->NN);
 }
 
 static int fail(cgd_ctx *c, int code, const std::string &msg) {
@@ -448,15 +456,15 @@ static int ctx_build(cgd_ctx *c, const cgd_desc *ds, int nmem, hipStream_t st) {
   c->color_off.assign(ncol + 1, 0);
   for (int e = 0; e < NF; ++e) c->color_off[color[e] + 1]++;
   for (int k = 0; k < ncol; ++k) c->color_off[k + 1] += c->color_off[k];
-  // slot order: colour, then member, then element number within the member
+  // elements are stored in the caller's order (neighbours lie close, so the
+  // nodes they share are read again while cached); elist: colour by colour,
+  // then member, then element number within the member
   std::vector<int> elist(NF);
   {
     std::vector<int> fp(c->color_off.begin(), c->color_off.end() - 1);
     for (int e = 0; e < NF; ++e) elist[fp[color[e]]++] = e;
   }
-  std::vector<int> slot(NF);
-  for (int q = 0; q < NF; ++q) slot[elist[q]] = q;
-  // global node -> element copies (slot*NN + node) in colour order
+  // global node -> element copies (e*NN + node) in colour order
   std::vector<int> cptr(NumG + 1, 0), ccopy((size_t)NF * NN);
   for (int v : g32) cptr[v + 1]++;
   for (int i = 0; i < NumG; ++i) cptr[i + 1] += cptr[i];
@@ -464,24 +472,32 @@ static int ctx_build(cgd_ctx *c, const cgd_desc *ds, int nmem, hipStream_t st) {
     std::vector<int> fp(cptr.begin(), cptr.end() - 1);
     for (int q = 0; q < NF; ++q) {
       const int e = elist[q];
-      for (int i = 0; i < NN; ++i) ccopy[fp[g32[(size_t)e * NN + i]]++] = q * NN + i;
+      for (int i = 0; i < NN; ++i) ccopy[fp[g32[(size_t)e * NN + i]]++] = e * NN + i;
     }
   }
-  // numbering by slot, bit 31 marking the first copy of each node
-  std::vector<int> gslot((size_t)NF * NN);
-  for (int q = 0; q < NF; ++q)
-    for (int i = 0; i < NN; ++i) gslot[(size_t)q * NN + i] = g32[(size_t)elist[q] * NN + i];
+  // the same as fixed-width lists (an even number of entries, -1 past the
+  // last copy), per global node and per element node
+  int mult = 4;
+  for (int gn = 0; gn < NumG; ++gn) mult = std::max(mult, cptr[gn + 1] - cptr[gn]);
+  const int cpw = (mult + 1) / 2 * 2;
+  std::vector<int> gcpy((size_t)NumG * cpw, -1), cpy((size_t)NF * NN * cpw, -1);
+  for (int gn = 0; gn < NumG; ++gn)
+    std::copy(ccopy.begin() + cptr[gn], ccopy.begin() + cptr[gn + 1], gcpy.begin() + (size_t)gn * cpw);
+  for (size_t i = 0; i < g32.size(); ++i)
+    std::copy_n(gcpy.begin() + (size_t)g32[i] * cpw, cpw, cpy.begin() + i * cpw);
+  // numbering, bit 31 marking the first copy of each node
+  std::vector<int> gslot = g32;
   for (int gn = 0; gn < NumG; ++gn)
     if (cptr[gn + 1] > cptr[gn]) gslot[ccopy[cptr[gn]]] |= (int)0x80000000u;
-  // hyperviscosity per slot (the member's coefficients)
+  // hyperviscosity per element (the member's coefficients)
   std::vector<double> kvis((size_t)NF * 3);
   for (int m = 0; m < nmem; ++m)
     for (int e = c->mem_e0[m]; e < c->mem_e0[m + 1]; ++e) {
-      kvis[(size_t)slot[e] * 3] = ds[m].HyperDCurl;
-      kvis[(size_t)slot[e] * 3 + 1] = ds[m].HyperDGrad;
-      kvis[(size_t)slot[e] * 3 + 2] = ds[m].HyperDDiv;
+      kvis[(size_t)e * 3] = ds[m].HyperDCurl;
+      kvis[(size_t)e * 3 + 1] = ds[m].HyperDGrad;
+      kvis[(size_t)e * 3 + 2] = ds[m].HyperDDiv;
     }
-  // HorLimit: the stencil of every slot (FE.Stencil, NumberingFem.jl:133-157:
+  // HorLimit: the stencil of every element (FE.Stencil, NumberingFem.jl:133-157:
   // the element and those sharing a grid node with it, padded with itself)
   c->horlimit = d->HorLimit != 0;
   std::vector<int> stencil;
@@ -490,10 +506,10 @@ static int ctx_build(cgd_ctx *c, const cgd_desc *ds, int nmem, hipStream_t st) {
     element_adjacency(g32, NN, NF, NumG, aptr, adj);
     stencil.assign((size_t)NF * 13, 0);
     for (int e = 0; e < NF; ++e) {
-      const int q = slot[e];
+      const int q = e;
       if (aptr[e + 1] - aptr[e] > 12) return fail(c, CGD_ERR_ARG, "HorLimit: an element has more than 12 neighbours");
       for (int k = 0; k < 13; ++k) stencil[(size_t)q * 13 + k] = q;
-      for (int k = aptr[e]; k < aptr[e + 1]; ++k) stencil[(size_t)q * 13 + 1 + (k - aptr[e])] = slot[adj[k]];
+      for (int k = aptr[e]; k < aptr[e + 1]; ++k) stencil[(size_t)q * 13 + 1 + (k - aptr[e])] = adj[k];
     }
     std::vector<double> wg(c->N);
     HIPCHK(c, hipMemcpyAsync(wg.data(), d->w, c->N * sizeof(double), hipMemcpyDeviceToHost, st));
@@ -507,7 +523,11 @@ static int ctx_build(cgd_ctx *c, const cgd_desc *ds, int nmem, hipStream_t st) {
   const size_t ng = (size_t)NumG * Nz;
   const int nchunk_max = (Nz + 7) / 8;
   HIPCHK(c, hipMalloc(&c->d_glob, gslot.size() * sizeof(int)));
-  HIPCHK(c, hipMalloc(&c->d_slot, (size_t)NF * sizeof(int)));
+  HIPCHK(c, hipMalloc(&c->d_clist, (size_t)NF * sizeof(int)));
+  HIPCHK(c, hipMalloc(&c->d_cpy, cpy.size() * sizeof(int)));
+  HIPCHK(c, hipMalloc(&c->d_gcpy, gcpy.size() * sizeof(int)));
+  HIPCHK(c, hipMalloc(&c->d_e1, npt * 5 * sizeof(double)));
+  HIPCHK(c, hipMalloc(&c->d_e2, npt * 5 * sizeof(double)));
   HIPCHK(c, hipMalloc(&c->d_met, npt * CGD_NMET * sizeof(double)));
   HIPCHK(c, hipMalloc(&c->d_met1, npt * CGD_NMET1 * sizeof(double)));
   HIPCHK(c, hipMalloc(&c->d_ms, ng * sizeof(double)));
@@ -519,7 +539,9 @@ static int ctx_build(cgd_ctx *c, const cgd_desc *ds, int nmem, hipStream_t st) {
   HIPCHK(c, hipMemcpyAsync(c->d_nptr, cptr.data(), cptr.size() * sizeof(int), hipMemcpyHostToDevice, st));
   HIPCHK(c, hipMemcpyAsync(c->d_ncopy, ccopy.data(), ccopy.size() * sizeof(int), hipMemcpyHostToDevice, st));
   HIPCHK(c, hipMemcpyAsync(c->d_glob, gslot.data(), gslot.size() * sizeof(int), hipMemcpyHostToDevice, st));
-  HIPCHK(c, hipMemcpyAsync(c->d_slot, slot.data(), slot.size() * sizeof(int), hipMemcpyHostToDevice, st));
+  HIPCHK(c, hipMemcpyAsync(c->d_clist, elist.data(), elist.size() * sizeof(int), hipMemcpyHostToDevice, st));
+  HIPCHK(c, hipMemcpyAsync(c->d_cpy, cpy.data(), cpy.size() * sizeof(int), hipMemcpyHostToDevice, st));
+  HIPCHK(c, hipMemcpyAsync(c->d_gcpy, gcpy.data(), gcpy.size() * sizeof(int), hipMemcpyHostToDevice, st));
   HIPCHK(c, hipMemcpyAsync(c->d_kvis, kvis.data(), kvis.size() * sizeof(double), hipMemcpyHostToDevice, st));
   if (c->horlimit) {
     const size_t nb = (size_t)c->ntr * NF * Nz;
@@ -580,7 +602,7 @@ static int ctx_build(cgd_ctx *c, const cgd_desc *ds, int nmem, hipStream_t st) {
   for (int m = 0; m < nmem; ++m) {
     const size_t nptm = (size_t)ds[m].NF * NN * Nz;
     hipLaunchKernelGGL(k_relayout_metric, dim3(grid_for(nptm, 256)), dim3(256), 0, st, ds[m].dXdxI, ds[m].J,
-                       ds[m].X, c->d_slot + c->mem_e0[m], c->d_met, c->d_met1, NN, Nz, ds[m].NF, d->Omega);
+                       ds[m].X, (size_t)c->mem_e0[m], c->d_met, c->d_met1, NN, Nz, ds[m].NF, d->Omega);
     HIPCHK(c, hipGetLastError());
   }
   hipLaunchKernelGGL(k_msum, dim3(grid_for(ng, 256)), dim3(256), 0, st, c->M, c->d_ms, ng);
@@ -620,6 +642,18 @@ static int ctx_build(cgd_ctx *c, const cgd_desc *ds, int nmem, hipStream_t st) {
       c->d_met = metp;
       c->d_met1 = nullptr;
       c->cm = 1;
+      // regular (CGD_METRIC=compact keeps the general kernel)
+      int *d_bad = nullptr, bad = 1;
+      HIPCHK(c, hipMalloc(&d_bad, sizeof(int)));
+      HIPCHK(c, hipMalloc(&c->d_iMn, (size_t)NumG * sizeof(double)));
+      HIPCHK(c, hipMemsetAsync(d_bad, 0, sizeof(int), st));
+      hipLaunchKernelGGL(k_met_regular, dim3(2048), dim3(256), 0, st, c->d_metn, c->d_met, c->M, c->d_ms, NF, NN, NumG,
+                         Nz, c->d_iMn, d_bad);
+      HIPCHK(c, hipGetLastError());
+      HIPCHK(c, hipMemcpyAsync(&bad, d_bad, sizeof(int), hipMemcpyDeviceToHost, st));
+      HIPCHK(c, hipStreamSynchronize(st));
+      HIPCHK(c, hipFree(d_bad));
+      c->reg = !bad && !(ev && strcmp(ev, "compact") == 0);
     }
   }
   if (c->mixed) {
@@ -656,6 +690,11 @@ static int ctx_build(cgd_ctx *c, const cgd_desc *ds, int nmem, hipStream_t st) {
       a.DWm[i * c->N + k] = hdw[i + c->N * k];
     }
   a.glob = c->d_glob;
+  a.clist = c->d_clist;
+  a.cpy = c->d_cpy;
+  a.gcpy = c->d_gcpy;
+  a.cpw = cpw;
+  a.ecs = npt;
   a.met = c->d_met;
   a.metn = c->d_metn;
   a.met1n = c->d_met1n;
@@ -665,16 +704,14 @@ static int ctx_build(cgd_ctx *c, const cgd_desc *ds, int nmem, hipStream_t st) {
   a.M32 = c->d_m32;
   a.metp32 = c->d_metp32;
   a.M = c->M;
+  a.iMn = c->reg ? c->d_iMn : nullptr;
   a.kvis = c->d_kvis;
   a.iv = d->State == CGD_MOIST ? d->RhoVPos - 1 : -1;
   a.ic = d->State == CGD_MOIST ? d->RhoCPos - 1 : -1;
   a.Cpv = d->Cpv;
   a.Cpl = d->Cpl;
   a.Rv = d->Rv;
-  // persistent stage launches: colour offsets and the grid barrier (zero)
-  HIPCHK(c, hipMalloc(&c->d_coff, c->color_off.size() * sizeof(int)));
-  HIPCHK(c, hipMemcpyAsync(c->d_coff, c->color_off.data(), c->color_off.size() * sizeof(int), hipMemcpyHostToDevice,
-                           st));
+  // persistent stage launches: the grid barrier (zero)
   HIPCHK(c, hipMalloc(&c->d_bar, sizeof(GridBar)));
   HIPCHK(c, hipMemsetAsync(c->d_bar, 0, sizeof(GridBar), st));
   HIPCHK(c, hipStreamSynchronize(st));
@@ -718,11 +755,11 @@ extern "C" int cgd_ctx_destroy(cgd_ctx *c) {
   if (c->gstream) (void)hipStreamDestroy(c->gstream);
   for (void *p : {(void *)c->d_stencil, (void *)c->d_qmin, (void *)c->d_qmax})
     if (p) (void)hipFree(p);
-  for (void *p : {(void *)c->d_glob, (void *)c->d_slot, (void *)c->d_met, (void *)c->d_met1, (void *)c->d_metn,
+  for (void *p : {(void *)c->d_glob, (void *)c->d_clist, (void *)c->d_cpy, (void *)c->d_gcpy,
+                  (void *)c->d_e1, (void *)c->d_e2, (void *)c->d_iMn, (void *)c->d_met, (void *)c->d_met1, (void *)c->d_metn,
                   (void *)c->d_met1n, (void *)c->d_ms, (void *)c->d_ims32, (void *)c->d_m32, (void *)c->d_metp32,
                   (void *)c->d_bwork, (void *)c->d_f4x, (void *)c->d_nptr, (void *)c->d_ncopy, (void *)c->d_kvis,
-                  (void *)c->d_M, (void *)c->d_dz, (void *)c->d_zP, (void *)c->d_xS, (void *)c->d_coff,
-                  (void *)c->d_bar})
+                  (void *)c->d_M, (void *)c->d_dz, (void *)c->d_zP, (void *)c->d_xS, (void *)c->d_bar})
     if (p) (void)hipFree(p);
   prof_free(c);
   delete c;
@@ -798,27 +835,33 @@ extern "C" int cgd_profile_read(cgd_ctx *c, int which, double *total_ms, long lo
 // template dispatch on (N, chunk height, metric layout); R is the tendency
 // type (double, or float in the mixed-precision mode)
 template <int N, int NZT, bool CM, typename R>
-static void fcn1_t(cgd_ctx *c, int nitems, hipStream_t st, int slot0, const R *UR, R *T1, const double *U64,
-                   double *T1th) {
+static void fcn1_t(cgd_ctx *c, int nitems, hipStream_t st, const R *UR, R *E, const double *U64, double *Eth) {
   if (c->items1 == 2)
     hipLaunchKernelGGL((k_fcn1<N, NZT, CM, R, 2>), dim3((nitems + 1) / 2), dim3(c->block1), lds_fcn1<R>(c), st,
-                       c->ka, slot0, c->nchunk1, nitems, UR, T1, U64, T1th);
+                       c->ka, c->nchunk1, nitems, UR, E, U64, Eth);
   else
-    hipLaunchKernelGGL((k_fcn1<N, NZT, CM, R, 1>), dim3(nitems), dim3(c->block1), lds_fcn1<R>(c), st, c->ka, slot0,
-                       c->nchunk1, nitems, UR, T1, U64, T1th);
+    hipLaunchKernelGGL((k_fcn1<N, NZT, CM, R, 1>), dim3(nitems), dim3(c->block1), lds_fcn1<R>(c), st, c->ka,
+                       c->nchunk1, nitems, UR, E, U64, Eth);
 }
 template <int N, int NZT, bool CM, typename R>
-static void fcn2_t(cgd_ctx *c, dim3 g, hipStream_t st, int slot0, const double *U, const R *UR, const R *T1,
-                   const double *P, R *F, const double *T1th) {
-  if constexpr (std::is_same<R, double>::value) {
-    if (c->smooth) {  // kink-smoothed upwind flux (FP64 only)
-      hipLaunchKernelGGL((k_fcn2<N, NZT, CM, R, true>), g, dim3(c->block), lds_fcn2<R>(c), st, c->ka, slot0,
-                         c->nchunk, U, UR, T1, P, F, reinterpret_cast<R *>(c->d_f4x), T1th);
+static void fcn2_t(cgd_ctx *c, dim3 g, hipStream_t st, const double *U, const R *UR, const R *E1, const double *P,
+                   R *E2, const double *E1th, double *Cout) {
+  if constexpr (std::is_same<R, double>::value && CM) {
+    if (c->reg && !c->smooth) {
+      hipLaunchKernelGGL((k_fcn2r<N, NZT>), g, dim3(c->block), lds_fcn2r(c), st, c->ka, c->nchunk, U, E1, P, E2,
+                         c->d_f4x, Cout);
       return;
     }
   }
-  hipLaunchKernelGGL((k_fcn2<N, NZT, CM, R, false>), g, dim3(c->block), lds_fcn2<R>(c), st, c->ka, slot0,
-                     c->nchunk, U, UR, T1, P, F, reinterpret_cast<R *>(c->d_f4x), T1th);
+  if constexpr (std::is_same<R, double>::value) {
+    if (c->smooth) {  // kink-smoothed upwind flux (FP64 only)
+      hipLaunchKernelGGL((k_fcn2<N, NZT, CM, R, true>), g, dim3(c->block), lds_fcn2<R>(c), st, c->ka, c->nchunk, U,
+                         UR, E1, P, E2, reinterpret_cast<R *>(c->d_f4x), E1th, Cout);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((k_fcn2<N, NZT, CM, R, false>), g, dim3(c->block), lds_fcn2<R>(c), st, c->ka, c->nchunk, U,
+                     UR, E1, P, E2, reinterpret_cast<R *>(c->d_f4x), E1th, Cout);
 }
 #define CGD_DISPATCH(FN, R, NZTV, ...)                             \
   do {                                                             \
@@ -855,14 +898,13 @@ static void tr2lim_t(cgd_ctx *c, int nitems, hipStream_t st, int slot0, const do
 }
 
 template <typename R>
-static void launch_fcn1(cgd_ctx *c, int nitems, hipStream_t st, int slot0, const R *UR, R *T1, const double *U64,
-                        double *T1th) {
-  CGD_DISPATCH(fcn1_t, R, c->nzt1, nitems, st, slot0, UR, T1, U64, T1th);
+static void launch_fcn1(cgd_ctx *c, int nitems, hipStream_t st, const R *UR, R *E, const double *U64, double *Eth) {
+  CGD_DISPATCH(fcn1_t, R, c->nzt1, nitems, st, UR, E, U64, Eth);
 }
 template <typename R>
-static void launch_fcn2(cgd_ctx *c, dim3 g, hipStream_t st, int slot0, const double *U, const R *UR, const R *T1,
-                        const double *P, R *F, const double *T1th) {
-  CGD_DISPATCH(fcn2_t, R, c->nzt, g, st, slot0, U, UR, T1, P, F, T1th);
+static void launch_fcn2(cgd_ctx *c, dim3 g, hipStream_t st, const double *U, const R *UR, const R *E1,
+                        const double *P, R *E2, const double *E1th, double *Cout) {
+  CGD_DISPATCH(fcn2_t, R, c->nzt, g, st, U, UR, E1, P, E2, E1th, Cout);
 }
 
 extern "C" int cgd_prepare(cgd_ctx *c, const double *U, double *AuxG, void *stream) {
@@ -875,30 +917,30 @@ extern "C" int cgd_prepare(cgd_ctx *c, const double *U, double *AuxG, void *stre
   return CGD_OK;
 }
 
-// Both tendency passes; with f4fix the chunk-interface w terms are added by
-// k_f4fix (cgd_fcn), without it the caller consumes the side sums itself
-// (the fused stage kernel of cgd_rw_step).  U is the FP64 state; UR the
-// state the R-typed terms read (U itself, or its FP32 shadow).
+static bool has_hooks(const cgd_ctx *c) { return c->hooks.forcing || c->hooks.damping || c->hooks.micro; }
+
+// The element copies of the pass-1 cache (FP32 mode: four FP32 components,
+// then the FP64 theta cache)
+template <typename R> static double *e1_theta(cgd_ctx *c) {
+  return std::is_same<R, double>::value ? nullptr : c->d_e1 + 4 * c->ka.ecs;
+}
+
+// Both tendency passes.  The dynamics' tendency ends as element copies in
+// d_e2; with want_f (cgd_fcn; U = UR, R = double) and wherever physics hooks
+// add to it, it is summed into F, and with want_f the cache into Temp1.
+// The tracers' tendencies and caches are summed in F and Temp1 either way.
+// U is the FP64 state; UR the state the R-typed terms read (U itself, or
+// its FP32 shadow).
 template <typename R>
 static int run_fcn(cgd_ctx *c, R *F, const double *U, const R *UR, R *Temp1, const double *AuxG, hipStream_t st,
-                   bool f4fix) {
+                   bool want_f) {
   int r;
-  // every global node is written by its first element (colour order) and
-  // accumulated by the others, so Temp1 and F need no zero fill.  The FP32
-  // kernels keep the theta hyperviscosity cache in FP64 in Temp1 at the
-  // offset of component 4 in doubles (beyond the four FP32 components, below
-  // the tracers' caches from component 6 on)
-  double *const T1th = std::is_same<R, double>::value ? nullptr
-                                                       : reinterpret_cast<double *>(Temp1) + 3 * (size_t)c->NumG * c->Nz;
+  R *const E1 = reinterpret_cast<R *>(c->d_e1), *const E2 = reinterpret_cast<R *>(c->d_e2);
+  double *const E1th = e1_theta<R>(c);
   prof_begin(c, st, 0);
-  int launches = 0;
-  for (int k = 0; k < c->ncolor; ++k) {
-    const int ne = c->color_off[k + 1] - c->color_off[k];
-    if (!ne) continue;
-    launch_fcn1<R>(c, ne * c->nchunk1, st, c->color_off[k], UR, Temp1, U, T1th);
-    HIPCHK(c, hipGetLastError());
-    ++launches;
-  }
+  int launches = 1;
+  launch_fcn1<R>(c, c->NF * c->nchunk1, st, UR, E1, U, E1th);
+  HIPCHK(c, hipGetLastError());
   // the tracers run in FP64 in both modes: their tendencies and caches are
   // components 6.. of the FP64 F and Temp1 (the mixed mode's FP32 dynamics
   // occupies only the first five components' worth of those buffers)
@@ -915,10 +957,12 @@ static int run_fcn(cgd_ctx *c, R *F, const double *U, const R *UR, R *Temp1, con
   if ((r = prof_end(c, st, 0, launches))) return r;
   prof_begin(c, st, 1);
   launches = 0;
-  for (int k = 0; k < c->ncolor; ++k) {
-    const int ne = c->color_off[k + 1] - c->color_off[k];
-    if (!ne) continue;
-    launch_fcn2<R>(c, dim3(ne * c->nchunk), st, c->color_off[k], U, UR, Temp1, AuxG, F, T1th);
+  launch_fcn2<R>(c, dim3(c->NF * c->nchunk), st, U, UR, E1, AuxG, E2, E1th, want_f ? T1d : nullptr);
+  HIPCHK(c, hipGetLastError());
+  ++launches;
+  if (want_f || has_hooks(c)) {
+    hipLaunchKernelGGL((k_dss<R>), dim3(grid_for((size_t)c->NumG * c->Nz, 256)), dim3(256), 0, st, c->ka, E2,
+                       reinterpret_cast<const R *>(c->d_f4x), F, c->nchunk, c->nzt);
     HIPCHK(c, hipGetLastError());
     ++launches;
   }
@@ -948,20 +992,11 @@ static int run_fcn(cgd_ctx *c, R *F, const double *U, const R *UR, R *Temp1, con
       }
     }
   }
-  if (c->hooks.forcing || c->hooks.damping || c->hooks.micro) {
+  if (has_hooks(c)) {
     const size_t n = (size_t)c->NumG * c->Nz;
     hipLaunchKernelGGL((k_hooks<R>), dim3(grid_for(n, 256)), dim3(256), 0, st, c->ka, c->hooks, U, AuxG, F, Fd, n);
     HIPCHK(c, hipGetLastError());
     ++launches;
-  }
-  if constexpr (std::is_same<R, double>::value) {
-    if (f4fix && c->nchunk > 1) {
-      const size_t nfix = (size_t)c->NumG * (c->nchunk - 1);
-      hipLaunchKernelGGL(k_f4fix, dim3(grid_for(nfix, 256)), dim3(256), 0, st, c->d_nptr, c->d_ncopy, c->d_f4x, F,
-                         c->NumG, c->Nz, c->nchunk, c->nzt);
-      HIPCHK(c, hipGetLastError());
-      ++launches;
-    }
   }
   return prof_end(c, st, 1, launches);
 }
@@ -1046,54 +1081,55 @@ static bool persist_supported(const cgd_ctx *c, std::string *why) {
   return !w;
 }
 
-template <int N, typename R, int W> static const void *persist_fn() {
-  return reinterpret_cast<const void *>(&k_stage_persist<N, true, R, W>);
+template <int N, typename R, int W> static const void *persist_fn(const cgd_ctx *c) {
+  if constexpr (std::is_same<R, double>::value)
+    if (c->reg) return reinterpret_cast<const void *>(&k_stage_persist<N, true, R, W, true>);
+  return reinterpret_cast<const void *>(&k_stage_persist<N, true, R, W, false>);
+}
+template <typename R> static size_t lds_persist(const cgd_ctx *c) {
+  return std::max(lds_fcn1<R>(c), std::is_same<R, double>::value && c->reg ? lds_fcn2r(c) : lds_fcn2<R>(c));
 }
 
 // The grid: every workgroup resident at once (the kernel's occupancy per CU
 // times the CUs), and no more than the largest phase has work for.
 template <typename R, int W> static int persist_grid(cgd_ctx *c, int &G) {
-  const void *fn = c->N == 5 ? persist_fn<5, R, W>() : persist_fn<4, R, W>();
-  const size_t lds = std::max(lds_fcn1<R>(c), lds_fcn2<R>(c));
+  const void *fn = c->N == 5 ? persist_fn<5, R, W>(c) : persist_fn<4, R, W>(c);
+  const size_t lds = lds_persist<R>(c);
   int per_cu = 0, dev = 0, ncu = 0;
   HIPCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, c->block, lds));
   HIPCHK(c, hipGetDevice(&dev));
   HIPCHK(c, hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
   if (per_cu < 1) return fail(c, CGD_ERR_UNSUPPORTED, "persistent stage launch: the kernel does not fit a CU");
   int need = (c->NumG + c->colblock / c->colw - 1) / (c->colblock / c->colw);
-  for (int k = 0; k < c->ncolor; ++k) {
-    const int ne = c->color_off[k + 1] - c->color_off[k];
-    need = std::max(need, ne * std::max(c->nchunk, c->nchunk1));
-  }
+  need = std::max(need, c->NF * std::max(c->nchunk, c->nchunk1));
   G = std::max(1, std::min(per_cu * ncu, need));
   return CGD_OK;
 }
 
 template <typename R, int W>
-static int launch_persist(cgd_ctx *c, int is, const RWStage<R> &rw, const double *U, const R *UR, R *T1, double *T1th,
-                          const double *P, R *F, hipStream_t st) {
+static int launch_persist(cgd_ctx *c, int is, const RWStage<R> &rw, const double *U, const R *UR, const double *P,
+                          hipStream_t st) {
   int r;
   if (!c->pgrid && (r = persist_grid<R, W>(c, c->pgrid))) return r;
   StagePersist<R> p{};
-  p.coff = c->d_coff;
-  p.ncolor = c->ncolor;
+  p.nf = c->NF;
   p.nchunk1 = c->nchunk1;
   p.nchunk = c->nchunk;
   p.UR = UR;
-  p.T1 = T1;
+  p.T1 = reinterpret_cast<R *>(c->d_e1);
   p.U = U;
-  p.T1th = T1th;
+  p.T1th = e1_theta<R>(c);
   p.P = P;
-  p.F = F;
+  p.F = reinterpret_cast<R *>(c->d_e2);
   p.F4x = reinterpret_cast<R *>(c->d_f4x);
   p.bar = c->d_bar;
   p.deadline = c->bar_ticks;
   p.stage_blocks = (unsigned)((c->NumG + c->colblock / W - 1) / (c->colblock / W));
-  const size_t lds = std::max(lds_fcn1<R>(c), lds_fcn2<R>(c));
-  if (c->N == 5)
-    hipLaunchKernelGGL((k_stage_persist<5, true, R, W>), dim3(c->pgrid), dim3(c->block), lds, st, c->ka, p, rw, is);
-  else
-    hipLaunchKernelGGL((k_stage_persist<4, true, R, W>), dim3(c->pgrid), dim3(c->block), lds, st, c->ka, p, rw, is);
+  const size_t lds = lds_persist<R>(c);
+  const void *fn = c->N == 5 ? persist_fn<5, R, W>(c) : persist_fn<4, R, W>(c);
+  RWStage<R> rws = rw;
+  void *args[] = {&c->ka, &p, &rws, &is};
+  HIPCHK(c, hipLaunchKernel(fn, dim3(c->pgrid), dim3(c->block), args, lds, st));
   HIPCHK(c, hipGetLastError());
   return CGD_OK;
 }
@@ -1128,7 +1164,8 @@ static int rw_step_fused(cgd_ctx *c, double *V, double dt, const cgd_rw_work *w,
   for (int is = 0; is < 3; ++is) {
     if (!c->persistent && (r = run_fcn<R>(c, F, V, UR, T1, w->AuxG, st, false))) return r;
     RWStage<R> rw{};
-    rw.fV = F;
+    rw.fV = has_hooks(c) ? F : nullptr;
+    rw.Fe = reinterpret_cast<const R *>(c->d_e2);
     rw.V32 = (is < 2 || more) ? V32 : nullptr;
     // the stage increments are stored as R (FP32 in the mixed mode: they
     // are ~dt*F, so their rounding is ~1e-7 of an increment)
@@ -1148,8 +1185,6 @@ static int rw_step_fused(cgd_ctx *c, double *V, double dt, const cgd_rw_work *w,
     rw.k = is < 2 ? kR[is] : nullptr;  // k_3 is consumed in registers
     rw.P = (is < 2 || more) ? w->AuxG : nullptr;
     rw.F4x = reinterpret_cast<const R *>(c->d_f4x);
-    rw.nptr = c->d_nptr;
-    rw.ncopy = c->d_ncopy;
     rw.nchunk = c->nchunk;
     rw.nzt = c->nzt;
     rw.fac = dt * gamma;
@@ -1157,11 +1192,9 @@ static int rw_step_fused(cgd_ctx *c, double *V, double dt, const cgd_rw_work *w,
     rw.invfac2 = rw.invfac / rw.fac;
     rw.thomas = c->thomas;
     if (c->persistent) {  // both passes and the column stage in one launch (timed as the column pass)
-      double *const T1th =
-          mixed ? reinterpret_cast<double *>(w->Temp1) + 3 * (size_t)c->NumG * c->Nz : nullptr;
       prof_begin(c, st, 2);
-      r = c->colw == 32 ? launch_persist<R, 32>(c, is, rw, V, UR, T1, T1th, w->AuxG, F, st)
-                        : launch_persist<R, 64>(c, is, rw, V, UR, T1, T1th, w->AuxG, F, st);
+      r = c->colw == 32 ? launch_persist<R, 32>(c, is, rw, V, UR, w->AuxG, st)
+                        : launch_persist<R, 64>(c, is, rw, V, UR, w->AuxG, st);
       if (r) return r;
       if ((r = prof_end(c, st, 2, 1))) return r;
       continue;
@@ -1560,4 +1593,5 @@ extern "C" int cgd_autotune(cgd_ctx *c, double *V, double dt, const cgd_rw_work 
 
 // ------------------------------------------------------------------------
 // Adjoint of the FP64 path
+#pragma clang fp contract(fast)
 #include "cgd_adjoint.hip"

@@ -233,7 +233,7 @@ __global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64)
   load_dmats<N>(a, Ds, DWs);
   const int Nz = a.Nz;
   const int eb = blockIdx.x / nchunk, chunk = blockIdx.x - eb * nchunk;
-  const int e = slot0 + eb;  // element slot (one colour per launch)
+  const int e = a.clist[slot0 + eb];  // one colour per launch
   const int t = threadIdx.x, node = t / NZT, l = t - node * NZT;
   const int iz = chunk * NZT + l;
   const bool in_tile = node < NN, valid = in_tile && iz < Nz;
@@ -787,7 +787,7 @@ __global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64)
   load_dmats<N>(a, Ds, DWs);
   const int Nz = a.Nz;
   const int eb = blockIdx.x / nchunk, chunk = blockIdx.x - eb * nchunk;
-  const int e = slot0 + eb;  // element slot (one colour per launch)
+  const int e = a.clist[slot0 + eb];  // one colour per launch
   const int t = threadIdx.x, node = t / NZT, l = t - node * NZT;
   const int iz = chunk * NZT + l;
   const bool in_tile = node < NN, valid = in_tile && iz < Nz;

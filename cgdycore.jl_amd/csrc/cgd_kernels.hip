@@ -13,15 +13,23 @@
 // level = t % NZT, so a chunk column fills whole 16-lane DPP rows.
 // Horizontal derivatives exchange values through LDS tiles
 // tile[f][node][level]; vertical neighbours come from the neighbouring
-// lanes by DPP row shifts, with one global load at each chunk edge.  The DSS is a non-atomic
-// read-modify-write: one launch per element colour (no two elements of a
-// colour share a global node), so every global node accumulates its element
-// contributions in a fixed order.
+// lanes by DPP row shifts, with one global load at each chunk edge.
+//
+// DSS: the dynamics' element passes write each element's contributions to
+// an array of its own, X[c][e*NN + node][iz], all elements in one launch,
+// and the consumer of a field sums a node's copies in colour order (a
+// fixed order, no atomics).  The tracer kernels accumulate in place, one
+// launch per element colour (no two elements of a colour share a node).
 #include <hip/hip_runtime.h>
 
 #include <stdint.h>
 
 #include <type_traits>
+
+// Multiply-adds are fused within an expression, by the front end, and not
+// wherever the code generator finds them: a kernel body that is inlined in
+// two kernels (separate and persistent launches) then rounds the same way.
+#pragma clang fp contract(on)
 
 #define CGD_NMAX 5
 #define CGD_NMET 17  // pass-2 metric components
@@ -35,17 +43,23 @@ struct KArgs {
   double Rd_p0, eos_y, dpd_y;      // Rd/p0, 1/(1-kappa), kappa/(1-kappa)
   double D[CGD_NMAX * CGD_NMAX];   // D[i*N + k] = DS[i,k]
   double DWm[CGD_NMAX * CGD_NMAX]; // DW[i*N + k]
-  const int *glob;                 // [slot][NN]: 0-based node | bit 31 set on the node's first copy
-  const double *met;               // [slot][17][NN][Nz], or [slot][4][NN][Nz] in the compact layout
-  const double *met1;              // [slot][5][NN][Nz] (full layout only)
-  const double *metn;              // compact layout: [slot][13][NN]
-  const double *met1n;             // compact layout: [slot][5][NN]
+  const int *glob;                 // [e][NN]: 0-based node | bit 31 set on the node's first copy (colour order)
+  const int *clist;                // elements by colour (the tracer and adjoint kernels' launch order)
+  const int *cpy;                  // [e][NN][cpw]: the node's copies e'*NN + node' in colour order, then -1
+  const int *gcpy;                 // [NumG][cpw]: the same per global node
+  int cpw;                         // a multiple of 2, at least 4
+  size_t ecs;                      // NF*NN*Nz: values per component of an element-copy array
+  const double *met;               // [e][17][NN][Nz], or [e][5][NN][Nz] in the compact layout
+  const double *met1;              // [element][5][NN][Nz] (full layout only)
+  const double *metn;              // compact layout: [element][13][NN]
+  const double *met1n;             // compact layout: [element][5][NN]
   const double *iMs;               // [NumG][Nz]: 1 / (M1 + M2)
   const float *iMs32;              // the same in FP32 (mixed-precision mode)
   const float *M32;                // M in FP32 (mixed-precision mode)
   const float *metp32;             // compact layout's per-point components in FP32 (mixed precision)
   const double *M;                 // [2][NumG][Nz]
-  const double *kvis;              // [slot][3]: HyperDCurl, HyperDGrad, HyperDDiv of the element's grid
+  const double *iMn;               // regular metric (cgd_pass2r_body.inc): [NumG], 1 / (M1 + M2); else null
+  const double *kvis;              // [element][3]: HyperDCurl, HyperDGrad, HyperDDiv of the element's grid
   // Models.Moist: 0-based components of the vapour and cloud densities (-1: dry)
   int iv, ic;
   double Cpv, Cpl, Rv;
@@ -350,21 +364,21 @@ template <int N, typename R> __device__ __forceinline__ void load_dmats(const KA
 
 // ------------------------------------------------------------------------
 // Pass 1: HyperViscKernel! (src/GPU/ViscKernel.jl:1-84).
-// Grid: one workgroup per ITEMS consecutive work items of the colour, an
+// Grid: one workgroup per ITEMS consecutive work items, an
 // item being one (element, level chunk).  With ITEMS = 2 the loads of both
 // items are issued before the first item's derivative phases, so a wave has
 // twice the memory requests in flight (the kernel is latency-bound: its
-// waves mostly wait on memory).  nitems = elements of the colour x nchunk.
+// waves mostly wait on memory).  nitems = elements x nchunk.
 // R is the arithmetic and storage type of the state it reads (U: the state,
 // or its FP32 shadow), of Temp1 and of the LDS tiles: double, or float in
 // the mixed-precision mode.
 template <typename R> struct Pass1In {
   R S11, S12, S21, S22, Js, iMs;
   R rho, u, v, rth;
-  R o1, o2, o3, o4, o5;
-  double rho_d, rth_d, o5d;  // FP32 kernel: the FP64 rho, rho*theta and theta-cache accumulator
-  unsigned ui;
-  bool first, valid;
+  double rho_d, rth_d;  // FP32 kernel: the FP64 rho and rho*theta
+  unsigned eo;          // offset of the point in its element's copies
+  int e;
+  bool valid;
 };
 
 // The FP32 (mixed-precision) element kernels compute the theta
@@ -380,12 +394,11 @@ template <int N, int NZ> struct ThetaHV {
 };
 
 template <int N, int NZT, bool CM, typename R>
-__device__ __forceinline__ Pass1In<R> pass1_load(const KArgs &a, int slot0, int nchunk, int nitems, int L,
-                                                 const R *__restrict__ U, const R *__restrict__ T1,
-                                                 const double *__restrict__ U64, const double *__restrict__ T1th) {
+__device__ __forceinline__ Pass1In<R> pass1_load(const KArgs &a, int nchunk, int nitems, int L,
+                                                 const R *__restrict__ U, const double *__restrict__ U64) {
   constexpr int NN = N * N;
   const int Nz = a.Nz;
-  const int e = slot0 + L / nchunk;  // element slot (elements are stored in colour order)
+  const int e = L / nchunk;
   const int chunk = L - (L / nchunk) * nchunk;
   const int t = threadIdx.x;
   const int node = t / NZT, l = t - node * NZT;
@@ -394,14 +407,15 @@ __device__ __forceinline__ Pass1In<R> pass1_load(const KArgs &a, int slot0, int 
   const size_t NNZ = (size_t)NN * Nz;
   Pass1In<R> in{};
   in.valid = L < nitems && node < NN && iz < Nz;
+  in.e = e;
   in.Js = 1;
   in.iMs = 1;
   if (!in.valid) return in;
   // uniform bases + 32-bit lane offsets (the host checks NumG*Nz < 2^28)
-  const int gv = a.glob[e * NN + node];
-  in.first = gv < 0;
-  in.ui = (unsigned)(gv & 0x7fffffff) * (unsigned)Nz + iz;
-  __builtin_assume(in.ui < (1u << 28));
+  const int gv = a.glob[(size_t)e * NN + node];
+  const unsigned ui = (unsigned)(gv & 0x7fffffff) * (unsigned)Nz + iz;
+  __builtin_assume(ui < (1u << 28));
+  in.eo = (unsigned)(node * Nz + iz);
   if constexpr (CM) {
     const double *mN = a.met1n + (size_t)e * CGD_NMET1 * NN;
     const unsigned nd = (unsigned)node;
@@ -422,44 +436,34 @@ __device__ __forceinline__ Pass1In<R> pass1_load(const KArgs &a, int slot0, int 
   }
   const R *iMsR = std::is_same<R, double>::value ? reinterpret_cast<const R *>(a.iMs)
                                                   : reinterpret_cast<const R *>(a.iMs32);
-  in.iMs = at(iMsR, in.ui);
-  // the DSS accumulators of this node: no other element of the colour
-  // touches them, so they are read now, with the state, not after the
-  // derivative phases
-  if (!in.first) {
-    in.o1 = at(T1, in.ui);
-    in.o2 = at(T1 + vs, in.ui);
-    in.o3 = at(T1 + 2 * vs, in.ui);
-    in.o4 = at(T1 + 3 * vs, in.ui);
-    if constexpr (std::is_same<R, double>::value) in.o5 = at(T1 + 4 * vs, in.ui);
-  }
-  in.rho = at(U, in.ui);
-  in.u = at(U + vs, in.ui);
-  in.v = at(U + 2 * vs, in.ui);
+  in.iMs = at(iMsR, ui);
+  in.rho = at(U, ui);
+  in.u = at(U + vs, ui);
+  in.v = at(U + 2 * vs, ui);
   if constexpr (std::is_same<R, double>::value) {
-    in.rth = at(U + 4 * vs, in.ui);
+    in.rth = at(U + 4 * vs, ui);
   } else {
-    in.rho_d = at(U64, in.ui);
-    in.rth_d = at(U64 + 4 * vs, in.ui);
-    if (!in.first) in.o5d = at(T1th, in.ui);
+    in.rho_d = at(U64, ui);
+    in.rth_d = at(U64 + 4 * vs, ui);
   }
   return in;
 }
 
-// the derivative phases of one item and its DSS write; every lane of the
+// the derivative phases of one item and the write of its element copies
+// (E; the FP64 theta cache Eth of the FP32 kernel); every lane of the
 // workgroup calls it (two barriers)
 template <int N, int NZT, typename R>
 __device__ __forceinline__ void pass1_compute(const KArgs &a, const Pass1In<R> &in, const R *Ds, const R *DWs,
                                               const Tiles<N, NZT, R> &T, const Tiles<N, NZT, R> &TB,
-                                              R *__restrict__ T1, const ThetaHV<N, NZT> &H,
-                                              double *__restrict__ T1th) {
+                                              R *__restrict__ E, const ThetaHV<N, NZT> &H,
+                                              double *__restrict__ Eth) {
   constexpr bool F32 = !std::is_same<R, double>::value;
   constexpr int NN = N * N;
   const int t = threadIdx.x;
   const int node = t / NZT, l = t - node * NZT;
   const bool in_tile = node < NN;
   const int I = node % N, J = node / N;
-  const size_t vs = (size_t)a.NumG * a.Nz;
+  const size_t eb = (size_t)in.e * NN * a.Nz;
   R uC = 0, vC = 0, uD = 0, vD = 0, Th = 0;
   if (in.valid) {
     uC = in.S11 * in.v - in.S12 * in.u;  // Curl12
@@ -528,43 +532,35 @@ __device__ __forceinline__ void pass1_compute(const KArgs &a, const Pass1In<R> &
     const R FvC = -in.S11 * DxCurl - in.S21 * DyCurl;
     const R FuD = in.S11 * DxDiv + in.S21 * DyDiv;  // Grad12
     const R FvD = in.S12 * DxDiv + in.S22 * DyDiv;
-    // DSS: the first element (in colour order) holding the node writes,
-    // the others accumulate
     const R iMs = in.iMs;
-    const R r1 = -FuC * iMs, r2 = -FvC * iMs, r3 = FuD * iMs, r4 = FvD * iMs, r5 = DivTh * iMs;
-    R *T1a = T1, *T1b = T1 + vs, *T1c = T1 + 2 * vs, *T1d = T1 + 3 * vs, *T1e = T1 + 4 * vs;
-    at(T1a, in.ui) = in.first ? r1 : in.o1 + r1;
-    at(T1b, in.ui) = in.first ? r2 : in.o2 + r2;
-    at(T1c, in.ui) = in.first ? r3 : in.o3 + r3;
-    at(T1d, in.ui) = in.first ? r4 : in.o4 + r4;
-    if constexpr (F32) {
-      const double r5d = dxy<N, NZT, double>(H.DWd, H.B, 0, 1, I, J, l) * double(iMs);
-      at(T1th, in.ui) = in.first ? r5d : in.o5d + r5d;
-    } else {
-      at(T1e, in.ui) = in.first ? r5 : in.o5 + r5;
-    }
+    R *Ea = E + eb, *Eb = Ea + a.ecs, *Ec = Eb + a.ecs, *Ed = Ec + a.ecs, *Ee = Ed + a.ecs;
+    at(Ea, in.eo) = -FuC * iMs;
+    at(Eb, in.eo) = -FvC * iMs;
+    at(Ec, in.eo) = FuD * iMs;
+    at(Ed, in.eo) = FvD * iMs;
+    if constexpr (F32) at(Eth + eb, in.eo) = dxy<N, NZT, double>(H.DWd, H.B, 0, 1, I, J, l) * double(iMs);
+    else at(Ee, in.eo) = DivTh * iMs;
   }
 }
 
-// U64, T1th: the FP64 state and the FP64 theta cache of the FP32 kernel
+// U64, Eth: the FP64 state and the FP64 theta cache of the FP32 kernel
 // (unused by the FP64 one).  The body is shared by the kernel and by
 // fcn1_block, a workgroup's share in a persistent launch (items item*ITEMS
-// .. item*ITEMS + ITEMS - 1 of a colour).
+// .. item*ITEMS + ITEMS - 1).
 template <int N, int NZT, bool CM, typename R, int ITEMS>
-__device__ __forceinline__ void fcn1_block(int item, const KArgs &a, int slot0, int nchunk, int nitems,
-                                           const R *__restrict__ U, R *__restrict__ T1,
-                                           const double *__restrict__ U64, double *__restrict__ T1th) {
+__device__ __forceinline__ void fcn1_block(int item, const KArgs &a, int nchunk, int nitems, const R *__restrict__ U,
+                                           R *__restrict__ E, const double *__restrict__ U64,
+                                           double *__restrict__ Eth) {
 #define CGD_ITEM item
 #include "cgd_pass1_body.inc"
 #undef CGD_ITEM
 }
 
 template <int N, int NZT, bool CM, typename R, int ITEMS>
-__global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64) k_fcn1(KArgs a, int slot0, int nchunk, int nitems,
-                                                                       const R *__restrict__ U,
-                                                                       R *__restrict__ T1,
+__global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64) k_fcn1(KArgs a, int nchunk, int nitems,
+                                                                       const R *__restrict__ U, R *__restrict__ E,
                                                                        const double *__restrict__ U64,
-                                                                       double *__restrict__ T1th) {
+                                                                       double *__restrict__ Eth) {
 #define CGD_ITEM xcd_logical(blockIdx.x, gridDim.x)
 #include "cgd_pass1_body.inc"
 #undef CGD_ITEM
@@ -575,8 +571,8 @@ __global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64) k_fcn1(KArgs a, 
 // GradFullKernel! + DivRhoTrUpwind3New2Kernel! fused into one element pass
 // (src/GPU/ViscKernel.jl:86-167, src/GPU/MomentumKernel.jl:1-178,
 // src/GPU/GradKineticKernel.jl:1-129, src/GPU/OperatorKernel.jl:637-720).
-// Launched once per colour over (element, level chunk) workgroups; the
-// chunks of one element are independent.
+// One launch over (element, level chunk) workgroups; the chunks of one
+// element are independent.
 //
 // Phase 0 computes every term that couples levels (vertical momentum
 // fluxes, kinetic-energy and pressure differences, the upwind mass and
@@ -585,22 +581,25 @@ __global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64) k_fcn1(KArgs a, 
 // thread adds the fluxes of both its interfaces to its own level (the
 // reference adds them from the owner of the interface); F4 of interface iz
 // combines this layer's upper terms with the layer above's lower terms.
+// C holds the pass-1 cache as element copies (each point sums its node's),
+// F receives the element copies of the tendency, and Cout (FP64, may be
+// null) the summed cache in the layout of Temp1.
 // R is the arithmetic and storage type of the tendency (F, the chunk side
-// sums F4x), of the hyperviscosity cache C = Temp1, of the winds and rho*theta
+// sums F4x), of the hyperviscosity cache C, of the winds and rho*theta
 // it reads (UR: the state, or its FP32 shadow) and of the LDS tiles: double,
 // or float in the mixed-precision mode.  FP64 in both modes: rho (from the
 // FP64 state U), the pressure P, the w-interface balance of pressure
 // gradient and gravity (rho, p, J and dXdxI[3,3] in FP64), the horizontal
 // pressure gradient (an FP64 tile and derivative) and the theta
 // hyperviscosity (its FP64 cache Cth, FP64 tiles and derivatives).
-// The body is shared by the kernel and by fcn2_block, one item of a colour
-// in a persistent launch.
+// The body is shared by the kernel and by fcn2_block, one item of a
+// persistent launch.
 template <int N, int NZT, bool CM, typename R, bool SM>
-__device__ __forceinline__ void fcn2_block(int item, const KArgs &a, int slot0, int nchunk,
+__device__ __forceinline__ void fcn2_block(int item, const KArgs &a, int nchunk,
                                            const double *__restrict__ U, const R *__restrict__ UR,
                                            const R *__restrict__ C, const double *__restrict__ P,
                                            R *__restrict__ F, R *__restrict__ F4x,
-                                           const double *__restrict__ Cth) {
+                                           const double *__restrict__ Cth, double *__restrict__ Cout) {
 #define CGD_ITEM item
 #define CGD_EARLY_HALO false
 #include "cgd_pass2_body.inc"
@@ -609,15 +608,50 @@ __device__ __forceinline__ void fcn2_block(int item, const KArgs &a, int slot0, 
 }
 
 template <int N, int NZT, bool CM, typename R, bool SM>
-__global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64) __attribute__((amdgpu_waves_per_eu(std::is_same<R, float>::value ? 5 : 4))) k_fcn2(KArgs a, int slot0, int nchunk,
+__global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64) __attribute__((amdgpu_waves_per_eu(std::is_same<R, float>::value ? 5 : 4))) k_fcn2(KArgs a, int nchunk,
                                                const double *__restrict__ U, const R *__restrict__ UR,
                                                const R *__restrict__ C, const double *__restrict__ P,
                                                R *__restrict__ F, R *__restrict__ F4x,
-                                               const double *__restrict__ Cth) {
+                                               const double *__restrict__ Cth, double *__restrict__ Cout) {
 #define CGD_ITEM xcd_logical(blockIdx.x, gridDim.x)
 #define CGD_EARLY_HALO true
 #include "cgd_pass2_body.inc"
 #undef CGD_EARLY_HALO
+#undef CGD_ITEM
+}
+
+// any_value: an unspecified value, for a variable that only some lanes set
+// (no instruction to initialise it).
+// pin computes its arguments here: an empty asm that reads and writes them, so
+// that the code generator, which orders arithmetic within a block by its
+// own measure, does not hold the inputs of a long block's later sums (LDS
+// values, neighbour levels) in registers and spill them.
+__device__ __forceinline__ double any_value() { return __builtin_nondeterministic_value(0.0); }
+__device__ __forceinline__ void pin(double &x) { asm volatile("" : "+v"(x)); }
+template <typename... D> __device__ __forceinline__ void pin(double &x, D &...y) {
+  pin(x);
+  pin(y...);
+}
+
+// Pass 2 for the regular compact metric (FP64): the same terms, reduced by
+// what such a metric and mass share between levels and vertical nodes.
+template <int N, int NZT>
+__device__ __forceinline__ void fcn2r_block(int item, const KArgs &a, int nchunk, const double *__restrict__ U,
+                                            const double *__restrict__ C, const double *__restrict__ P,
+                                            double *__restrict__ F, double *__restrict__ F4x,
+                                            double *__restrict__ Cout) {
+#define CGD_ITEM item
+#include "cgd_pass2r_body.inc"
+#undef CGD_ITEM
+}
+
+template <int N, int NZT>
+__global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64) __attribute__((amdgpu_waves_per_eu(5)))
+    k_fcn2r(KArgs a, int nchunk, const double *__restrict__ U, const double *__restrict__ C,
+            const double *__restrict__ P, double *__restrict__ F, double *__restrict__ F4x,
+            double *__restrict__ Cout) {
+#define CGD_ITEM xcd_logical(blockIdx.x, gridDim.x)
+#include "cgd_pass2r_body.inc"
 #undef CGD_ITEM
 }
 
@@ -709,7 +743,7 @@ __global__ void k_hooks(KArgs a, Hooks hk, const double *__restrict__ U, const d
 // k_fcn1/k_fcn2), over (element, level chunk) workgroups, all tracers in one
 // launch.  Tracers do not feed back on the dynamics.
 
-// metric component c of element slot e at (node, level), either layout
+// metric component c of element e at (node, level), either layout
 template <int NN, bool CM>
 __device__ __forceinline__ double met_at(const KArgs &a, size_t e, int c, int node, int iz) {
   const size_t Nz = (size_t)a.Nz;
@@ -732,7 +766,7 @@ __global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64) k_tr1(KArgs a, i
   load_dmats<N>(a, Ds, DWs);
   const int Nz = a.Nz;
   const int L = xcd_logical(blockIdx.x, gridDim.x);
-  const int e = slot0 + L / nchunk;
+  const int e = a.clist[slot0 + L / nchunk];
   const int chunk = L - (L / nchunk) * nchunk;
   const int t = threadIdx.x;
   const int node = t / NZT, l = t - node * NZT;
@@ -821,7 +855,7 @@ __global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64) k_tr2(KArgs a, i
   load_dmats<N>(a, Ds, DWs);
   const int Nz = a.Nz;
   const int L = xcd_logical(blockIdx.x, gridDim.x);
-  const int e = slot0 + L / nchunk;
+  const int e = a.clist[slot0 + L / nchunk];
   const int chunk = L - (L / nchunk) * nchunk;
   const int t = threadIdx.x;
   const int node = t / NZT, l = t - node * NZT;
@@ -1021,9 +1055,9 @@ __global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64) k_tr2(KArgs a, i
 // ------------------------------------------------------------------------
 // HorLimit (src/GPU/HorLimiterKernel.jl)
 
-// LimitKernel! (HorLimiterKernel.jl:2-22): per tracer, element slot and
+// LimitKernel! (HorLimiterKernel.jl:2-22): per tracer, element and
 // level, the min and max over the element's nodes of the mixing ratio;
-// qmin/qmax[(tr*NF + slot)*Nz + iz]
+// qmin/qmax[(tr*NF + element)*Nz + iz]
 __global__ void k_lim_bounds(KArgs a, int NF, int NN, int ntr, const double *__restrict__ U,
                              double *__restrict__ qmin, double *__restrict__ qmax) {
   const int Nz = a.Nz;
@@ -1101,7 +1135,7 @@ __global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64)
   if (threadIdx.x < NN) Ds[threadIdx.x] = a.D[threadIdx.x];
   const int Nz = a.Nz;
   const int L = xcd_logical(blockIdx.x, gridDim.x);
-  const int e = slot0 + L / nchunk;
+  const int e = a.clist[slot0 + L / nchunk];
   const int chunk = L - (L / nchunk) * nchunk;
   const int t = threadIdx.x;
   const int node = t / NZT, l = t - node * NZT;
@@ -1358,21 +1392,49 @@ __global__ void k_rw_tr(const double *__restrict__ fV, const double *__restrict_
   }
 }
 
-// F4 of the interfaces between level chunks: the lower-interface term of a
-// chunk's first level, summed over the elements sharing the node in the
-// fixed order of nodecopy (colour order), added to F after all colours.
-__global__ void k_f4fix(const int *__restrict__ nptr, const int *__restrict__ ncopy, const double *__restrict__ F4x,
-                        double *__restrict__ F, int NumG, int Nz, int nchunk, int nzt) {
-  const size_t total = (size_t)NumG * (nchunk - 1);
-  const size_t vs = (size_t)NumG * Nz;
-  for (size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x; q < total; q += (size_t)gridDim.x * blockDim.x) {
-    const int g = (int)(q / (nchunk - 1));
-    const int ch = 1 + (int)(q - (size_t)g * (nchunk - 1));
-    const int iz = ch * nzt;
-    if (iz >= Nz) continue;
-    double s = 0.0;
-    for (int c = nptr[g]; c < nptr[g + 1]; ++c) s += F4x[(size_t)ncopy[c] * nchunk + ch];
-    F[3 * vs + (size_t)g * Nz + iz - 1] += s;
+// The tendency of the dynamics from its element copies E: F = the sum over
+// each node's copies in colour order, plus for w the chunk-interface terms
+// (the lower-interface terms of the first levels of the chunks above, F4x).
+// For callers that want F itself (cgd_fcn, the physics hooks); the stage
+// kernel sums the copies in registers instead.
+template <typename R>
+__global__ void k_dss(KArgs a, const R *__restrict__ E, const R *__restrict__ F4x, R *__restrict__ F, int nchunk,
+                      int nzt) {
+  const int Nz = a.Nz;
+  const size_t vs = (size_t)a.NumG * Nz;
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < vs; i += (size_t)gridDim.x * blockDim.x) {
+    const size_t g = i / Nz;
+    const int iz = (int)(i - g * Nz);
+    const bool edge = nchunk > 1 && (iz + 1) % nzt == 0 && iz + 1 < Nz;
+    const int ch = (iz + 1) / nzt;
+    R s[5] = {0, 0, 0, 0, 0}, s4 = 0;
+    for (int r0 = 0; r0 < a.cpw; r0 += 2) {
+      const int2 cq = *reinterpret_cast<const int2 *>(a.gcpy + g * a.cpw + r0);
+      if (cq.x < 0) break;
+      const int cpq[2] = {cq.x, cq.y};
+      R x[2][5], x4[2];
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        x4[j] = 0;
+#pragma unroll
+        for (int q = 0; q < 5; ++q) x[j][q] = 0;
+        if (cpq[j] >= 0) {
+          const R *Ec = E + (size_t)cpq[j] * Nz + iz;
+#pragma unroll
+          for (int q = 0; q < 5; ++q) x[j][q] = Ec[q * a.ecs];
+          if (edge) x4[j] = F4x[(size_t)cpq[j] * nchunk + ch];
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+#pragma unroll
+        for (int q = 0; q < 5; ++q) s[q] += x[j][q];
+        s4 += x4[j];
+      }
+    }
+    if (edge) s[3] += s4;
+#pragma unroll
+    for (int q = 0; q < 5; ++q) F[q * vs + i] = s[q];
   }
 }
 
@@ -1664,8 +1726,8 @@ __global__ void k_jac(KArgs a, const double *__restrict__ U, const double *__res
 //  - the frozen Jacobian (JacSchurGPU! of the stage-1 state, which is Vn)
 //    and the Schur tri matrix are rebuilt from Vn in every stage, with the
 //    same arithmetic as k_jac and the tri build of k_schur_col;
-//  - the w tendency of the interfaces between level chunks (the side sums
-//    of k_fcn2) is added here, in k_f4fix's order;
+//  - the tendency is summed here from its element copies, in k_dss's
+//    order, with the w terms of the interfaces between level chunks;
 //  - fV + sum_j (c_ij/dt) k_j, the Schur solve, and the next stage state
 //    V = Vn + sum_j a_{i+1,j} k_j (or the final V = Vn + sum_j m_j k_j)
 //    follow in registers, and the pressure of the next stage's
@@ -1675,7 +1737,8 @@ __global__ void k_jac(KArgs a, const double *__restrict__ U, const double *__res
 // few MB of L2 per XCD), so their loads and stores are non-temporal: at
 // ne=60, nz=64 that takes 6 % off the stage kernel's time.
 template <typename R> struct RWStage {
-  const R *fV;             // this stage's tendency (FP32 in the mixed-precision mode)
+  const R *fV;             // this stage's tendency (FP32 in the mixed-precision mode); null: its element copies
+  const R *Fe;             // element copies of the tendency
   float *V32;              // FP32 shadow of the next stage state (mixed-precision mode; else null)
   const R *kprev[2];       // k_1, k_2 (earlier stages; FP32 storage in the mixed mode)
   double cf[2];            // c_ij / dt
@@ -1687,7 +1750,6 @@ template <typename R> struct RWStage {
   R *k;                    // this stage's increment (null: not stored)
   double *P;               // AuxG[:,:,1] for the next stage (null: not written)
   const R *F4x;            // chunk-interface w terms of k_fcn2
-  const int *nptr, *ncopy; // node -> element copies, colour order
   int nchunk, nzt;
   double fac;              // dt * gamma
   double invfac, invfac2;  // 1/fac and (1/fac)/fac
@@ -1713,10 +1775,10 @@ __global__ void __launch_bounds__(256) k_rw_stage(KArgs a, RWStage<R> rw) {
 }
 
 // ------------------------------------------------------------------------
-// One persistent launch per Rosenbrock-W stage: pass 1 over every colour,
-// pass 2 over every colour, then the column stage, in one grid whose
+// One persistent launch per Rosenbrock-W stage: pass 1, pass 2, then the
+// column stage, in one grid whose
 // workgroups are all resident at once (the host sizes the grid from the
-// kernel's occupancy).  A grid-wide barrier separates the colours and the
+// kernel's occupancy).  A grid-wide barrier separates the
 // passes, where the ordinary path has kernel boundaries; the arithmetic is
 // the same per item, so the results are bit-identical to the ordinary
 // launches.
@@ -1837,12 +1899,11 @@ __device__ __forceinline__ void grid_sync(GridBar *gb, unsigned &n, unsigned nbl
 }
 
 template <typename R> struct StagePersist {
-  const int *coff;      // first element slot of each colour, ncolor + 1 entries
-  int ncolor, nchunk1, nchunk;
+  int nf, nchunk1, nchunk;  // elements, level chunks of the passes
   const R *UR;          // pass 1 and pass 2: the state the R-typed terms read
-  R *T1;                // hyperviscosity cache (Temp1)
+  R *T1;                // hyperviscosity cache (element copies)
   const double *U;      // FP64 state
-  double *T1th;         // FP32 mode: the FP64 theta cache
+  double *T1th;         // FP32 mode: the FP64 theta cache (element copies)
   const double *P;      // pressure
   R *F, *F4x;           // tendency, chunk-interface side sums
   GridBar *bar;
@@ -1856,7 +1917,7 @@ template <typename R> struct StagePersist {
 // tendency and caches written by one phase are read by the next.
 // Occupancy: 3 waves per SIMD, the most that holds the three phases without
 // spilling (4 waves spill 68-136 bytes per lane).
-template <int N, bool CM, typename R, int W>
+template <int N, bool CM, typename R, int W, bool REG>
 __global__ void __launch_bounds__((N * N * 8 + 63) / 64 * 64) __attribute__((amdgpu_waves_per_eu(3)))
     k_stage_persist(KArgs a, StagePersist<R> p, RWStage<R> rw, int stage) {
   if (__hip_atomic_load(&p.bar->err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
@@ -1865,22 +1926,19 @@ __global__ void __launch_bounds__((N * N * 8 + 63) / 64 * 64) __attribute__((amd
   const unsigned xcc = xcc_id() & 15u;
   unsigned nbar = 0, nx = 0, ngroups = 0;
   if (threadIdx.x == 0) __hip_atomic_fetch_add(&p.bar->members[xcc][0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  for (int k = 0; k < p.ncolor; ++k) {
-    const int s0 = p.coff[k], ni = (p.coff[k + 1] - s0) * p.nchunk1;
-    for (int L = b; L < ni; L += G) {
-      fcn1_block<N, 8, CM, R, 1>(L, a, s0, p.nchunk1, ni, p.UR, p.T1, p.U, p.T1th);
-      __syncthreads();  // the next item rewrites the LDS tiles
-    }
-    grid_sync(p.bar, nbar, G, xcc, nx, ngroups, p.deadline);
+  for (int L = b, ni = p.nf * p.nchunk1; L < ni; L += G) {
+    fcn1_block<N, 8, CM, R, 1>(L, a, p.nchunk1, ni, p.UR, p.T1, p.U, p.T1th);
+    __syncthreads();  // the next item rewrites the LDS tiles
   }
-  for (int k = 0; k < p.ncolor; ++k) {
-    const int s0 = p.coff[k], ni = (p.coff[k + 1] - s0) * p.nchunk;
-    for (int L = b; L < ni; L += G) {
-      fcn2_block<N, 8, CM, R, false>(L, a, s0, p.nchunk, p.U, p.UR, p.T1, p.P, p.F, p.F4x, p.T1th);
-      __syncthreads();
-    }
-    grid_sync(p.bar, nbar, G, xcc, nx, ngroups, p.deadline);
+  grid_sync(p.bar, nbar, G, xcc, nx, ngroups, p.deadline);
+  for (int L = b, ni = p.nf * p.nchunk; L < ni; L += G) {
+    if constexpr (REG && std::is_same<R, double>::value)
+      fcn2r_block<N, 8>(L, a, p.nchunk, p.U, p.T1, p.P, p.F, p.F4x, nullptr);
+    else
+      fcn2_block<N, 8, CM, R, false>(L, a, p.nchunk, p.U, p.UR, p.T1, p.P, p.F, p.F4x, p.T1th, nullptr);
+    __syncthreads();
   }
+  grid_sync(p.bar, nbar, G, xcc, nx, ngroups, p.deadline);
   for (unsigned s = blockIdx.x; s < p.stage_blocks; s += G) {
     if (stage == 0) rw_stage_block<0, R, W>(s, a, rw);
     else if (stage == 1) rw_stage_block<1, R, W>(s, a, rw);
@@ -2016,9 +2074,9 @@ __global__ void k_axpy3(double *__restrict__ y, const double *__restrict__ x0, c
 
 // ------------------------------------------------------------------------
 // Context set-up: level-fastest metric for the element kernels.
-// met[slot][c][ID][iz] from dXdxI (3,3,2,NN,Nz,NF), J (NN,2,Nz,NF), X (NN,2,3,Nz,NF)
+// met[element][c][ID][iz] from dXdxI (3,3,2,NN,Nz,NF), J (NN,2,Nz,NF), X (NN,2,3,Nz,NF)
 __global__ void k_relayout_metric(const double *__restrict__ dXdxI, const double *__restrict__ Jm,
-                                  const double *__restrict__ X, const int *__restrict__ slot,
+                                  const double *__restrict__ X, size_t e0,
                                   double *__restrict__ met, double *__restrict__ met1, int NN, int Nz, int NF,
                                   double Omega) {
   const size_t total = (size_t)NF * NN * Nz;
@@ -2036,7 +2094,7 @@ __global__ void k_relayout_metric(const double *__restrict__ dXdxI, const double
                                        Jm[(size_t)ID + (size_t)NN * (0 + 2 * ((size_t)iz + (size_t)Nz * e))],
                                        Jm[(size_t)ID + (size_t)NN * (1 + 2 * ((size_t)iz + (size_t)Nz * e))]};
     const size_t NNZ = (size_t)NN * Nz;
-    const size_t es = (size_t)slot[e];  // stored in colour order
+    const size_t es = e0 + e;
     const size_t mb = (es * CGD_NMET * NN + ID) * (size_t)Nz + iz;
     for (int c = 0; c < CGD_NMET - 1; ++c) met[mb + c * NNZ] = vals[c];
     // CoriolisShallow at the layer midpoint (Coriolis.jl:16-28, MomentumKernel.jl:156-159)
@@ -2057,12 +2115,44 @@ __global__ void k_relayout_metric(const double *__restrict__ dXdxI, const double
   }
 }
 
-// Bit mask of the metric components (met[slot][c][node][iz], ncomp
+// Whether a compact metric is regular (cgd_pass2r_body.inc): flag[0] is set
+// to 1 where it is not.  metn: [NF][12][NN]; met: [NF][5][NN][Nz]; M:
+// [2][NumG][Nz].  Where it is, iMn[g] = 1 / (M1 + M2) (ms: that, per point).
+__global__ void k_met_regular(const double *__restrict__ metn, const double *__restrict__ met,
+                              const double *__restrict__ M, const double *__restrict__ ms, int NF, int NN, int NumG,
+                              int Nz, double *__restrict__ iMn, int *__restrict__ flag) {
+  bool bad = false;
+  const size_t ne = (size_t)NF * NN, np = ne * Nz, ng = (size_t)NumG * Nz;
+  const size_t t0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x, st = (size_t)gridDim.x * blockDim.x;
+  for (size_t q = t0; q < ne; q += st) {
+    const double *m = metn + (q / NN) * CGD_NMETN * NN + q % NN;
+    const int pair[6][2] = {{M111, M112}, {M121, M122}, {M211, M212}, {M221, M222}, {M331, M332}, {MJ1, MJ2}};
+    for (int k = 0; k < 6; ++k)
+      if (!(m[met_nidx(pair[k][0]) * NN] == m[met_nidx(pair[k][1]) * NN])) bad = true;
+  }
+  for (size_t q = t0; q < np; q += st) {
+    const size_t r = q / Nz, e = r / NN, nd = r - e * NN;
+    const int iz = (int)(q - r * Nz);
+    if (iz + 1 >= Nz) continue;
+    const double *m = met + (e * CGD_NMETP * NN + nd) * Nz + iz;
+    const size_t cs = (size_t)NN * Nz;
+    if (!(m[met_pidx(M312) * cs] == m[met_pidx(M311) * cs + 1] && m[met_pidx(M322) * cs] == m[met_pidx(M321) * cs + 1]))
+      bad = true;
+  }
+  for (size_t q = t0; q < ng; q += st) {
+    const size_t g = q / Nz;
+    if (!(M[q] == M[ng + q] && M[q] == M[g * Nz])) bad = true;
+    if (q == g * Nz) iMn[g] = ms[q];
+  }
+  if (bad) *flag = 1;
+}
+
+// Bit mask of the metric components (met[element][c][node][iz], ncomp
 // components) whose value differs between levels of some element node.
 __global__ void k_met_invariant(const double *__restrict__ met, int ncomp, int NF, int NN, int Nz,
                                 unsigned *__restrict__ mask) {
   unsigned m = 0;
-  const size_t total = (size_t)NF * ncomp * NN;  // (slot, c, node) columns
+  const size_t total = (size_t)NF * ncomp * NN;  // (element, c, node) columns
   for (size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x; q < total; q += (size_t)gridDim.x * blockDim.x) {
     const int c = (int)((q / NN) % ncomp);
     const double *col = met + q * Nz;

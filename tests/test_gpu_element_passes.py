@@ -1,0 +1,87 @@
+"""The element kernels and the column kernels at the sizes where they can go
+wrong (edges of level chunks and of wavefronts, both orders), through the C
+ABI, against the CPU oracle.
+
+FP64 results are held to 1e-12 relative L2 per component on a state with
+noise in the wind: the sums have a few dozen terms of 1.1e-16 relative
+rounding each, with cancellation of up to 1e2 in the noisy state.  Steps of
+the mixed mode are held to 1e-5, the bar of that mode's FP32 tendency.
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-12
+
+
+def rel_l2(a, b):
+    den = np.linalg.norm(np.ravel(b))
+    return float(np.linalg.norm(np.ravel(a - b)) / (den if den > 0 else 1.0))
+
+
+@pytest.fixture(scope="module")
+def torch_cuda():
+    import torch
+
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    return torch
+
+
+def noisy_state(pkg, disc, seed):
+    U = pkg.state.jet_state(disc, seed=seed)
+    rng = np.random.default_rng(seed)
+    U[1] += 5.0 * rng.standard_normal(U[1].shape)
+    U[2] += 5.0 * rng.standard_normal(U[2].shape)
+    U[3] += 0.5 * rng.standard_normal(U[3].shape)
+    U[3][:, -1] = 0.0
+    return U
+
+
+def setup(pkg, oracle_mod, ne, p, nz, H=30000.0, **kw):
+    disc = pkg.discretization.build(ne, p, nz, H)
+    phys = pkg.discretization.Phys()
+    dev = pkg.host.device_setup(disc, phys, device="cuda", **kw)
+    hd = pkg.host.hyperdiffusion_for(ne)
+    kw.pop("precision", None)
+    orc = oracle_mod.Oracle(disc, phys, (hd, hd, hd), **kw)
+    return disc, phys, dev, orc
+
+
+def tendency(torch, host, phys, dev, U0):
+    FE, Metric, Global, Cache, JCache = dev
+    U = torch.as_tensor(U0, device="cuda")
+    F = torch.full_like(U, 7.0)
+    eq = host.CompressibleShallow()
+    host.FcnPrepareGPU(U, FE, Metric, phys, Cache, None, Global, None, eq)
+    host.FcnGPU(F, U, FE, Metric, phys, Cache, None, Global, None, eq)
+    torch.cuda.synchronize()
+    return F.cpu().numpy(), Cache.Temp1.cpu().numpy()
+
+
+@pytest.mark.parametrize("metric", ["regular", "compact", "full"])
+@pytest.mark.parametrize("H", [30000.0, None])
+@pytest.mark.parametrize("p,nz,chunk", [(4, 3, 8), (4, 8, 8), (4, 9, 8), (4, 17, 16), (4, 31, 16), (3, 7, 8),
+                                        (3, 16, 8), (3, 25, 8)])
+def test_tendency_metric_kernels(pkg, oracle_mod, torch_cuda, monkeypatch, metric, p, nz, chunk, H):
+    """The tendency kernel of a regular metric, the general one on the same
+    metric, and the full layout; every face, edge and corner of the sphere
+    sums its element copies (ne = 2: every element touches a corner).  With
+    layers of 512 m (H = None) the metric for p = 4 is the same at all levels
+    to the bit, as the regular and the compact layout ask."""
+    if metric != "regular":
+        monkeypatch.setenv("CGD_METRIC", metric)
+    print(f"tendency {metric} p={p} nz={nz} chunk={chunk}", flush=True)
+    disc, phys, dev, orc = setup(pkg, oracle_mod, 2, p, nz, H=H or 512.0 * nz)
+    ctx = pkg.host.init_context(dev[0], dev[1], phys, dev[2])
+    ctx.set_launch_shape(chunk_levels=chunk)
+    if metric == "full" or (H is None and p == 4):
+        assert ctx.info()[2] == (metric != "full")
+    U0 = noisy_state(pkg, disc, 3)
+    F, T1 = tendency(torch_cuda, pkg.host, phys, dev, U0)
+    Fo, T1o = orc.fcn(U0.copy(), orc.prepare(U0.copy()))
+    for v in range(5):
+        assert rel_l2(T1[v], T1o[v]) <= TOL, f"Temp1[{v}] {rel_l2(T1[v], T1o[v]):.3e}"
+        assert rel_l2(F[v], Fo[v]) <= TOL, f"F{v + 1} {rel_l2(F[v], Fo[v]):.3e}"
+    assert np.all(F[3][:, -1] == 0.0)
