@@ -63,6 +63,7 @@ struct cgd_ctx {
   // column launch shape of the fused stage kernel: lanes per column (64,
   // or 32 for two columns per wavefront when Nz <= 32) and workgroup size
   int colw = 64, colblock = 256;
+  int col1 = 0;    // pass 1 over whole columns (k_fcn1c), until its chunk height is set
   int items1 = 1;  // pass-1 work items (element, level chunk) per workgroup: 1 or 2
   // one persistent launch per RW stage (k_stage_persist): on/off, its grid
   // (workgroups resident at once), the grid barrier's state and wait bound
@@ -102,6 +103,9 @@ template <typename R> static size_t lds_fcn2(const cgd_ctx *c) {
   if (std::is_same<R, double>::value) return base + r;
   return base + (r + 7) / 8 * 8 + sizeof(double) * (c->NN + 3 * c->NN * c->nzt);
 }
+
+// k_fcn1c: three tiles of whole columns, one of them FP64
+static size_t lds_fcn1c(const cgd_ctx *c, size_t r) { return (size_t)c->NN * 64 * (sizeof(double) + 2 * r); }
 
 // k_fcn2r: D, DW, 12 tiles, four tiles with the level below, its sums, the
 // horizontal metric and 1/(2 M)
@@ -688,6 +692,8 @@ static int ctx_build(cgd_ctx *c, const cgd_desc *ds, int nmem, hipStream_t st) {
     for (int k = 0; k < c->N; ++k) {
       a.D[i * c->N + k] = hds[i + c->N * k];
       a.DWm[i * c->N + k] = hdw[i + c->N * k];
+      a.Df[i * c->N + k] = (float)a.D[i * c->N + k];
+      a.DWf[i * c->N + k] = (float)a.DWm[i * c->N + k];
     }
   a.glob = c->d_glob;
   a.clist = c->d_clist;
@@ -721,6 +727,10 @@ static int ctx_build(cgd_ctx *c, const cgd_desc *ds, int nmem, hipStream_t st) {
     HIPCHK(c, hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev));
     c->bar_ticks = (long long)std::max(khz, 1000) * 250;  // 250 ms
   }
+  // Pass 1 over whole columns has a lane per level: at Nz = 64 it takes 127 us
+  // instead of 190 (ne = 30), at Nz = 40 the idle lanes make it 1 % slower
+  // than the chunks, so it is taken from three quarters of a wavefront on.
+  c->col1 = c->cm && Nz >= 48 && Nz <= 64;
   c->ok = true;
   return CGD_OK;
 }
@@ -899,6 +909,12 @@ static void tr2lim_t(cgd_ctx *c, int nitems, hipStream_t st, int slot0, const do
 
 template <typename R>
 static void launch_fcn1(cgd_ctx *c, int nitems, hipStream_t st, const R *UR, R *E, const double *U64, double *Eth) {
+  if (c->col1) {
+    const size_t lds = lds_fcn1c(c, sizeof(R));
+    if (c->N == 5) hipLaunchKernelGGL((k_fcn1c<5, R>), dim3(c->NF), dim3(320), lds, st, c->ka, UR, E, U64, Eth);
+    else hipLaunchKernelGGL((k_fcn1c<4, R>), dim3(c->NF), dim3(256), lds, st, c->ka, UR, E, U64, Eth);
+    return;
+  }
   CGD_DISPATCH(fcn1_t, R, c->nzt1, nitems, st, UR, E, U64, Eth);
 }
 template <typename R>
@@ -1384,6 +1400,7 @@ extern "C" int cgd_set_launch_shape(cgd_ctx *c, const cgd_launch_shape *shape) {
                 "-1; a persistent launch takes chunk heights 8, pass1_items 1 and col_block = 64 * ceil(N*N*8 / 64)");
   graph_free(c);  // a captured graph keeps the old shapes
   apply_shape(c, sh);
+  if (shape->pass1_chunk_levels) c->col1 = 0;
   return CGD_OK;
 }
 

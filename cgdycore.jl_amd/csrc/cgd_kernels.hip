@@ -43,6 +43,7 @@ struct KArgs {
   double Rd_p0, eos_y, dpd_y;      // Rd/p0, 1/(1-kappa), kappa/(1-kappa)
   double D[CGD_NMAX * CGD_NMAX];   // D[i*N + k] = DS[i,k]
   double DWm[CGD_NMAX * CGD_NMAX]; // DW[i*N + k]
+  float Df[CGD_NMAX * CGD_NMAX], DWf[CGD_NMAX * CGD_NMAX];  // both in FP32 (mixed precision)
   const int *glob;                 // [e][NN]: 0-based node | bit 31 set on the node's first copy (colour order)
   const int *clist;                // elements by colour (the tracer and adjoint kernels' launch order)
   const int *cpy;                  // [e][NN][cpw]: the node's copies e'*NN + node' in colour order, then -1
@@ -128,6 +129,14 @@ template <typename T> __device__ __forceinline__ T &at(T *base, unsigned i) {
 }
 template <typename T> __device__ __forceinline__ const T &at(const T *base, unsigned i) {
   return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + i * (unsigned)sizeof(T));
+}
+
+// A table that nothing writes while the kernel runs, at a uniform address:
+// read through the constant address space, so that the loads are scalar ones
+// (the compiler cannot tell the kernel's stores from the tables otherwise).
+template <typename T> using Const = const __attribute__((address_space(4))) T *;
+template <typename T> __device__ __forceinline__ Const<T> as_const(const T *p) {
+  return (Const<T>)reinterpret_cast<uintptr_t>(p);
 }
 
 // The value of x in lane `lane` (uniform), on every lane.
@@ -362,6 +371,20 @@ template <int N, typename R> __device__ __forceinline__ void load_dmats(const KA
   }
 }
 
+// any_value: an unspecified value, for a variable that only some lanes set
+// (no instruction to initialise it).
+// pin computes its arguments here: an empty asm that reads and writes them, so
+// that the code generator, which orders arithmetic within a block by its
+// own measure, does not hold the inputs of a long block's later sums (LDS
+// values, neighbour levels) in registers and spill them.
+__device__ __forceinline__ double any_value() { return __builtin_nondeterministic_value(0.0); }
+__device__ __forceinline__ void pin(double &x) { asm volatile("" : "+v"(x)); }
+__device__ __forceinline__ void pin(float &x) { asm volatile("" : "+v"(x)); }
+template <typename R, typename... D> __device__ __forceinline__ void pin(R &x, D &...y) {
+  pin(x);
+  pin(y...);
+}
+
 // ------------------------------------------------------------------------
 // Pass 1: HyperViscKernel! (src/GPU/ViscKernel.jl:1-84).
 // Grid: one workgroup per ITEMS consecutive work items, an
@@ -566,6 +589,136 @@ __global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64) k_fcn1(KArgs a, 
 #undef CGD_ITEM
 }
 
+// Pass 1 over whole columns (compact metric, Nz <= 64): one workgroup per
+// element, one wavefront per row J of its nodes, lane = level, so a lane
+// holds the N nodes of its row.
+// - Every load and store is one node's column, a whole run of 8 Nz bytes; the
+//   chunked kernel's 64-byte pieces are what bounds it (724 us at ne = 60,
+//   nz = 64, all of it loads and stores); the same bytes in columns take
+//   450 us, this kernel 503 us.
+// - The derivatives along the row need no LDS, and the node's metric, the
+//   derivative matrices and the addresses are uniform (scalar registers);
+//   only the derivatives across the rows exchange values through LDS.
+// The operations are those of k_fcn1, term by term.
+template <int N, typename R>
+__device__ __forceinline__ void fcn1c_block(int e, const KArgs &a, const R *__restrict__ U, R *__restrict__ E,
+                                            const double *__restrict__ U64, double *__restrict__ Eth) {
+  constexpr int NN = N * N;
+  constexpr bool F32 = !std::is_same<R, double>::value;
+  extern __shared__ double smem[];
+  double *TD = smem;                                     // theta, then its flux across the rows
+  R *T0 = reinterpret_cast<R *>(smem + NN * 64), *T1 = T0 + NN * 64;  // the curl's and the divergence's
+  const int Nz = a.Nz;
+  const int lane = threadIdx.x & 63, J = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const bool valid = lane < Nz;
+  const unsigned iz = valid ? lane : Nz - 1;
+  const size_t vs = (size_t)a.NumG * Nz;
+  const Const<int> gE = as_const(a.glob + (size_t)e * NN + J * N);
+  const Const<double> mE = as_const(a.met1n + (size_t)e * CGD_NMET1 * NN + J * N);
+  const R *iMsR = F32 ? reinterpret_cast<const R *>(a.iMs32) : reinterpret_cast<const R *>(a.iMs);
+  const R *Dm = F32 ? reinterpret_cast<const R *>(a.Df) : reinterpret_cast<const R *>(a.D);
+  const R *DWm = F32 ? reinterpret_cast<const R *>(a.DWf) : reinterpret_cast<const R *>(a.DWm);
+  R u[N], v[N], iMs[N];
+  double rho[N], rth[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const size_t c0 = (size_t)(gE[i] & 0x7fffffff) * Nz;
+    u[i] = at(U + vs + c0, iz);
+    v[i] = at(U + 2 * vs + c0, iz);
+    rho[i] = at(U64 + c0, iz);
+    rth[i] = at(U64 + 4 * vs + c0, iz);
+    iMs[i] = at(iMsR + c0, iz);
+  }
+  R uC[N], uD[N];
+  double Th[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const R S11 = R(mE[i]), S12 = R(mE[NN + i]), S21 = R(mE[2 * NN + i]), S22 = R(mE[3 * NN + i]);
+    const int o = (J * N + i) * 64 + lane;
+    uC[i] = S11 * v[i] - S12 * u[i];  // Curl12
+    T0[o] = S21 * v[i] - S22 * u[i];
+    uD[i] = S11 * u[i] + S12 * v[i];  // Contra12
+    T1[o] = S21 * u[i] + S22 * v[i];
+    Th[i] = rth[i] * rcp(rho[i]);
+    TD[o] = Th[i];
+  }
+  __syncthreads();
+  R Curl[N], Div[N];
+  double ThCx[N], ThCy[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    R cu = Dm[i * N] * uC[0] + Dm[J * N] * T0[i * 64 + lane];
+    R dv = Dm[i * N] * uD[0] + Dm[J * N] * T1[i * 64 + lane];
+    double cx = a.D[i * N] * Th[0], cy = a.D[J * N] * TD[i * 64 + lane];
+#pragma unroll
+    for (int q = 1; q < N; ++q) {
+      const int o = (i + q * N) * 64 + lane;
+      cu += Dm[i * N + q] * uC[q] + Dm[J * N + q] * T0[o];
+      dv += Dm[i * N + q] * uD[q] + Dm[J * N + q] * T1[o];
+      cx += a.D[i * N + q] * Th[q];
+      cy += a.D[J * N + q] * TD[o];
+    }
+    const double S11 = R(mE[i]), S12 = R(mE[NN + i]), S21 = R(mE[2 * NN + i]), S22 = R(mE[3 * NN + i]);
+    const R Js = R(mE[4 * NN + i]);
+    const R iJs = rcp(Js);
+    Curl[i] = cu * iJs;
+    Div[i] = dv * iJs;
+    const double iJd = rcp(double(Js));
+    const double gx = (S11 * cx + S21 * cy) * iJd;  // Grad12 with J
+    const double gy = (S12 * cx + S22 * cy) * iJd;
+    ThCx[i] = S11 * gx + S12 * gy;  // Contra12
+    ThCy[i] = S21 * gx + S22 * gy;
+    pin(Curl[i], Div[i], ThCx[i], ThCy[i]);
+  }
+  __syncthreads();  // the tiles have been read
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const int o = (J * N + i) * 64 + lane;
+    T0[o] = Curl[i];
+    T1[o] = Div[i];
+    TD[o] = ThCy[i];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    R xC = DWm[i * N] * Curl[0], yC = DWm[J * N] * T0[i * 64 + lane];
+    R xD = DWm[i * N] * Div[0], yD = DWm[J * N] * T1[i * 64 + lane];
+    double dt = a.DWm[i * N] * ThCx[0] + a.DWm[J * N] * TD[i * 64 + lane];
+#pragma unroll
+    for (int q = 1; q < N; ++q) {
+      const int o = (i + q * N) * 64 + lane;
+      xC += DWm[i * N + q] * Curl[q];
+      yC += DWm[J * N + q] * T0[o];
+      xD += DWm[i * N + q] * Div[q];
+      yD += DWm[J * N + q] * T1[o];
+      dt += a.DWm[i * N + q] * ThCx[q] + a.DWm[J * N + q] * TD[o];
+    }
+    const R S11 = R(mE[i]), S12 = R(mE[NN + i]), S21 = R(mE[2 * NN + i]), S22 = R(mE[3 * NN + i]);
+    const R FuC = S12 * xC + S22 * yC;  // Rot12
+    const R FvC = -S11 * xC - S21 * yC;
+    const R FuD = S11 * xD + S21 * yD;  // Grad12
+    const R FvD = S12 * xD + S22 * yD;
+    R o1 = -FuC * iMs[i], o2 = -FvC * iMs[i], o3 = FuD * iMs[i], o4 = FvD * iMs[i];
+    double o5 = dt * double(iMs[i]);
+    pin(o1, o2, o3, o4, o5);
+    if (valid) {
+      R *Ea = E + ((size_t)e * NN + J * N + i) * Nz;
+      at(Ea, iz) = o1;
+      at(Ea + a.ecs, iz) = o2;
+      at(Ea + 2 * a.ecs, iz) = o3;
+      at(Ea + 3 * a.ecs, iz) = o4;
+      if constexpr (F32) at(Eth + ((size_t)e * NN + J * N + i) * Nz, iz) = o5;
+      else at(Ea + 4 * a.ecs, iz) = o5;
+    }
+  }
+}
+
+template <int N, typename R>
+__global__ void __launch_bounds__(N * 64) __attribute__((amdgpu_waves_per_eu(5))) k_fcn1c(KArgs a, const R *__restrict__ U, R *__restrict__ E,
+                                                  const double *__restrict__ U64, double *__restrict__ Eth) {
+  fcn1c_block<N, R>(xcd_logical(blockIdx.x, gridDim.x), a, U, E, U64, Eth);
+}
+
 // ------------------------------------------------------------------------
 // Pass 2: HyperViscKoeffKernel! + MomentumVectorInvariantCoriolisKernel! +
 // GradFullKernel! + DivRhoTrUpwind3New2Kernel! fused into one element pass
@@ -618,19 +771,6 @@ __global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64) __attribute__((a
 #include "cgd_pass2_body.inc"
 #undef CGD_EARLY_HALO
 #undef CGD_ITEM
-}
-
-// any_value: an unspecified value, for a variable that only some lanes set
-// (no instruction to initialise it).
-// pin computes its arguments here: an empty asm that reads and writes them, so
-// that the code generator, which orders arithmetic within a block by its
-// own measure, does not hold the inputs of a long block's later sums (LDS
-// values, neighbour levels) in registers and spill them.
-__device__ __forceinline__ double any_value() { return __builtin_nondeterministic_value(0.0); }
-__device__ __forceinline__ void pin(double &x) { asm volatile("" : "+v"(x)); }
-template <typename... D> __device__ __forceinline__ void pin(double &x, D &...y) {
-  pin(x);
-  pin(y...);
 }
 
 // Pass 2 for the regular compact metric (FP64): the same terms, reduced by

@@ -85,3 +85,36 @@ def test_tendency_metric_kernels(pkg, oracle_mod, torch_cuda, monkeypatch, metri
         assert rel_l2(T1[v], T1o[v]) <= TOL, f"Temp1[{v}] {rel_l2(T1[v], T1o[v]):.3e}"
         assert rel_l2(F[v], Fo[v]) <= TOL, f"F{v + 1} {rel_l2(F[v], Fo[v]):.3e}"
     assert np.all(F[3][:, -1] == 0.0)
+
+
+@pytest.mark.parametrize("chunk", [0, 8])
+@pytest.mark.parametrize("p,nz", [(4, 47), (4, 48), (4, 63), (3, 48), (3, 64)])
+def test_pass1_columns(pkg, oracle_mod, torch_cuda, p, nz, chunk):
+    """Pass 1 over whole columns (48 <= nz <= 64 unless a chunk height is set)
+    and in level chunks, and in the mixed mode's steps."""
+    torch, host = torch_cuda, pkg.host
+    print(f"pass 1 p={p} nz={nz} chunk={chunk}", flush=True)
+    disc, phys, dev, orc = setup(pkg, oracle_mod, 2, p, nz)
+    ctx = host.init_context(dev[0], dev[1], phys, dev[2])
+    if chunk:
+        ctx.set_launch_shape(pass1_chunk_levels=chunk)
+    U0 = noisy_state(pkg, disc, 4)
+    F, T1 = tendency(torch, host, phys, dev, U0)
+    Fo, T1o = orc.fcn(U0.copy(), orc.prepare(U0.copy()))
+    for v in range(5):
+        assert rel_l2(T1[v], T1o[v]) <= TOL, f"Temp1[{v}] {rel_l2(T1[v], T1o[v]):.3e}"
+        assert rel_l2(F[v], Fo[v]) <= TOL, f"F{v + 1} {rel_l2(F[v], Fo[v]):.3e}"
+    disc, phys, dev, orc = setup(pkg, oracle_mod, 2, p, nz, precision="mixed")
+    FE, Metric, Global, Cache, JCache = dev
+    ctx = host.init_context(FE, Metric, phys, Global)
+    if chunk:
+        ctx.set_launch_shape(pass1_chunk_levels=chunk)
+    U0 = pkg.state.jet_state(disc, seed=5)
+    V = torch.as_tensor(U0, device="cuda").clone()
+    host.TimeStepper(V, 300.0, 2, FE, Metric, phys, Cache, JCache, Global)
+    torch.cuda.synchronize()
+    Vo = U0.copy()
+    orc.rw_step(Vo, 300.0, 2)
+    for c in range(5):
+        e = rel_l2(V[c].cpu().numpy(), Vo[c])
+        assert e <= 1e-5, f"mixed V{c + 1} {e:.3e}"
