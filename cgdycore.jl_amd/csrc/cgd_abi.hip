@@ -976,12 +976,6 @@ static int run_fcn(cgd_ctx *c, R *F, const double *U, const R *UR, R *Temp1, con
   launch_fcn2<R>(c, dim3(c->NF * c->nchunk), st, U, UR, E1, AuxG, E2, E1th, want_f ? T1d : nullptr);
   HIPCHK(c, hipGetLastError());
   ++launches;
-  if (want_f || has_hooks(c)) {
-    hipLaunchKernelGGL((k_dss<R>), dim3(grid_for((size_t)c->NumG * c->Nz, 256)), dim3(256), 0, st, c->ka, E2,
-                       reinterpret_cast<const R *>(c->d_f4x), F, c->nchunk, c->nzt);
-    HIPCHK(c, hipGetLastError());
-    ++launches;
-  }
   {
     if (c->ntr > 0 && c->horlimit) {
       // LimitKernel! on the state, then DivRhoTrUpwind3LimKernel! per colour
@@ -1008,9 +1002,15 @@ static int run_fcn(cgd_ctx *c, R *F, const double *U, const R *UR, R *Temp1, con
       }
     }
   }
-  if (has_hooks(c)) {
-    const size_t n = (size_t)c->NumG * c->Nz;
-    hipLaunchKernelGGL((k_hooks<R>), dim3(grid_for(n, 256)), dim3(256), 0, st, c->ka, c->hooks, U, AuxG, F, Fd, n);
+  if (want_f || has_hooks(c)) {
+    const dim3 g(grid_for((size_t)c->NumG * c->Nz, 256));
+    const R *F4x = reinterpret_cast<const R *>(c->d_f4x);
+    if (has_hooks(c))
+      hipLaunchKernelGGL((k_dss<R, true>), g, dim3(256), 0, st, c->ka, c->hooks, U, AuxG, E2, F4x, F, Fd,
+                         c->nchunk, c->nzt);
+    else
+      hipLaunchKernelGGL((k_dss<R, false>), g, dim3(256), 0, st, c->ka, c->hooks, U, AuxG, E2, F4x, F, Fd,
+                         c->nchunk, c->nzt);
     HIPCHK(c, hipGetLastError());
     ++launches;
   }

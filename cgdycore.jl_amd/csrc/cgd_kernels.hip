@@ -808,66 +808,65 @@ struct Hooks {
   const double *xS;  // (2, NumG)
   const double *zP;  // (Nz, NumG)
 };
-// F: the tendency of the dynamics (R-typed); Ftr: the same buffer as FP64,
-// whose components 6.. are the tracers' tendencies in both modes
+// s: the five components of the dynamics' tendency at point i (R-typed);
+// Ftr: the FP64 tendency array, whose components 6.. are the tracers'
 template <typename R>
-__global__ void k_hooks(KArgs a, Hooks hk, const double *__restrict__ U, const double *__restrict__ P,
-                        R *__restrict__ F, double *__restrict__ Ftr, size_t n) {
+__device__ __forceinline__ void hooks_point(const KArgs &a, const Hooks &hk, const double *__restrict__ U,
+                                            const double *__restrict__ P, R (&s)[5], double *__restrict__ Ftr,
+                                            size_t i, size_t n) {
   const size_t vs = n;
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-    if (hk.forcing) {
-      const size_t ig = i / a.Nz;
-      const double rho = U[i], u = U[vs + i], v = U[2 * vs + i];
-      const double lat = hk.xS[2 * ig + 1];
-      const double Sigma = P[i] / a.p0;
-      const double SigmaPowKappa = exp(a.kappa * log(Sigma));  // fast_powGPU
-      const double hf = jmax(0.0, (Sigma - hk.sigma_b) / (1.0 - hk.sigma_b));
-      const double coslat = cos(lat), sinlat = sin(lat);
-      F[vs + i] = R(double(F[vs + i]) + -(hk.k_f * hf) * u);
-      F[2 * vs + i] = R(double(F[2 * vs + i]) + -(hk.k_f * hf) * v);
-      const double kT = Sigma < 0.7 ? hk.k_a + (hk.k_s - hk.k_a) * hf * coslat * coslat * coslat * coslat : 0.0;
-      double Teq = (hk.T_equator - hk.DeltaT_y * sinlat * sinlat - hk.DeltaTh_z * log(Sigma) * coslat * coslat) *
-                   SigmaPowKappa;
-      Teq = jmax(hk.T_min, Teq);
-      const double DeltaT = kT * (a.p0 * Sigma / (rho * a.Rd) - Teq);
-      F[4 * vs + i] = R(double(F[4 * vs + i]) + -rho * DeltaT / SigmaPowKappa);
-    }
-    if (hk.micro) {
-      // SimpleMicrophysics (src/Models/Microphysics.jl:6-40) through
-      // MicrophysicsKernel! (OperatorKernel.jl:1082-1089): relaxation of the
-      // vapour towards saturation (fpvs, src/Thermodynamics/Thermodynamics.jl:27-35)
-      // through cloud, the latent heating in rho*theta (LatHeat, :83-85), and
-      // the rain-out fraction Rain of the condensate leaving rho
-      const double p = P[i];
-      const double Rho = U[i], RhoTh = U[4 * vs + i];
-      const double RhoV = jmax(U[(size_t)a.iv * vs + i], 0.0), RhoC = jmax(U[(size_t)a.ic * vs + i], 0.0);
-      const double RhoD = Rho - RhoV - RhoC;
-      const double Cpml = a.Cpd * RhoD + a.Cpv * RhoV + a.Cpl * RhoC;
-      const double Rm = a.Rd * RhoD + a.Rv * RhoV;
-      const double T = p / Rm;
-      const double T_C = T - hk.T0;
-      const double p_vs = 611.2 * exp(17.62 * T_C / (243.12 + T_C));
-      const double am = p_vs / (a.Rv * T) - RhoV;
-      const double bm = RhoC;
-      const double FPh = 0.5 * hk.RelCloud * (am + bm - sqrt(am * am + bm * bm));
-      const double L = hk.L00 - (a.Cpl - a.Cpv) * (T - hk.T0);
-      const double FR = -FPh * hk.Rain;
-      const double lp = log(p / a.p0);
-      const double FRhoTh =
-          RhoTh * ((-L / (Cpml * T) - lp * (Rm / Cpml) * (a.Rv / Rm + (a.Cpl - a.Cpv) / Cpml) + a.Rv / Rm) * FPh +
-                   (1.0 / Rho - lp * (Rm / Cpml) * (a.Cpl / Cpml)) * FR);
-      F[i] = R(double(F[i]) + -FR);
-      F[4 * vs + i] = R(double(F[4 * vs + i]) + FRhoTh);
-      Ftr[(size_t)a.iv * vs + i] += FPh;
-      Ftr[(size_t)a.ic * vs + i] += -FPh - FR;
-    }
-    if (hk.damping) {
-      const double z = hk.zP[i];
-      if (z >= hk.H - hk.Stride) {
-        const double sn = sin(0.5 * M_PI * (1.0 - (hk.H - z) / hk.Stride));
-        const double Damp = hk.Relax * (sn * sn);
-        F[3 * vs + i] = R(double(F[3 * vs + i]) + -Damp * U[3 * vs + i]);
-      }
+  if (hk.forcing) {
+    const size_t ig = i / a.Nz;
+    const double rho = U[i], u = U[vs + i], v = U[2 * vs + i];
+    const double lat = hk.xS[2 * ig + 1];
+    const double Sigma = P[i] / a.p0;
+    const double SigmaPowKappa = exp(a.kappa * log(Sigma));  // fast_powGPU
+    const double hf = jmax(0.0, (Sigma - hk.sigma_b) / (1.0 - hk.sigma_b));
+    const double coslat = cos(lat), sinlat = sin(lat);
+    s[1] = R(double(s[1]) + -(hk.k_f * hf) * u);
+    s[2] = R(double(s[2]) + -(hk.k_f * hf) * v);
+    const double kT = Sigma < 0.7 ? hk.k_a + (hk.k_s - hk.k_a) * hf * coslat * coslat * coslat * coslat : 0.0;
+    double Teq = (hk.T_equator - hk.DeltaT_y * sinlat * sinlat - hk.DeltaTh_z * log(Sigma) * coslat * coslat) *
+                 SigmaPowKappa;
+    Teq = jmax(hk.T_min, Teq);
+    const double DeltaT = kT * (a.p0 * Sigma / (rho * a.Rd) - Teq);
+    s[4] = R(double(s[4]) + -rho * DeltaT / SigmaPowKappa);
+  }
+  if (hk.micro) {
+    // SimpleMicrophysics (src/Models/Microphysics.jl:6-40) through
+    // MicrophysicsKernel! (OperatorKernel.jl:1082-1089): relaxation of the
+    // vapour towards saturation (fpvs, src/Thermodynamics/Thermodynamics.jl:27-35)
+    // through cloud, the latent heating in rho*theta (LatHeat, :83-85), and
+    // the rain-out fraction Rain of the condensate leaving rho
+    const double p = P[i];
+    const double Rho = U[i], RhoTh = U[4 * vs + i];
+    const double RhoV = jmax(U[(size_t)a.iv * vs + i], 0.0), RhoC = jmax(U[(size_t)a.ic * vs + i], 0.0);
+    const double RhoD = Rho - RhoV - RhoC;
+    const double Cpml = a.Cpd * RhoD + a.Cpv * RhoV + a.Cpl * RhoC;
+    const double Rm = a.Rd * RhoD + a.Rv * RhoV;
+    const double T = p / Rm;
+    const double T_C = T - hk.T0;
+    const double p_vs = 611.2 * exp(17.62 * T_C / (243.12 + T_C));
+    const double am = p_vs / (a.Rv * T) - RhoV;
+    const double bm = RhoC;
+    const double FPh = 0.5 * hk.RelCloud * (am + bm - sqrt(am * am + bm * bm));
+    const double L = hk.L00 - (a.Cpl - a.Cpv) * (T - hk.T0);
+    const double FR = -FPh * hk.Rain;
+    const double lp = log(p / a.p0);
+    const double FRhoTh =
+        RhoTh * ((-L / (Cpml * T) - lp * (Rm / Cpml) * (a.Rv / Rm + (a.Cpl - a.Cpv) / Cpml) + a.Rv / Rm) * FPh +
+                 (1.0 / Rho - lp * (Rm / Cpml) * (a.Cpl / Cpml)) * FR);
+    s[0] = R(double(s[0]) + -FR);
+    s[4] = R(double(s[4]) + FRhoTh);
+    Ftr[(size_t)a.iv * vs + i] += FPh;
+    Ftr[(size_t)a.ic * vs + i] += -FPh - FR;
+  }
+  if (hk.damping) {
+    const double z = hk.zP[i];
+    if (z >= hk.H - hk.Stride) {
+      const double sn = sin(0.5 * M_PI * (1.0 - (hk.H - z) / hk.Stride));
+      const double Damp = hk.Relax * (sn * sn);
+      s[3] = R(double(s[3]) + -Damp * U[3 * vs + i]);
     }
   }
 }
@@ -1535,11 +1534,13 @@ __global__ void k_rw_tr(const double *__restrict__ fV, const double *__restrict_
 // The tendency of the dynamics from its element copies E: F = the sum over
 // each node's copies in colour order, plus for w the chunk-interface terms
 // (the lower-interface terms of the first levels of the chunks above, F4x).
-// For callers that want F itself (cgd_fcn, the physics hooks); the stage
+// For callers that want F itself (cgd_fcn) and for the physics hooks (HK),
+// which add to the sums before they are stored; without hooks the stage
 // kernel sums the copies in registers instead.
-template <typename R>
-__global__ void k_dss(KArgs a, const R *__restrict__ E, const R *__restrict__ F4x, R *__restrict__ F, int nchunk,
-                      int nzt) {
+template <typename R, bool HK>
+__global__ void k_dss(KArgs a, Hooks hk, const double *__restrict__ U, const double *__restrict__ P,
+                      const R *__restrict__ E, const R *__restrict__ F4x, R *__restrict__ F, double *__restrict__ Ftr,
+                      int nchunk, int nzt) {
   const int Nz = a.Nz;
   const size_t vs = (size_t)a.NumG * Nz;
   for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < vs; i += (size_t)gridDim.x * blockDim.x) {
@@ -1573,6 +1574,7 @@ __global__ void k_dss(KArgs a, const R *__restrict__ E, const R *__restrict__ F4
       }
     }
     if (edge) s[3] += s4;
+    if constexpr (HK) hooks_point<R>(a, hk, U, P, s, Ftr, i, vs);
 #pragma unroll
     for (int q = 0; q < 5; ++q) F[q * vs + i] = s[q];
   }

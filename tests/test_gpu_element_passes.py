@@ -118,3 +118,31 @@ def test_pass1_columns(pkg, oracle_mod, torch_cuda, p, nz, chunk):
     for c in range(5):
         e = rel_l2(V[c].cpu().numpy(), Vo[c])
         assert e <= 1e-5, f"mixed V{c + 1} {e:.3e}"
+
+
+@pytest.mark.parametrize("p,nz,ntr", [(3, 7, 0), (4, 11, 0), (3, 50, 2)])
+def test_hooks_with_the_copies(pkg, oracle_mod, torch_cuda, p, nz, ntr):
+    """Forcing and damping where the copies are summed (point counts that no
+    workgroup divides), in the tendency and in the step."""
+    torch, host = torch_cuda, pkg.host
+    damping = (30000.0, 12000.0, 0.05)
+    print(f"hooks p={p} nz={nz} NumTr={ntr}", flush=True)
+    disc = pkg.discretization.build(2, p, nz, 30000.0)
+    phys = pkg.discretization.Phys()
+    dev = host.device_setup(disc, phys, device="cuda", NumTr=ntr, damping=damping, forcing=True)
+    FE, Metric, Global, Cache, JCache = dev
+    hd = host.hyperdiffusion_for(2)
+    orc = oracle_mod.Oracle(disc, phys, (hd, hd, hd), NumTr=ntr, damping=damping, forcing=host.held_suarez_param())
+    U0 = noisy_state(pkg, disc, 6)
+    U0 = np.concatenate([U0] + [0.01 * (t + 1) * U0[0:1] for t in range(ntr)], axis=0)
+    F, _ = tendency(torch, host, phys, dev, U0)
+    Fo, _ = orc.fcn(U0.copy(), orc.prepare(U0.copy()))
+    for v in range(5 + ntr):
+        assert rel_l2(F[v], Fo[v]) <= TOL, f"F{v + 1} {rel_l2(F[v], Fo[v]):.3e}"
+    V = torch.as_tensor(U0, device="cuda").clone()
+    host.TimeStepper(V, 100.0, 2, FE, Metric, phys, Cache, JCache, Global)
+    torch.cuda.synchronize()
+    Vo = U0.copy()
+    orc.rw_step(Vo, 100.0, 2)
+    for v in range(5 + ntr):
+        assert rel_l2(V[v].cpu().numpy(), Vo[v]) <= TOL, f"V{v + 1} {rel_l2(V[v].cpu().numpy(), Vo[v]):.3e}"
