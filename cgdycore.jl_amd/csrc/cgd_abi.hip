@@ -27,7 +27,7 @@ struct cgd_ctx {
   int *d_clist = nullptr;      // elements by colour, ascending within one
   int *d_cpy = nullptr, *d_gcpy = nullptr;  // the copies of each element node / global node, colour order
   double *d_e1 = nullptr, *d_e2 = nullptr;  // element copies of the pass-1 cache and of the tendency (5 each)
-  double *d_met = nullptr, *d_met1 = nullptr, *d_ms = nullptr, *d_bwork = nullptr;
+  double *d_met = nullptr, *d_met1 = nullptr, *d_ms = nullptr;
   double *d_metn = nullptr, *d_met1n = nullptr;  // compact metric layout: per element node
   int cm = 0;                                    // 1: compact metric layout
   int reg = 0;                                   // 1: regular compact metric (k_fcn2r)
@@ -535,7 +535,6 @@ static int ctx_build(cgd_ctx *c, const cgd_desc *ds, int nmem, hipStream_t st) {
   HIPCHK(c, hipMalloc(&c->d_met, npt * CGD_NMET * sizeof(double)));
   HIPCHK(c, hipMalloc(&c->d_met1, npt * CGD_NMET1 * sizeof(double)));
   HIPCHK(c, hipMalloc(&c->d_ms, ng * sizeof(double)));
-  HIPCHK(c, hipMalloc(&c->d_bwork, (size_t)NumG * (Nz - 1) * sizeof(double)));
   HIPCHK(c, hipMalloc(&c->d_f4x, (size_t)NF * NN * nchunk_max * sizeof(double)));
   HIPCHK(c, hipMalloc(&c->d_nptr, cptr.size() * sizeof(int)));
   HIPCHK(c, hipMalloc(&c->d_ncopy, ccopy.size() * sizeof(int)));
@@ -768,7 +767,7 @@ extern "C" int cgd_ctx_destroy(cgd_ctx *c) {
   for (void *p : {(void *)c->d_glob, (void *)c->d_clist, (void *)c->d_cpy, (void *)c->d_gcpy,
                   (void *)c->d_e1, (void *)c->d_e2, (void *)c->d_iMn, (void *)c->d_met, (void *)c->d_met1, (void *)c->d_metn,
                   (void *)c->d_met1n, (void *)c->d_ms, (void *)c->d_ims32, (void *)c->d_m32, (void *)c->d_metp32,
-                  (void *)c->d_bwork, (void *)c->d_f4x, (void *)c->d_nptr, (void *)c->d_ncopy, (void *)c->d_kvis,
+                  (void *)c->d_f4x, (void *)c->d_nptr, (void *)c->d_ncopy, (void *)c->d_kvis,
                   (void *)c->d_M, (void *)c->d_dz, (void *)c->d_zP, (void *)c->d_xS, (void *)c->d_bar})
     if (p) (void)hipFree(p);
   prof_free(c);
@@ -1045,6 +1044,12 @@ extern "C" int cgd_jac(cgd_ctx *c, double *JRhoW, double *JWRho, double *JWRhoTh
   return CGD_OK;
 }
 
+// f(std::integral_constant<int, W>) for the workgroup of a tall column
+template <typename F> static void launch_tall(int Nz, F f) {
+  if (Nz <= 128) f(std::integral_constant<int, 128>{});
+  else f(std::integral_constant<int, 256>{});
+}
+
 extern "C" int cgd_schur(cgd_ctx *c, double *k, double *v, const double *JRhoW, const double *JWRho,
                          const double *JWRhoTh, const double *JRhoThW, double *tri, double fac, int comp_tri,
                          void *stream) {
@@ -1059,8 +1064,11 @@ extern "C" int cgd_schur(cgd_ctx *c, double *k, double *v, const double *JRhoW, 
     hipLaunchKernelGGL(k_schur_col, dim3((c->NumG + 3) / 4), dim3(256), 0, st, c->ka, k, v, JRhoW, JWRho, JWRhoTh,
                        JRhoThW, tri, fac, invfac2, comp_tri, c->thomas);
   else
-    hipLaunchKernelGGL(k_schur, dim3(grid_for(c->NumG, 64)), dim3(64), 0, st, c->ka, k, v, JRhoW, JWRho, JWRhoTh,
-                       JRhoThW, tri, c->d_bwork, fac, comp_tri);
+    launch_tall(c->Nz, [&](auto w) {
+      constexpr int W = decltype(w)::value;
+      hipLaunchKernelGGL(k_schur_tall<W>, dim3(c->NumG), dim3(W), 0, st, c->ka, k, v, JRhoW, JWRho, JWRhoTh, JRhoThW,
+                         tri, fac, invfac2, comp_tri);
+    });
   HIPCHK(c, hipGetLastError());
   if (c->ntr > 0) {
     const size_t ng = (size_t)c->NumG * c->Nz, nt = (size_t)c->ntr * ng;
@@ -1150,7 +1158,7 @@ static int launch_persist(cgd_ctx *c, int is, const RWStage<R> &rw, const double
   return CGD_OK;
 }
 
-// Fused step for Nz <= 64: the first pressure, then per stage the two
+// Fused step: the first pressure, then per stage the two
 // tendency passes and one column kernel (Jacobian, tri, stage terms, Schur
 // solve, next state and its pressure; the first also stores Vn = V).  With
 // R = float (mixed precision) the FP32 tendency and its FP32 state shadow
@@ -1216,7 +1224,16 @@ static int rw_step_fused(cgd_ctx *c, double *V, double dt, const cgd_rw_work *w,
       continue;
     }
     prof_begin(c, st, 2);
-    if (c->colw == 32) launch_stage<R, 32>(c, is, rw, st);
+    if (c->Nz > 64) {
+      if constexpr (std::is_same<R, double>::value)
+        launch_tall(c->Nz, [&](auto w) {
+          constexpr int W = decltype(w)::value;
+          const dim3 g(c->NumG), b(W);
+          if (is == 0) hipLaunchKernelGGL((k_rw_stage_tall<0, W>), g, b, 0, st, c->ka, rw);
+          else if (is == 1) hipLaunchKernelGGL((k_rw_stage_tall<1, W>), g, b, 0, st, c->ka, rw);
+          else hipLaunchKernelGGL((k_rw_stage_tall<2, W>), g, b, 0, st, c->ka, rw);
+        });
+    } else if (c->colw == 32) launch_stage<R, 32>(c, is, rw, st);
     else launch_stage<R, 64>(c, is, rw, st);
     HIPCHK(c, hipGetLastError());
     if (c->ntr > 0) {  // the tracers' stage terms and next state, FP64 in both modes
@@ -1248,7 +1265,7 @@ static int rw_step_fused(cgd_ctx *c, double *V, double dt, const cgd_rw_work *w,
 
 // One SSP-Knoth step as the reference's sequence of calls (FP64): prepare,
 // tendency, the Jacobian at the first stage, the stage terms by k_axpy and
-// the Schur solves.  Used for tall columns and by the adjoint's forward runs.
+// the Schur solves.  Used by the adjoint's forward runs.
 static int rw_composed_step(cgd_ctx *c, double *V, double dt, const cgd_rw_work *w, hipStream_t st) {
   int r;
   const double A[3][3] = {{0, 0, 0}, {1.0, 0, 0}, {0.25, 0.25, 0}};
@@ -1301,18 +1318,13 @@ static int rw_run(cgd_ctx *c, double *V, double dt, const cgd_rw_work *w, int ns
   const double gamma = 1.0;
   const size_t ng = (size_t)c->NumG * c->Nz, n5 = (size_t)(5 + c->ntr) * ng;  // (Nz, NumG, 5 + NumTr)
   double *k[3] = {w->k, w->k + n5, w->k + 2 * n5};
-  if (c->Nz <= 64) {
-    for (int s = 0; s < nsteps; ++s) {
-      const bool begin = s == 0, more = s + 1 < nsteps;
-      r = c->mixed ? rw_step_fused<float>(c, V, dt, w, st, k, A, Cc, Mw, gamma, begin, more)
-                   : rw_step_fused<double>(c, V, dt, w, st, k, A, Cc, Mw, gamma, begin, more);
-      if (r) return r;
-    }
-    return CGD_OK;
+  // tall columns step in FP64 in either precision mode
+  for (int s = 0; s < nsteps; ++s) {
+    const bool begin = s == 0, more = s + 1 < nsteps;
+    r = c->mixed && c->Nz <= 64 ? rw_step_fused<float>(c, V, dt, w, st, k, A, Cc, Mw, gamma, begin, more)
+                                : rw_step_fused<double>(c, V, dt, w, st, k, A, Cc, Mw, gamma, begin, more);
+    if (r) return r;
   }
-  // tall columns: the reference's sequence of calls, stage terms by k_axpy
-  for (int s = 0; s < nsteps; ++s)
-    if ((r = rw_composed_step(c, V, dt, w, st))) return r;
   return CGD_OK;
 }
 

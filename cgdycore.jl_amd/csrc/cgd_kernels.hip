@@ -1917,6 +1917,273 @@ __global__ void __launch_bounds__(256) k_rw_stage(KArgs a, RWStage<R> rw) {
 }
 
 // ------------------------------------------------------------------------
+// Columns taller than a wavefront (64 < Nz <= 256): one workgroup of W = 128
+// or 256 threads per column, thread = level.  Values of other levels are
+// exchanged through LDS: put() stores four per thread and meets one barrier
+// (two buffers in turn, so a buffer is rewritten only after every thread has
+// passed the next barrier); the tridiagonal system is solved by cyclic
+// reduction as in col_solve.  The loads and stores are whole columns; the
+// one-thread-per-column Thomas solve that this replaces took 1132 us for
+// 38402 columns of 70 levels, 48 % of a step over terrain at ne = 20.
+template <int W> struct TallX {
+  double *q;  // LDS: 2 * 4 * W
+  int i, ph;
+  __device__ __forceinline__ void put(double a, double b, double c, double d) {
+    ph ^= 1;
+    double *p = q + ph * 4 * W + i;
+    p[0] = a;
+    p[W] = b;
+    p[2 * W] = c;
+    p[3 * W] = d;
+    __syncthreads();
+  }
+  __device__ __forceinline__ void put(double a) {
+    ph ^= 1;
+    q[ph * 4 * W + i] = a;
+    __syncthreads();
+  }
+  // value `f` of the last put at level i + o, or `def` outside the workgroup
+  __device__ __forceinline__ double get(int f, int o, double def) const {
+    const int j = i + o;
+    return j >= 0 && j < W ? q[ph * 4 * W + f * W + j] : def;
+  }
+};
+
+// (s, lo) - a b, with the rounding errors of the product and of the
+// difference (Knuth's two-sum) gathered in lo
+__device__ __forceinline__ void sub_product(double &s, double &lo, double a, double b) {
+  const double p = a * b, t = s - p, z = t - s;
+  lo += ((s - (t - z)) - (p + z)) - fma(a, b, -p);
+  s = t;
+}
+
+// Solution of the tridiagonal system, one row per thread: cyclic reduction as
+// in col_solve, then one step of refinement with the same multipliers (they
+// stay in registers, so a sweep exchanges one value) from a residual with its
+// rounding errors.  The reduction's rounding grows with the height, as the
+// layers get thin against fac: against an extended-precision solve it is ten
+// times that of the elimination in order, refined it is smaller than that.
+template <int W>
+__device__ __forceinline__ double tall_solve(TallX<W> &X, double t0, double t1, double t2, double rhs, int n) {
+  constexpr int S = W == 128 ? 7 : 8;
+  static_assert(W == 1 << S, "one level per thread");
+  const int i = X.i;
+  const bool row = i < n;
+  X.put(t0, t2, 0.0, 0.0);
+  const double a0 = i > 0 && row ? X.get(1, -1, 0.0) : 0.0, c0 = i < n - 1 ? X.get(0, 1, 0.0) : 0.0;
+  double ra = a0, rb = row ? t1 : 1.0, rc = c0, rd = row ? rhs : 0.0;
+  double k1[S], k2[S];
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    const int st = 1 << s;
+    k1[s] = k2[s] = 0.0;
+    if (st < n) {
+      X.put(ra, rb, rc, rd);
+      const double am = X.get(0, -st, 0.0), bm = X.get(1, -st, 1.0), cm = X.get(2, -st, 0.0), dm = X.get(3, -st, 0.0);
+      const double ap = X.get(0, st, 0.0), bp = X.get(1, st, 1.0), cp = X.get(2, st, 0.0), dp = X.get(3, st, 0.0);
+      k1[s] = ra * rcp(bm);
+      k2[s] = rc * rcp(bp);
+      rb = rb - cm * k1[s] - ap * k2[s];
+      rd = rd - dm * k1[s] - dp * k2[s];
+      ra = -am * k1[s];
+      rc = -cp * k2[s];
+    }
+  }
+  const double ib = rcp(rb), x = row ? rd * ib : 0.0;
+  X.put(x);
+  double r = 0.0;
+  if (row) {
+    double lo = 0.0;
+    r = rhs;
+    sub_product(r, lo, t1, x);
+    sub_product(r, lo, a0, X.get(0, -1, 0.0));
+    sub_product(r, lo, c0, X.get(0, 1, 0.0));
+    r += lo;
+  }
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    const int st = 1 << s;
+    if (st < n) {
+      X.put(r);
+      r = r - X.get(0, -st, 0.0) * k1[s] - X.get(0, st, 0.0) * k2[s];
+    }
+  }
+  return row ? x + r * ib : 0.0;
+}
+
+// The tri matrix of row i from the J blocks of rows i-1, i, i+1 (as col_tri)
+template <int W>
+__device__ __forceinline__ void tall_tri(TallX<W> &X, const JacBlocks &J, double invfac2, int n, double &t0,
+                                         double &t1, double &t2) {
+  const int i = X.i;
+  X.put(J.wr0, J.wt0, J.wr1, J.wt1);
+  const double wr0m = X.get(0, -1, 0.0), wt0m = X.get(1, -1, 0.0), wr1p = X.get(2, 1, 0.0), wt1p = X.get(3, 1, 0.0);
+  t0 = 0.0;
+  t1 = 1.0;
+  t2 = 0.0;
+  if (i < n) {
+    t1 = invfac2 - J.wr1 * J.rw0 - J.wr0 * J.rw1 - J.wt1 * J.tw0 - J.wt0 * J.tw1;
+    t0 = i == 0 ? 0.0 : -wr0m * J.rw0 - wt0m * J.tw0;
+    t2 = i == n - 1 ? 0.0 : -wr1p * J.rw1 - wt1p * J.tw1;
+  }
+}
+
+// SchurSolveGPU! (as k_schur_col)
+template <int W>
+__global__ void __launch_bounds__(W)
+    k_schur_tall(KArgs a, double *__restrict__ k, double *__restrict__ v, const double *__restrict__ JRhoW,
+                 const double *__restrict__ JWRho, const double *__restrict__ JWRhoTh,
+                 const double *__restrict__ JRhoThW, double *__restrict__ tri, double fac, double invfac2,
+                 int comp_tri) {
+  __shared__ double lds[8 * W];
+  TallX<W> X{lds, (int)threadIdx.x, 0};
+  const int Nz = a.Nz, n = Nz - 1, i = X.i;
+  const size_t ig = blockIdx.x;
+  const size_t vs = (size_t)a.NumG * Nz, c0 = ig * Nz + i;
+  const bool row = i < n, lev = i < Nz;
+  const size_t jb = (ig * (size_t)n + i) * 2, tb = (ig * (size_t)n + i) * 3;
+  JacBlocks J{0, 0, 0, 0, 0, 0, 0, 0};
+  if (row)
+    J = JacBlocks{JRhoW[jb],   JRhoW[jb + 1],   JWRho[jb],   JWRho[jb + 1],
+                  JWRhoTh[jb], JWRhoTh[jb + 1], JRhoThW[jb], JRhoThW[jb + 1]};
+  double v1 = 0, v2 = 0, v3 = 0, v4 = 0, v5 = 0;
+  if (lev) {
+    v1 = v[c0];
+    v2 = v[c0 + vs];
+    v3 = v[c0 + 2 * vs];
+    v4 = v[c0 + 3 * vs];
+    v5 = v[c0 + 4 * vs];
+  }
+  double t0 = 0, t1 = 1, t2 = 0;
+  if (comp_tri) {
+    tall_tri(X, J, invfac2, n, t0, t1, t2);
+    if (row) {
+      tri[tb] = t0;
+      tri[tb + 1] = t1;
+      tri[tb + 2] = t2;
+    }
+  } else if (row) {
+    t0 = tri[tb];
+    t1 = tri[tb + 1];
+    t2 = tri[tb + 2];
+  }
+  X.put(v1, v5, 0.0, 0.0);
+  const double v1p = X.get(0, 1, 0.0), v5p = X.get(1, 1, 0.0);
+  if (row) {
+    v4 = v4 / fac + J.wr1 * v1 + J.wr0 * v1p + J.wt1 * v5 + J.wt0 * v5p;
+    v[c0 + 3 * vs] = v4;
+  }
+  const double k4 = tall_solve(X, t0, t1, t2, v4, n);
+  X.put(k4, J.rw1, J.tw1, 0.0);
+  const double k4m = X.get(0, -1, 0.0), rw1m = X.get(1, -1, 0.0), tw1m = X.get(2, -1, 0.0);
+  if (lev) {
+    if (row) {
+      v1 += J.rw0 * k4;
+      v5 += J.tw0 * k4;
+    }
+    if (i > 0) {
+      v1 += rw1m * k4m;
+      v5 += tw1m * k4m;
+    }
+    k[c0] = fac * v1;
+    k[c0 + vs] = fac * v2;
+    k[c0 + 2 * vs] = fac * v3;
+    k[c0 + 3 * vs] = k4;
+    k[c0 + 4 * vs] = fac * v5;
+    v[c0] = v1;
+    v[c0 + 4 * vs] = v5;
+  }
+}
+
+// The Rosenbrock stage (as k_rw_stage), FP64
+template <int STAGE, int W>
+__global__ void __launch_bounds__(W) k_rw_stage_tall(KArgs a, RWStage<double> rw) {
+  __shared__ double lds[8 * W];
+  TallX<W> X{lds, (int)threadIdx.x, 0};
+  const int Nz = a.Nz, n = Nz - 1, i = X.i;
+  const size_t ig = blockIdx.x;
+  const size_t vs = (size_t)a.NumG * Nz, c0 = ig * Nz + i;
+  const bool row = i < n, lev = i < Nz;
+  const double fac = rw.fac;
+  double vn[5] = {0, 0, 0, 0, 0}, v[5] = {0, 0, 0, 0, 0}, kp[2][5] = {{0, 0, 0, 0, 0}, {0, 0, 0, 0, 0}};
+  double dzi = 1.0;
+  if (lev) {
+    const double *src = STAGE == 0 ? rw.V : rw.Vn;
+#pragma unroll
+    for (int q = 0; q < 5; ++q) vn[q] = __builtin_nontemporal_load(&src[c0 + q * vs]);
+    if constexpr (STAGE == 0) {
+#pragma unroll
+      for (int q = 0; q < 5; ++q) __builtin_nontemporal_store(vn[q], &rw.Vnw[c0 + q * vs]);
+    }
+    dzi = rw.dz[c0];
+    if (rw.fV) {
+#pragma unroll
+      for (int q = 0; q < 5; ++q) v[q] = __builtin_nontemporal_load(&rw.fV[c0 + q * vs]);
+    } else {
+      const bool edge = rw.nchunk > 1 && (i + 1) % rw.nzt == 0 && i + 1 < Nz;
+      const int ch = (i + 1) / rw.nzt;
+      const Const<int> cp = as_const(a.gcpy + ig * a.cpw);
+      double s4 = 0;
+      for (int q = 0; q < a.cpw; ++q) {
+        const int c = cp[q];
+        if (c < 0) break;
+        const double *Ec = rw.Fe + (size_t)c * Nz + i;
+#pragma unroll
+        for (int f = 0; f < 5; ++f) v[f] += __builtin_nontemporal_load(Ec + f * a.ecs);
+        if (edge) s4 += rw.F4x[(size_t)c * rw.nchunk + ch];
+      }
+      if (edge) v[3] += s4;
+    }
+#pragma unroll
+    for (int j = 0; j < STAGE; ++j) {
+#pragma unroll
+      for (int q = 0; q < 5; ++q) {
+        kp[j][q] = __builtin_nontemporal_load(&rw.kprev[j][c0 + q * vs]);
+        v[q] = v[q] + rw.cf[j] * kp[j][q];
+      }
+    }
+  }
+  const double dpd = lev ? eos_dpdrhoth(a, vn[4]) : 0.0;
+  X.put(vn[0], vn[4], dpd, dzi);
+  JacBlocks J{0, 0, 0, 0, 0, 0, 0, 0};
+  if (row) J = jac_blocks(a, vn[0], X.get(0, 1, 0.0), vn[4], X.get(1, 1, 0.0), dpd, X.get(2, 1, 0.0), dzi, X.get(3, 1, 1.0));
+  double t0, t1, t2;
+  tall_tri(X, J, rw.invfac2, n, t0, t1, t2);
+  X.put(v[0], v[4], 0.0, 0.0);
+  double rhs = 0.0;
+  if (row)
+    rhs = v[3] * rw.invfac + J.wr1 * v[0] + J.wr0 * X.get(0, 1, 0.0) + J.wt1 * v[4] + J.wt0 * X.get(1, 1, 0.0);
+  const double k4 = tall_solve(X, t0, t1, t2, rhs, n);
+  X.put(k4, J.rw1, J.tw1, 0.0);
+  if (!lev) return;
+  if (row) {
+    v[0] += J.rw0 * k4;
+    v[4] += J.tw0 * k4;
+  }
+  if (i > 0) {
+    const double k4m = X.get(0, -1, 0.0);
+    v[0] += X.get(1, -1, 0.0) * k4m;
+    v[4] += X.get(2, -1, 0.0) * k4m;
+  }
+  const double kc[5] = {fac * v[0], fac * v[1], fac * v[2], k4, fac * v[4]};
+  if (rw.k) {
+#pragma unroll
+    for (int q = 0; q < 5; ++q) __builtin_nontemporal_store(kc[q], &rw.k[c0 + q * vs]);
+  }
+  double rt = 0.0;
+#pragma unroll
+  for (int q = 0; q < 5; ++q) {
+    double r = vn[q];
+#pragma unroll
+    for (int j = 0; j < STAGE; ++j) r = r + rw.av[j] * kp[j][q];
+    r = r + rw.av[STAGE] * kc[q];
+    __builtin_nontemporal_store(r, &rw.V[c0 + q * vs]);
+    if (q == 4) rt = r;
+  }
+  if (rw.P) rw.P[c0] = eos_p(a, rt);
+}
+
+// ------------------------------------------------------------------------
 // One persistent launch per Rosenbrock-W stage: pass 1, pass 2, then the
 // column stage, in one grid whose
 // workgroups are all resident at once (the host sizes the grid from the
@@ -2119,74 +2386,6 @@ __global__ void k_rw_begin(KArgs a, const double *__restrict__ V, double *__rest
 __global__ void k_to_f32(const double *__restrict__ x, float *__restrict__ y, size_t n) {
   for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
     y[i] = float(x[i]);
-}
-
-// SchurSolveGPU! (src/Integration/SchurSolve.jl:45-177): tri build,
-// SchurSolveFKernel!, triSolve! (Thomas) and SchurSolveBKernel! for one
-// column per thread.  bwork holds the Thomas right-hand side copy.
-__global__ void k_schur(KArgs a, double *__restrict__ k, double *__restrict__ v, const double *__restrict__ JRhoW,
-                        const double *__restrict__ JWRho, const double *__restrict__ JWRhoTh,
-                        const double *__restrict__ JRhoThW, double *__restrict__ tri, double *__restrict__ bwork,
-                        double fac, int comp_tri) {
-  const int Nz = a.Nz, n = Nz - 1;
-  const size_t ig = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (ig >= (size_t)a.NumG) return;
-  const size_t vs = (size_t)a.NumG * Nz;
-  const size_t c0 = ig * Nz;
-  const size_t jb = ig * (size_t)n * 2, tb = ig * (size_t)n * 3;
-#define JBk(A, c, i) A[jb + 2 * (size_t)(i) + (c)]
-#define TRk(c, i) tri[tb + 3 * (size_t)(i) + (c)]
-  if (comp_tri) {
-    const double invfac = 1.0 / fac, invfac2 = invfac / fac;
-    for (int i = 0; i < n; ++i) {
-      TRk(1, i) = invfac2 - JBk(JWRho, 1, i) * JBk(JRhoW, 0, i) - JBk(JWRho, 0, i) * JBk(JRhoW, 1, i) -
-                  JBk(JWRhoTh, 1, i) * JBk(JRhoThW, 0, i) - JBk(JWRhoTh, 0, i) * JBk(JRhoThW, 1, i);
-      TRk(0, i) = (i == 0) ? 0.0
-                           : -JBk(JWRho, 0, i - 1) * JBk(JRhoW, 0, i) - JBk(JWRhoTh, 0, i - 1) * JBk(JRhoThW, 0, i);
-      TRk(2, i) = (i == n - 1) ? 0.0
-                               : -JBk(JWRho, 1, i + 1) * JBk(JRhoW, 1, i) -
-                                     JBk(JWRhoTh, 1, i + 1) * JBk(JRhoThW, 1, i);
-    }
-  }
-  double *v1 = v + c0, *v4 = v + c0 + 3 * vs, *v5 = v + c0 + 4 * vs;
-  double *k4 = k + c0 + 3 * vs;
-  double *b = bwork + ig * (size_t)n;
-  for (int iz = 0; iz < n; ++iz) {
-    v4[iz] = v4[iz] / fac + JBk(JWRho, 1, iz) * v1[iz] + JBk(JWRho, 0, iz) * v1[iz + 1] +
-             JBk(JWRhoTh, 1, iz) * v5[iz] + JBk(JWRhoTh, 0, iz) * v5[iz + 1];
-    b[iz] = v4[iz];
-  }
-  k4[n] = 0.0;
-  // triSolve!: x in k4
-  k4[0] = TRk(1, 0);
-  for (int i = 0; i < n - 1; ++i) {
-    const double q = TRk(2, i) / k4[i];
-    k4[i + 1] = TRk(1, i + 1) - q * TRk(0, i + 1);
-    b[i + 1] = b[i + 1] - q * b[i];
-  }
-  k4[n - 1] = b[n - 1] / k4[n - 1];
-  for (int i = n - 2; i >= 0; --i) k4[i] = (b[i] - TRk(0, i + 1) * k4[i + 1]) / k4[i];
-  // SchurSolveBKernel!
-  double *k1 = k + c0, *k2 = k + c0 + vs, *k3 = k + c0 + 2 * vs, *k5 = k + c0 + 4 * vs;
-  const double *v2 = v + c0 + vs, *v3 = v + c0 + 2 * vs;
-  for (int iz = 0; iz < Nz; ++iz) {
-    if (iz == 0) {
-      v1[iz] += JBk(JRhoW, 0, iz) * k4[iz];
-      v5[iz] += JBk(JRhoThW, 0, iz) * k4[iz];
-    } else if (iz == Nz - 1) {
-      v1[iz] += JBk(JRhoW, 1, iz - 1) * k4[iz - 1];
-      v5[iz] += JBk(JRhoThW, 1, iz - 1) * k4[iz - 1];
-    } else {
-      v1[iz] += JBk(JRhoW, 0, iz) * k4[iz] + JBk(JRhoW, 1, iz - 1) * k4[iz - 1];
-      v5[iz] += JBk(JRhoThW, 0, iz) * k4[iz] + JBk(JRhoThW, 1, iz - 1) * k4[iz - 1];
-    }
-    k1[iz] = fac * v1[iz];
-    k2[iz] = fac * v2[iz];
-    k3[iz] = fac * v3[iz];
-    k5[iz] = fac * v5[iz];
-  }
-#undef JBk
-#undef TRk
 }
 
 // y = x0 + a1*x1 (+ a2*x2), evaluated as ((x0 + a1 x1) + a2 x2) like the

@@ -146,3 +146,40 @@ def test_hooks_with_the_copies(pkg, oracle_mod, torch_cuda, p, nz, ntr):
     orc.rw_step(Vo, 100.0, 2)
     for v in range(5 + ntr):
         assert rel_l2(V[v].cpu().numpy(), Vo[v]) <= TOL, f"V{v + 1} {rel_l2(V[v].cpu().numpy(), Vo[v]):.3e}"
+
+
+@pytest.mark.parametrize("nz,precision", [(65, "fp64"), (128, "fp64"), (129, "fp64"), (256, "fp64"), (65, "mixed")])
+def test_tall_columns(pkg, oracle_mod, torch_cuda, nz, precision):
+    """Columns taller than a wavefront: the Schur solve (with and without a
+    new tri) and the steps, which are FP64 in the mixed mode too."""
+    torch, host = torch_cuda, pkg.host
+    print(f"tall columns nz={nz} {precision}", flush=True)
+    disc, phys, dev, orc = setup(pkg, oracle_mod, 2, 3, nz, precision=precision)
+    FE, Metric, Global, Cache, JCache = dev
+    U0 = pkg.state.jet_state(disc, seed=8)
+    U = torch.as_tensor(U0, device="cuda")
+    eq = host.CompressibleShallow()
+    host.FcnPrepareGPU(U, FE, Metric, phys, Cache, None, Global, None, eq)
+    host.JacSchurGPU(JCache, U, FE, Metric, phys, Cache, Global, None, eq)
+    blocks = orc.jac(U0.copy(), orc.prepare(U0.copy()))
+    JCache.CompTri = True
+    for solve in range(2):  # the second reuses tri
+        v0 = np.random.default_rng(solve).standard_normal(U0.shape)
+        v = torch.as_tensor(v0, device="cuda")
+        k = torch.zeros_like(v)
+        host.SchurSolveGPU(k, v, JCache, 150.0, Cache, Global)
+        torch.cuda.synchronize()
+        vo = v0.copy()
+        ko, trio = orc.schur(vo, blocks, 150.0)
+        assert rel_l2(JCache.tri.cpu().numpy(), trio) <= TOL
+        for c in range(5):
+            assert rel_l2(k[c].cpu().numpy(), ko[c]) <= TOL, f"k[{c}] {rel_l2(k[c].cpu().numpy(), ko[c]):.3e}"
+            assert rel_l2(v[c].cpu().numpy(), vo[c]) <= TOL, f"v[{c}]"
+    V = U.clone()
+    host.TimeStepper(V, 100.0, 2, FE, Metric, phys, Cache, JCache, Global)
+    torch.cuda.synchronize()
+    Vo = U0.copy()
+    orc.rw_step(Vo, 100.0, 2)
+    for c in range(5):
+        e = rel_l2(V[c].cpu().numpy(), Vo[c])
+        assert e <= TOL, f"V{c + 1} {e:.3e}"
