@@ -97,8 +97,10 @@ template <typename R> static size_t lds_fcn1(const cgd_ctx *c) {
   return (r + 7) / 8 * 8 + sizeof(double) * (2 * c->NN + 3 * c->NN * c->nzt1);
 }
 template <typename R> static size_t lds_fcn2(const cgd_ctx *c) {
-  // + a 12-entry per-node table of the horizontal metric (compact layout)
-  const size_t r = sizeof(R) * (2 * c->NN + 14 * c->NN * c->nzt + 12 * c->NN);
+  // + the horizontal metric: 12 values per node (compact layout), 10 per point
+  // (full layout, FP64)
+  const size_t hm = c->cm || !std::is_same<R, double>::value ? 12 * c->NN : 10 * c->NN * c->nzt;
+  const size_t r = sizeof(R) * (2 * c->NN + 14 * c->NN * c->nzt + hm);
   const size_t base = sizeof(double) * (c->NN + c->NN * c->nzt);
   if (std::is_same<R, double>::value) return base + r;
   return base + (r + 7) / 8 * 8 + sizeof(double) * (c->NN + 3 * c->NN * c->nzt);
