@@ -687,6 +687,7 @@ static int ctx_build(cgd_ctx *c, const cgd_desc *ds, int nmem, hipStream_t st) {
   a.kappa = d->kappa;
   a.Rd_p0 = d->Rd / d->p0;
   a.eos_y = 1.0 / (1.0 - d->kappa);
+  a.Rd_Cpd = d->Rd / d->Cpd;
   a.dpd_y = d->kappa / (1.0 - d->kappa);
   // DS, DW arrive column-major (Julia): DS[i,k] at i + N*k
   for (int i = 0; i < c->N; ++i)
@@ -929,7 +930,8 @@ extern "C" int cgd_prepare(cgd_ctx *c, const double *U, double *AuxG, void *stre
   if (r) return r;
   if (!U || !AuxG) return fail(c, CGD_ERR_ARG, "cgd_prepare: null array");
   const size_t n = (size_t)c->NumG * c->Nz;
-  hipLaunchKernelGGL(k_prepare, dim3(grid_for(n, 256)), dim3(256), 0, S(stream), c->ka, U, AuxG, n);
+  const auto kernel = c->ka.iv >= 0 ? k_prepare<true> : k_prepare<false>;
+  hipLaunchKernelGGL(kernel, dim3(grid_for(n, 256)), dim3(256), 0, S(stream), c->ka, U, AuxG, n);
   HIPCHK(c, hipGetLastError());
   return CGD_OK;
 }

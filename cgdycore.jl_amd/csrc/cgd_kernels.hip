@@ -41,6 +41,7 @@ struct KArgs {
   int Nz, NumG, nzt;
   double Grav, Omega, Rd, Cpd, p0, kappa;
   double Rd_p0, eos_y, dpd_y;      // Rd/p0, 1/(1-kappa), kappa/(1-kappa)
+  double Rd_Cpd;                   // Rd/Cpd
   double D[CGD_NMAX * CGD_NMAX];   // D[i*N + k] = DS[i,k]
   double DWm[CGD_NMAX * CGD_NMAX]; // DW[i*N + k]
   float Df[CGD_NMAX * CGD_NMAX], DWf[CGD_NMAX * CGD_NMAX];  // both in FP32 (mixed precision)
@@ -1776,10 +1777,16 @@ __device__ __forceinline__ void moist_ptth(const KArgs &a, double rho, double rt
   th = pow(a.p0 / p, km) * T;
 }
 
+// theta = (p0/p)^(Rd/Cpd) T: with kappa = Rd/Cpd that is rho*theta / rho, the
+// rounded quotient instead of the errors of log, exp and pow after each other.
+// The pow was most of the arithmetic: 80 us for 86402 columns of 64 levels,
+// whose five arrays take 51 us at the rate of a copy; without it, and with the moist state a
+// kernel of its own, 56 us.
+template <bool MOIST>
 __global__ void k_prepare(KArgs a, const double *__restrict__ U, double *__restrict__ AuxG, size_t n) {
   for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
     const double rho = U[i], rth = U[i + 4 * n];
-    if (a.iv >= 0) {
+    if constexpr (MOIST) {
       double p, T, th;
       moist_ptth(a, rho, rth, U[i + (size_t)a.iv * n], U[i + (size_t)a.ic * n], p, T, th);
       AuxG[i] = p;
@@ -1791,7 +1798,8 @@ __global__ void k_prepare(KArgs a, const double *__restrict__ U, double *__restr
     const double T = p / (a.Rd * rho);
     AuxG[i] = p;
     AuxG[i + n] = T;
-    AuxG[i + 2 * n] = pow(a.p0 / p, a.Rd / a.Cpd) * T;
+    const bool exact = a.kappa == a.Rd_Cpd && p > 0.0 && p < __builtin_huge_val();
+    AuxG[i + 2 * n] = exact ? rth / rho : pow(a.p0 / p, a.Rd_Cpd) * T;
   }
 }
 

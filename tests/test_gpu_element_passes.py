@@ -183,3 +183,31 @@ def test_tall_columns(pkg, oracle_mod, torch_cuda, nz, precision):
     for c in range(5):
         e = rel_l2(V[c].cpu().numpy(), Vo[c])
         assert e <= TOL, f"V{c + 1} {e:.3e}"
+
+
+@pytest.mark.parametrize("scale", [1.0, 1.01])
+def test_prepare_theta(pkg, torch_cuda, scale):
+    """theta of the prepare kernel: the quotient where kappa = Rd/Cpd, the
+    power of the pressure elsewhere and where the pressure is not a positive
+    number.  A handful of roundings: 1e-14."""
+    torch, host = torch_cuda, pkg.host
+
+    class P(pkg.discretization.Phys):
+        @property
+        def kappa(self):
+            return scale * (self.Rd / self.Cpd)
+
+    phys = P()
+    disc = pkg.discretization.build(2, 3, 11, 30000.0)
+    print(f"prepare theta scale={scale}", flush=True)
+    FE, Metric, Global, Cache, JCache = host.device_setup(disc, phys, device="cuda")
+    U = torch.as_tensor(pkg.state.jet_state(disc, seed=2), device="cuda")
+    U[4, 0, :3] = torch.tensor([-1.0, 0.0, float("nan")], dtype=U.dtype, device="cuda")
+    host.FcnPrepareGPU(U, FE, Metric, phys, Cache, None, Global, None, host.CompressibleShallow())
+    torch.cuda.synchronize()
+    p, T, th = Cache.AuxG[0], Cache.AuxG[1], Cache.AuxG[2]
+    want = (phys.p0 / p) ** (phys.Rd / phys.Cpd) * p / (phys.Rd * U[0])
+    bad = torch.zeros_like(p, dtype=torch.bool)
+    bad[0, :3] = True
+    assert torch.equal(torch.isnan(th), torch.isnan(want)) and torch.isnan(th[bad]).all()
+    assert float(((th - want) / want)[~bad].abs().max()) <= 1e-14
