@@ -26,7 +26,7 @@ struct cgd_ctx {
   int *d_glob = nullptr;       // [NF][NN] 0-based
   int *d_clist = nullptr;      // elements by colour, ascending within one
   int *d_cpy = nullptr, *d_gcpy = nullptr;  // the copies of each element node / global node, colour order
-  double *d_e1 = nullptr, *d_e2 = nullptr;  // element copies of the pass-1 cache and of the tendency (5 each)
+  double *d_e1 = nullptr, *d_e2 = nullptr;  // element copies of the pass-1 cache and of the tendency (5 + NumTr each)
   double *d_met = nullptr, *d_met1 = nullptr, *d_ms = nullptr;
   double *d_metn = nullptr, *d_met1n = nullptr;  // compact metric layout: per element node
   int cm = 0;                                    // 1: compact metric layout
@@ -532,8 +532,8 @@ static int ctx_build(cgd_ctx *c, const cgd_desc *ds, int nmem, hipStream_t st) {
   HIPCHK(c, hipMalloc(&c->d_clist, (size_t)NF * sizeof(int)));
   HIPCHK(c, hipMalloc(&c->d_cpy, cpy.size() * sizeof(int)));
   HIPCHK(c, hipMalloc(&c->d_gcpy, gcpy.size() * sizeof(int)));
-  HIPCHK(c, hipMalloc(&c->d_e1, npt * 5 * sizeof(double)));
-  HIPCHK(c, hipMalloc(&c->d_e2, npt * 5 * sizeof(double)));
+  HIPCHK(c, hipMalloc(&c->d_e1, npt * (5 + c->ntr) * sizeof(double)));
+  HIPCHK(c, hipMalloc(&c->d_e2, npt * (5 + c->ntr) * sizeof(double)));
   HIPCHK(c, hipMalloc(&c->d_met, npt * CGD_NMET * sizeof(double)));
   HIPCHK(c, hipMalloc(&c->d_met1, npt * CGD_NMET1 * sizeof(double)));
   HIPCHK(c, hipMalloc(&c->d_ms, ng * sizeof(double)));
@@ -888,25 +888,25 @@ static void fcn2_t(cgd_ctx *c, dim3 g, hipStream_t st, const double *U, const R 
       else FN<4, 8, false, R>(c, __VA_ARGS__);                     \
     }                                                              \
   } while (0)
+// the tracers' element copies: components 5.. of d_e1 and d_e2, FP64 in both modes
 template <int N, int NZT, bool CM, typename R>
-static void tr1_t(cgd_ctx *c, int nitems, hipStream_t st, int slot0, const double *U, double *T1) {
+static void tr1_t(cgd_ctx *c, int nitems, hipStream_t st, const double *U) {
   const size_t lds = sizeof(double) * (2 * c->NN + 3 * c->NN * NZT);
-  hipLaunchKernelGGL((k_tr1<N, NZT, CM>), dim3(nitems), dim3(c->block1), lds, st, c->ka, slot0, c->nchunk1, c->ntr,
-                     U, T1);
+  hipLaunchKernelGGL((k_tr1<N, NZT, CM>), dim3(nitems), dim3(c->block1), lds, st, c->ka, c->nchunk1, c->ntr, U,
+                     c->d_e1 + 5 * c->ka.ecs);
 }
 template <int N, int NZT, bool CM, typename R>
-static void tr2_t(cgd_ctx *c, int nitems, hipStream_t st, int slot0, const double *U, const double *T1,
-                  double *F) {
+static void tr2_t(cgd_ctx *c, int nitems, hipStream_t st, const double *U, double *Cout) {
   const size_t lds = sizeof(double) * (2 * c->NN + 10 * c->NN * NZT);
-  hipLaunchKernelGGL((k_tr2<N, NZT, CM>), dim3(nitems), dim3(c->block), lds, st, c->ka, slot0, c->nchunk, c->ntr, U,
-                     T1, F);
+  hipLaunchKernelGGL((k_tr2<N, NZT, CM>), dim3(nitems), dim3(c->block), lds, st, c->ka, c->nchunk, c->ntr, U,
+                     c->d_e1 + 5 * c->ka.ecs, Cout, c->d_e2 + 5 * c->ka.ecs);
 }
 
 template <int N, int NZT, bool CM, typename R>
-static void tr2lim_t(cgd_ctx *c, int nitems, hipStream_t st, int slot0, const double *U, double *F) {
+static void tr2lim_t(cgd_ctx *c, int nitems, hipStream_t st, const double *U) {
   const size_t lds = sizeof(double) * (c->NN + 7 * c->NN * NZT);
-  hipLaunchKernelGGL((k_tr2_lim<N, NZT, CM>), dim3(nitems), dim3(c->block), lds, st, c->ka, slot0, c->nchunk, c->ntr,
-                     U, c->d_stencil, c->NF, c->d_qmin, c->d_qmax, c->dtau, F);
+  hipLaunchKernelGGL((k_tr2_lim<N, NZT, CM>), dim3(nitems), dim3(c->block), lds, st, c->ka, c->nchunk, c->ntr, U,
+                     c->d_stencil, c->NF, c->d_qmin, c->d_qmax, c->dtau, c->d_e2 + 5 * c->ka.ecs);
 }
 
 template <typename R>
@@ -965,14 +965,11 @@ static int run_fcn(cgd_ctx *c, R *F, const double *U, const R *UR, R *Temp1, con
   // occupies only the first five components' worth of those buffers)
   double *const Fd = reinterpret_cast<double *>(F);
   double *const T1d = reinterpret_cast<double *>(Temp1);
-  if (c->ntr > 0 && !c->horlimit)  // HorLimit: no tracer hyperviscosity (FcnGPU.jl:747-751)
-    for (int k = 0; k < c->ncolor; ++k) {
-      const int ne = c->color_off[k + 1] - c->color_off[k];
-      if (!ne) continue;
-      CGD_DISPATCH(tr1_t, double, c->nzt1, ne * c->nchunk1, st, c->color_off[k], U, T1d);
-      HIPCHK(c, hipGetLastError());
-      ++launches;
-    }
+  if (c->ntr > 0 && !c->horlimit) {  // HorLimit: no tracer hyperviscosity (FcnGPU.jl:747-751)
+    CGD_DISPATCH(tr1_t, double, c->nzt1, c->NF * c->nchunk1, st, U);
+    HIPCHK(c, hipGetLastError());
+    ++launches;
+  }
   if ((r = prof_end(c, st, 0, launches))) return r;
   prof_begin(c, st, 1);
   launches = 0;
@@ -981,28 +978,27 @@ static int run_fcn(cgd_ctx *c, R *F, const double *U, const R *UR, R *Temp1, con
   ++launches;
   {
     if (c->ntr > 0 && c->horlimit) {
-      // LimitKernel! on the state, then DivRhoTrUpwind3LimKernel! per colour
+      // LimitKernel! on the state, then DivRhoTrUpwind3LimKernel!
       if (!(c->dtau > 0.0)) return fail(c, CGD_ERR_ARG, "HorLimit: the stage time step is not set (cgd_set_dtau)");
       const size_t nb = (size_t)c->ntr * c->NF * c->Nz;
       hipLaunchKernelGGL(k_lim_bounds, dim3(grid_for(nb, 256)), dim3(256), 0, st, c->ka, c->NF, c->NN, c->ntr, U,
                          c->d_qmin, c->d_qmax);
       HIPCHK(c, hipGetLastError());
       ++launches;
-      for (int k = 0; k < c->ncolor; ++k) {
-        const int ne = c->color_off[k + 1] - c->color_off[k];
-        if (!ne) continue;
-        CGD_DISPATCH(tr2lim_t, double, c->nzt, ne * c->nchunk, st, c->color_off[k], U, Fd);
-        HIPCHK(c, hipGetLastError());
-        ++launches;
-      }
+      CGD_DISPATCH(tr2lim_t, double, c->nzt, c->NF * c->nchunk, st, U);
+      HIPCHK(c, hipGetLastError());
+      ++launches;
     } else if (c->ntr > 0) {
-      for (int k = 0; k < c->ncolor; ++k) {
-        const int ne = c->color_off[k + 1] - c->color_off[k];
-        if (!ne) continue;
-        CGD_DISPATCH(tr2_t, double, c->nzt, ne * c->nchunk, st, c->color_off[k], U, T1d, Fd);
-        HIPCHK(c, hipGetLastError());
-        ++launches;
-      }
+      CGD_DISPATCH(tr2_t, double, c->nzt, c->NF * c->nchunk, st, U, want_f ? T1d : nullptr);
+      HIPCHK(c, hipGetLastError());
+      ++launches;
+    }
+    if (c->ntr > 0 && (want_f || c->hooks.micro)) {
+      const size_t ng = (size_t)c->NumG * c->Nz;
+      hipLaunchKernelGGL(k_tr_dss, dim3(grid_for(ng, 256), c->ntr), dim3(256), 0, st, c->ka, c->d_e2 + 5 * c->ka.ecs,
+                         Fd + 5 * ng, (unsigned)ng);
+      HIPCHK(c, hipGetLastError());
+      ++launches;
     }
   }
   if (want_f || has_hooks(c)) {
@@ -1241,20 +1237,13 @@ static int rw_step_fused(cgd_ctx *c, double *V, double dt, const cgd_rw_work *w,
     else launch_stage<R, 64>(c, is, rw, st);
     HIPCHK(c, hipGetLastError());
     if (c->ntr > 0) {  // the tracers' stage terms and next state, FP64 in both modes
-      const size_t nt = (size_t)c->ntr * ng, o = 5 * ng;
-      const double *fvt = w->fV + o, *k0 = k[0] + o, *k1 = k[1] + o;
+      const size_t o = 5 * ng;
+      const double *fvt = c->hooks.micro ? w->fV + o : nullptr, *k0 = k[0] + o, *k1 = k[1] + o;
       double *kout = is < 2 ? k[is] + o : nullptr;
       const double cf0 = is > 0 ? Cc[is][0] / dt : 0.0, cf1 = is > 1 ? Cc[is][1] / dt : 0.0;
-      const dim3 gt(grid_for(nt, 256)), bt(256);
-      if (is == 0)
-        hipLaunchKernelGGL(k_rw_tr<0>, gt, bt, 0, st, fvt, k0, k1, cf0, cf1, rw.av[0], rw.av[1], rw.av[2], rw.fac,
-                           V + o, w->Vn + o, kout, nt);
-      else if (is == 1)
-        hipLaunchKernelGGL(k_rw_tr<1>, gt, bt, 0, st, fvt, k0, k1, cf0, cf1, rw.av[0], rw.av[1], rw.av[2], rw.fac,
-                           V + o, w->Vn + o, kout, nt);
-      else
-        hipLaunchKernelGGL(k_rw_tr<2>, gt, bt, 0, st, fvt, k0, k1, cf0, cf1, rw.av[0], rw.av[1], rw.av[2], rw.fac,
-                           V + o, w->Vn + o, kout, nt);
+      const auto kernel = is == 0 ? k_rw_tr<0> : is == 1 ? k_rw_tr<1> : k_rw_tr<2>;
+      hipLaunchKernelGGL(kernel, dim3(grid_for(ng, 256), c->ntr), dim3(256), 0, st, c->ka, c->d_e2 + 5 * c->ka.ecs, fvt,
+                         k0, k1, cf0, cf1, rw.av[0], rw.av[1], rw.av[2], rw.fac, V + o, w->Vn + o, kout, (unsigned)ng);
       HIPCHK(c, hipGetLastError());
     }
     // Models.Moist: the pressure of the new state needs its tracers too

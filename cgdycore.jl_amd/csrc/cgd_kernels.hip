@@ -208,7 +208,7 @@ __device__ __forceinline__ void recu4_smooth(double cLL, double cL, double cR, d
 
 // RecU4 split in two: the weights of both sides depend on the layer volumes
 // only (computed once, e.g. for several tracers), the limited
-// reconstruction on c; the same operations as recu4, so the same bits
+// reconstruction on c
 template <typename R> struct RecW {
   R kRl, kLl, kLr, kRr;  // left-biased kR, kL; right-biased kL, kR
 };
@@ -229,17 +229,20 @@ template <typename R> __device__ __forceinline__ RecW<R> recu4_weights(R JLL, R 
   }
   return w;
 }
+// ... of equal volumes
+template <typename R> __device__ __forceinline__ RecW<R> recu4_equal() {
+  return RecW<R>{R(1) / R(3), R(1) / R(6), R(1) / R(3), R(1) / R(6)};
+}
+// The upwind flux through an interface with the contravariant mass flux wc
+// between cL (below) and cR (above): ((|w| + w)/4 cFL + (w - |w|)/4 cFR is
+// w/2 times the upwind side's limited value, so only that side is formed.
 template <typename R>
-__device__ __forceinline__ void recu4_apply(R cLL, R cL, R cR, R cRR, const RecW<R> &w, R &cFL, R &cFR) {
-  const R tiny = R(1.e-20), zero = R(0), one = R(1);
-  {
-    const R r = (cL - cLL) * rcp(cR - cL + tiny);
-    cFL = cL + jmax(zero, jmin(r, jmin(w.kLl * r + w.kRl, one))) * (cR - cL);
-  }
-  {
-    const R r = (cR - cRR) * rcp(cL - cR + tiny);
-    cFR = cR + jmax(zero, jmin(r, jmin(w.kRr * r + w.kLr, one))) * (cL - cR);
-  }
+__device__ __forceinline__ R recu4_flux(R cLL, R cL, R cR, R cRR, const RecW<R> &w, R wc) {
+  const bool up = wc >= R(0);
+  const R c = up ? cL : cR, d = (up ? cR : cL) - c, s = c - (up ? cLL : cRR);
+  const R r = s * rcp(d + R(1.e-20));
+  const R lim = jmin((up ? w.kLl : w.kRr) * r + (up ? w.kRl : w.kLr), R(1));
+  return R(0.5) * wc * (c + jmax(R(0), jmin(r, lim)) * d);
 }
 
 // ------------------------------------------------------------------------
@@ -879,9 +882,15 @@ __device__ __forceinline__ void hooks_point(const KArgs &a, const Hooks &hk, con
 // (ViscKernel.jl:169-218) in pass 1, HyperViscTracerKoeffKernel!
 // (:277-327) and the tracer loop of DivRhoTrUpwind3New2Kernel!
 // (OperatorKernel.jl:722-759) in pass 2.  The kernels run after the
-// corresponding main pass, one launch per colour (first-touch DSS as in
-// k_fcn1/k_fcn2), over (element, level chunk) workgroups, all tracers in one
-// launch.  Tracers do not feed back on the dynamics.
+// corresponding main pass, over (element, level chunk) workgroups, all tracers
+// in one launch; like the dynamics' passes they write element copies
+// ([tracer][element][node][Nz]) and read the sums of the previous pass's.
+// They are bound by the latency of their loads, so pass 2 issues the halo
+// levels' with the own level's, and in the compact layout, whose volumes are
+// the same at all levels, fits five waves per SIMD.  Per stage, two tracers,
+// ne = 24, nz = 40, with one launch per colour and sums in place before:
+// pass 1 80 -> 59 us, pass 2 244 -> 187, limited pass 2 352 -> 296.
+// Tracers do not feed back on the dynamics.
 
 // metric component c of element e at (node, level), either layout
 template <int NN, bool CM>
@@ -896,9 +905,9 @@ __device__ __forceinline__ double met_at(const KArgs &a, size_t e, int c, int no
 
 // pass 1: the tracer caches, r = div(grad c) / (M1 + M2) with c = q / rho
 template <int N, int NZT, bool CM>
-__global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64) k_tr1(KArgs a, int slot0, int nchunk, int ntr,
+__global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64) k_tr1(KArgs a, int nchunk, int ntr,
                                                                       const double *__restrict__ U,
-                                                                      double *__restrict__ T1) {
+                                                                      double *__restrict__ E1) {
   constexpr int NN = N * N;
   extern __shared__ double smem[];
   double *Ds = smem, *DWs = Ds + NN;
@@ -906,8 +915,8 @@ __global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64) k_tr1(KArgs a, i
   load_dmats<N>(a, Ds, DWs);
   const int Nz = a.Nz;
   const int L = xcd_logical(blockIdx.x, gridDim.x);
-  const int e = a.clist[slot0 + L / nchunk];
-  const int chunk = L - (L / nchunk) * nchunk;
+  const int e = L / nchunk;
+  const int chunk = L - e * nchunk;
   const int t = threadIdx.x;
   const int node = t / NZT, l = t - node * NZT;
   const int iz = chunk * NZT + l;
@@ -916,12 +925,9 @@ __global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64) k_tr1(KArgs a, i
   const int I = node % N, J = node / N;
   const size_t vs = (size_t)a.NumG * Nz;
   double S11 = 0, S12 = 0, S21 = 0, S22 = 0, iJs = 1, iMs = 1, irho = 1;
-  bool first = false;
   size_t ui = 0;
   if (valid) {
-    const int gv = a.glob[e * NN + node];
-    first = gv < 0;
-    ui = (size_t)(gv & 0x7fffffff) * Nz + iz;
+    ui = (size_t)(a.glob[e * NN + node] & 0x7fffffff) * Nz + iz;
     if constexpr (CM) {
       const double *mN = a.met1n + (size_t)e * CGD_NMET1 * NN;
       S11 = mN[node];
@@ -943,9 +949,7 @@ __global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64) k_tr1(KArgs a, i
   }
   for (int tr = 0; tr < ntr; ++tr) {
     const size_t off = (size_t)(5 + tr) * vs;
-    double o = 0;
     if (valid) {
-      if (!first) o = T1[off + ui];
       T.at(0, node, l) = U[off + ui] * irho;
     } else if (in_tile) {
       T.at(0, node, l) = 0;
@@ -965,10 +969,8 @@ __global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64) k_tr1(KArgs a, i
       T.at(2, node, l) = Cy;
     }
     __syncthreads();
-    if (valid) {
-      const double r = dxy<N, NZT, double>(DWs, T, 1, 2, I, J, l) * iMs;
-      T1[off + ui] = first ? r : o + r;
-    }
+    if (valid)
+      E1[tr * a.ecs + ((size_t)e * NN + node) * Nz + iz] = dxy<N, NZT, double>(DWs, T, 1, 2, I, J, l) * iMs;
     __syncthreads();  // the next tracer rewrites the tiles
   }
 }
@@ -981,10 +983,9 @@ __global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64) k_tr1(KArgs a, i
 // are addressed by uniform bases plus 32-bit offsets, and the compact
 // metric layout is read per node.
 template <int N, int NZT, bool CM>
-__global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64) k_tr2(KArgs a, int slot0, int nchunk, int ntr,
-                                                                      const double *__restrict__ U,
-                                                                      const double *__restrict__ T1,
-                                                                      double *__restrict__ F) {
+__global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64) __attribute__((amdgpu_waves_per_eu(CM ? 5 : 4)))
+    k_tr2(KArgs a, int nchunk, int ntr, const double *__restrict__ U, const double *__restrict__ E1,
+          double *__restrict__ Cout, double *__restrict__ E2) {
   constexpr int NN = N * N;
   static_assert(NZT >= 3 && NZT <= 16, "chunk heights 3..16 (the DPP neighbour reach is 2)");
   extern __shared__ double smem[];
@@ -995,8 +996,8 @@ __global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64) k_tr2(KArgs a, i
   load_dmats<N>(a, Ds, DWs);
   const int Nz = a.Nz;
   const int L = xcd_logical(blockIdx.x, gridDim.x);
-  const int e = a.clist[slot0 + L / nchunk];
-  const int chunk = L - (L / nchunk) * nchunk;
+  const int e = L / nchunk;
+  const int chunk = L - e * nchunk;
   const int t = threadIdx.x;
   const int node = t / NZT, l = t - node * NZT;
   const int iz = chunk * NZT + l;
@@ -1010,10 +1011,14 @@ __global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64) k_tr2(KArgs a, i
   const double *metE = a.met + (size_t)e * (CM ? CGD_NMETP : CGD_NMET) * NNZ;
   const double *metN = CM ? a.metn + (size_t)e * CGD_NMETN * NN : nullptr;
   unsigned ui = 0, mo = 0;
+  int cpa = 0, cpb = -1;  // the node's first two element copies
+  const int *cpl = a.cpy + ((size_t)e * NN + (in_tile ? node : 0)) * a.cpw;
   bool first = false;
   if (valid) {
     const int gv = a.glob[e * NN + node];
     first = gv < 0;
+    cpa = cpl[0];
+    cpb = cpl[1];
     ui = (unsigned)(gv & 0x7fffffff) * (unsigned)Nz + iz;
     mo = (unsigned)(node * Nz + iz);
   }
@@ -1043,11 +1048,36 @@ __global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64) k_tr2(KArgs a, i
     d331 = MET0(M331);
     d332 = MET0(M332);
   }
-  const double irho = rcp(rho), iJs = rcp(Js);
-  // neighbour levels (a node's chunk is one half of a 16-lane DPP row)
+  // neighbour levels (a node's chunk is one half of a 16-lane DPP row); the
+  // halo loads of the chunk-edge lanes are issued with the own level's
   const int lr = threadIdx.x & 15;
   const bool edge_m1 = l < 1 || lr < 1, edge_m2 = l < 2 || lr < 2;
   const bool edge_p1 = l + 1 >= NZT || lr + 1 > 15, edge_p2 = l + 2 >= NZT || lr + 2 > 15;
+  const bool hm1 = valid && has_lo && edge_m1, hm2 = valid && iz >= 2 && edge_m2;
+  const bool hp1 = valid && has_hi && edge_p1, hp2 = valid && iz + 2 <= Nz - 1 && edge_p2;
+  // (the lanes' lower and upper halo levels share registers: with chunks of at
+  // least 3 levels no lane has both)
+  double hrho = 1, hu = 0, hv = 0, hw = 0, h31 = 0, h32 = 0, h33 = 0, hJ = 1, hrho2 = 1, hJ2 = 1;
+  if (hm1 || hp1) {
+    const unsigned uh = hm1 ? ui - 1 : ui + 1;
+    hrho = at(U, uh);
+    hu = at(Uu, uh);
+    hv = at(Uv, uh);
+    hw = at(Uw, uh);
+    const int off = hm1 ? -1 : 1;
+    h31 = at(metE + (size_t)(CM ? met_pidx(M311) : M311) * NNZ + (hm1 ? NNZ : 0), mo + off);
+    h32 = at(metE + (size_t)(CM ? met_pidx(M321) : M321) * NNZ + (hm1 ? NNZ : 0), mo + off);
+    if constexpr (!CM) {
+      h33 = at(metE + (size_t)M331 * NNZ + (hm1 ? NNZ : 0), mo + off);
+      hJ = MET(MJ1, off) + MET(MJ2, off);
+    }
+  }
+  if (hm2 || hp2) {
+    const int off = hm2 ? -2 : 2;
+    hrho2 = at(U, ui + off);
+    if constexpr (!CM) hJ2 = MET(MJ1, off) + MET(MJ2, off);
+  }
+  const double irho = rcp(rho), iJs = rcp(Js);
   double rho_m = dpp_from_below<1>(rho), u_m = dpp_from_below<1>(u), v_m = dpp_from_below<1>(v);
   double w_m = dpp_from_below<1>(w), d312m = dpp_from_below<1>(d312), d322m = dpp_from_below<1>(d322);
   double d332m = CM ? d332 : dpp_from_below<1>(d332);
@@ -1056,91 +1086,88 @@ __global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64) k_tr2(KArgs a, i
   double d331p = CM ? d331 : dpp_from_above<1>(d331);
   double Jm = CM ? Js : dpp_from_below<1>(Js), Jmm = CM ? Js : dpp_from_below<2>(Js);
   double Jp = CM ? Js : dpp_from_above<1>(Js), Jpp = CM ? Js : dpp_from_above<2>(Js);
-  double irm = dpp_from_below<1>(irho), irmm = dpp_from_below<2>(irho);
-  double irp = dpp_from_above<1>(irho), irpp = dpp_from_above<2>(irho);
-  if (valid) {
-    if (has_lo && edge_m1) {
-      const unsigned um = ui - 1;
-      rho_m = at(U, um);
-      u_m = at(Uu, um);
-      v_m = at(Uv, um);
-      w_m = at(Uw, um);
-      irm = rcp(rho_m);
-      d312m = MET(M312, -1);
-      d322m = MET(M322, -1);
-      if constexpr (!CM) {
-        d332m = MET(M332, -1);
-        Jm = MET(MJ1, -1) + MET(MJ2, -1);
-      }
-    }
-    if (iz >= 2 && edge_m2) {
-      irmm = rcp(at(U, ui - 2));
-      if constexpr (!CM) Jmm = MET(MJ1, -2) + MET(MJ2, -2);
-    }
-    if (has_hi && edge_p1) {
-      const unsigned up = ui + 1;
-      rho_p = at(U, up);
-      u_p = at(Uu, up);
-      v_p = at(Uv, up);
-      irp = rcp(rho_p);
-      d311p = MET(M311, 1);
-      d321p = MET(M321, 1);
-      if constexpr (!CM) {
-        d331p = MET(M331, 1);
-        Jp = MET(MJ1, 1) + MET(MJ2, 1);
-      }
-    }
-    if (iz + 2 <= Nz - 1 && edge_p2) {
-      irpp = rcp(at(U, ui + 2));
-      if constexpr (!CM) Jpp = MET(MJ1, 2) + MET(MJ2, 2);
+  const double irh = rcp(hrho), irh2 = rcp(hrho2);
+  if (hm1) {
+    rho_m = hrho;
+    u_m = hu;
+    v_m = hv;
+    w_m = hw;
+    d312m = h31;
+    d322m = h32;
+    if constexpr (!CM) {
+      d332m = h33;
+      Jm = hJ;
     }
   }
+  if constexpr (!CM)
+    if (hm2) Jmm = hJ2;
+  if (hp1) {
+    rho_p = hrho;
+    u_p = hu;
+    v_p = hv;
+    d311p = h31;
+    d321p = h32;
+    if constexpr (!CM) {
+      d331p = h33;
+      Jp = hJ;
+    }
+  }
+  if constexpr (!CM)
+    if (hp2) Jpp = hJ2;
   // clamped levels iz-1, iz-2 >= 0 and iz+2 <= Nz-1 (the reference's max/min);
   // at iz = 0 the shifted values belong to another node's lanes
   if (iz == 0) Jm = Js;
-  if (iz == 1) {
-    irmm = irm;
-    Jmm = Jm;
-  }
-  if (iz + 2 > Nz - 1) {
-    irpp = irp;
-    Jpp = Jp;
-  }
+  if (iz == 1) Jmm = Jm;
+  if (iz + 2 > Nz - 1) Jpp = Jp;
   // contravariant mass fluxes through the interfaces (Contra3)
   double wlo = 0, wup = 0;
   if (valid && has_lo) wlo = rho_m * (d312m * u_m + d322m * v_m + d332m * w_m) + rho * (d311 * u + d321 * v + d331 * w_m);
   if (valid && has_hi) wup = rho * (d312 * u + d322 * v + d332 * w) + rho_p * (d311p * u_p + d321p * v_p + d331p * w);
   // RecU4 weights of the upper interface (and of the lower one, used by the
   // lanes at a chunk's bottom edge), shared by all tracers
-  const RecW<double> Wup = recu4_weights(Jm, Js, Jp, Jpp);
-  const RecW<double> Wlo = recu4_weights(Jmm, Jm, Js, has_hi ? Jp : Js);
+  // (the compact layout's volumes are those of every level)
+  const RecW<double> Wup = CM ? recu4_equal<double>() : recu4_weights(Jm, Js, Jp, Jpp);
+  const RecW<double> Wlo = CM ? recu4_equal<double>() : recu4_weights(Jmm, Jm, Js, has_hi ? Jp : Js);
+  pin(wlo, wup);
   // the tracer-independent tiles: (uc, vc) = Contra12(-rho, u, v)
   if (in_tile) {
     T.at(0, node, l) = -rho * (S11 * u + S12 * v);
     T.at(1, node, l) = -rho * (S21 * u + S22 * v);
   }
+  // Contra12 of Grad12 with rho / J: a symmetric matrix
+  double Gxx = (S11 * S11 + S12 * S12) * rho * iJs, Gxy = (S11 * S21 + S12 * S22) * rho * iJs;
+  double Gyy = (S21 * S21 + S22 * S22) * rho * iJs;
+  pin(Gxx, Gxy, Gyy);
   for (int tr = 0; tr < ntr; ++tr) {
     // two sets of per-tracer tiles (C, c, Cx, Cy) used alternately, so a
     // tracer's tiles are never rewritten before every lane has passed the
     // next tracer's first barrier
     const int b = 2 + 4 * (tr & 1);
     const double *Q = U + (size_t)(5 + tr) * vs;
-    const double *C = T1 + (size_t)(5 + tr) * vs;
-    double *Ft = F + (size_t)(5 + tr) * vs;
-    double o = 0, cown = 0, Cown = 0;
+    const double *C = E1 + tr * a.ecs;
+    double cown = 0, Cown = 0, Cb = 0, q1 = 0, q2 = 0;
     if (valid) {
-      if (!first) o = at(Ft, ui);
-      cown = at(Q, ui) * irho;
-      Cown = at(C, ui);
+      cown = at(Q, ui);
+      Cown = C[(size_t)cpa * Nz + iz];
     }
+    if (hm1 || hp1) q1 = at(Q, hm1 ? ui - 1 : ui + 1);
+    if (hm2 || hp2) q2 = at(Q, hm2 ? ui - 2 : ui + 2);
+    if (cpb >= 0) {
+      Cb = C[(size_t)cpb * Nz + iz];
+      for (int q = 2; q < a.cpw && cpl[q] >= 0; ++q) {
+        Cown += Cb;
+        Cb = C[(size_t)cpl[q] * Nz + iz];
+      }
+    }
+    cown *= irho;
     double c_m = dpp_from_below<1>(cown), c_mm = dpp_from_below<2>(cown);
     double c_p = dpp_from_above<1>(cown), c_pp = dpp_from_above<2>(cown);
-    if (valid) {
-      if (has_lo && edge_m1) c_m = at(Q, ui - 1) * irm;
-      if (iz >= 2 && edge_m2) c_mm = at(Q, ui - 2) * irmm;
-      if (has_hi && edge_p1) c_p = at(Q, ui + 1) * irp;
-      if (iz + 2 <= Nz - 1 && edge_p2) c_pp = at(Q, ui + 2) * irpp;
-    }
+    if (hm1) c_m = q1 * irh;
+    if (hm2) c_mm = q2 * irh2;
+    if (hp1) c_p = q1 * irh;
+    if (hp2) c_pp = q2 * irh2;
+    Cown += Cb;
+    if (Cout && first) at(Cout + (size_t)(5 + tr) * vs, ui) = Cown;  // Temp1
     if (iz == 0) c_m = cown;
     if (iz == 1) c_mm = c_m;
     if (iz + 2 > Nz - 1) c_pp = c_p;
@@ -1151,17 +1178,9 @@ __global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64) k_tr2(KArgs a, i
     // upper-interface flux; the lower one is the upper flux of the level
     // below, taken from its lane (lanes at a chunk's bottom edge compute it)
     double Fup = 0;
-    if (valid && has_hi) {
-      double cFL, cFR;
-      recu4_apply(c_m, cown, c_p, c_pp, Wup, cFL, cFR);
-      Fup = 0.25 * ((fabs(wup) + wup) * cFL + (-fabs(wup) + wup) * cFR);
-    }
+    if (valid && has_hi) Fup = recu4_flux(c_m, cown, c_p, c_pp, Wup, wup);
     double Flo = dpp_from_below<1>(Fup);
-    if (valid && has_lo && edge_m1) {
-      double cFL, cFR;
-      recu4_apply(c_mm, c_m, cown, has_hi ? c_p : cown, Wlo, cFL, cFR);
-      Flo = 0.25 * ((fabs(wlo) + wlo) * cFL + (-fabs(wlo) + wlo) * cFR);
-    }
+    if (valid && has_lo && edge_m1) Flo = recu4_flux(c_mm, c_m, cown, has_hi ? c_p : cown, Wlo, wlo);
     __syncthreads();
     double f = 0;
     if (in_tile) {
@@ -1169,22 +1188,20 @@ __global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64) k_tr2(KArgs a, i
       if (valid) {
         const double Dxc = dx<N, NZT, double>(Ds, T, b, I, J, l);
         const double Dyc = dy<N, NZT, double>(Ds, T, b, I, J, l);
-        const double GDx = (S11 * Dxc + S21 * Dyc) * iJs;
-        const double GDy = (S12 * Dxc + S22 * Dyc) * iJs;
-        Cx = rho * (S11 * GDx + S12 * GDy);  // Contra12 with rho
-        Cy = rho * (S21 * GDx + S22 * GDy);
+        Cx = Gxx * Dxc + Gxy * Dyc;
+        Cy = Gxy * Dxc + Gyy * Dyc;
         // horizontal transport: sum_k D (uc c) over the element row / column
-        f += dxy_prod<N, NZT, double>(Ds, T, 0, 1, b + 1, I, J, l) * iMs;
-        if (has_lo) f += Flo * iMs;
-        if (has_hi) f -= Fup * iMs;
+        f = dxy_prod<N, NZT, double>(Ds, T, 0, 1, b + 1, I, J, l);
+        if (has_lo) f += Flo;
+        f -= Fup;
       }
       T.at(b + 2, node, l) = Cx;
       T.at(b + 3, node, l) = Cy;
     }
     __syncthreads();
     if (valid) {
-      f += -Kd * dxy<N, NZT, double>(DWs, T, b + 2, b + 3, I, J, l) * iMs;
-      at(Ft, ui) = first ? f : o + f;
+      f = (f - Kd * dxy<N, NZT, double>(DWs, T, b + 2, b + 3, I, J, l)) * iMs;
+      E2[tr * a.ecs + (size_t)e * NNZ + mo] = f;
     }
   }
 #undef MET
@@ -1261,9 +1278,9 @@ __device__ __forceinline__ double half_tree_sum(double x) {
 // M1 + M2 (the reference indexes its 3-D M with two indices here).
 template <int N, int NZT, bool CM>
 __global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64)
-    k_tr2_lim(KArgs a, int slot0, int nchunk, int ntr, const double *__restrict__ U, const int *__restrict__ stencil,
+    k_tr2_lim(KArgs a, int nchunk, int ntr, const double *__restrict__ U, const int *__restrict__ stencil,
               int NF, const double *__restrict__ qmin, const double *__restrict__ qmax, double dtau,
-              double *__restrict__ F) {
+              double *__restrict__ E2) {
   constexpr int NN = N * N;
   static_assert(NN <= 32, "a 32-lane half of a wavefront holds the nodes of an element level");
   extern __shared__ double smem[];
@@ -1275,8 +1292,8 @@ __global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64)
   if (threadIdx.x < NN) Ds[threadIdx.x] = a.D[threadIdx.x];
   const int Nz = a.Nz;
   const int L = xcd_logical(blockIdx.x, gridDim.x);
-  const int e = a.clist[slot0 + L / nchunk];
-  const int chunk = L - (L / nchunk) * nchunk;
+  const int e = L / nchunk;
+  const int chunk = L - e * nchunk;
   const int t = threadIdx.x;
   const int node = t / NZT, l = t - node * NZT;
   const int iz = chunk * NZT + l;
@@ -1287,14 +1304,11 @@ __global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64)
   const bool has_lo = iz > 0, has_hi = iz < Nz - 1;
   auto M = [&](int c, int Lv) { return met_at<NN, CM>(a, (size_t)e, c, node, Lv); };
   size_t ui = 0;
-  bool first = false;
   double rho = 1, u = 0, v = 0, S11 = 0, S12 = 0, S21 = 0, S22 = 0, Js = 1, Ms = 1;
   double wlo = 0, wup = 0, rho_m = 1, rho_mm = 1, rho_p = 1, rho_pp = 1;
   double Jm = 1, Jmm = 1, Jp = 1, Jpp = 1;
   if (valid) {
-    const int gv = a.glob[(size_t)e * NN + node];
-    first = gv < 0;
-    ui = (size_t)(gv & 0x7fffffff) * Nz + iz;
+    ui = (size_t)(a.glob[(size_t)e * NN + node] & 0x7fffffff) * Nz + iz;
     rho = U[ui];
     u = U[vs + ui];
     v = U[2 * vs + ui];
@@ -1314,17 +1328,17 @@ __global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64)
     Jmm = M(MJ1, lmm) + M(MJ2, lmm);
     Jp = M(MJ1, lp) + M(MJ2, lp);
     Jpp = M(MJ1, lpp) + M(MJ2, lpp);
-    // Contra3 at the two interfaces (the reference's operation order)
-    if (has_lo) {
-      const double w = U[3 * vs + ui - 1];
-      wlo = rho_m * (M(M312, iz - 1) * U[vs + ui - 1] + M(M322, iz - 1) * U[2 * vs + ui - 1] + M(M332, iz - 1) * w) +
-            rho * (M(M311, iz) * u + M(M321, iz) * v + M(M331, iz) * w);
-    }
-    if (has_hi) {
-      const double w = U[3 * vs + ui];
-      wup = rho * (M(M312, iz) * u + M(M322, iz) * v + M(M332, iz) * w) +
-            rho_p * (M(M311, iz + 1) * U[vs + ui + 1] + M(M321, iz + 1) * U[2 * vs + ui + 1] + M(M331, iz + 1) * w);
-    }
+    // Contra3 at the two interfaces (the reference's operation order); the
+    // loads at clamped levels, so that they need no branch and all take one
+    // round trip
+    const double *um = U + ui - iz + lm, *up = U + ui - iz + lp;
+    const double wm = um[3 * vs], w = U[3 * vs + ui];
+    const double lo = rho_m * (M(M312, lm) * um[vs] + M(M322, lm) * um[2 * vs] + M(M332, lm) * wm) +
+                      rho * (M(M311, iz) * u + M(M321, iz) * v + M(M331, iz) * wm);
+    const double hi = rho * (M(M312, iz) * u + M(M322, iz) * v + M(M332, iz) * w) +
+                      rho_p * (M(M311, lp) * up[vs] + M(M321, lp) * up[2 * vs] + M(M331, lp) * w);
+    if (has_lo) wlo = lo;
+    if (has_hi) wup = hi;
   }
   if (in_tile) {
     T.at(0, node, l) = -rho * (S11 * u + S12 * v);  // Contra12(-rho, u, v)
@@ -1348,8 +1362,9 @@ __global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64)
     }
   };
   // RecU4 weights of both interfaces, shared by all tracers
-  const RecW<double> Wup = recu4_weights(Jm, Js, Jp, Jpp);
-  const RecW<double> Wlo = recu4_weights(Jmm, Jm, Js, has_hi ? Jp : Js);
+  // (the compact layout's volumes are those of every level)
+  const RecW<double> Wup = CM ? recu4_equal<double>() : recu4_weights(Jm, Js, Jp, Jpp);
+  const RecW<double> Wlo = CM ? recu4_equal<double>() : recu4_weights(Jmm, Jm, Js, has_hi ? Jp : Js);
   // a node's levels sit in one DPP row (or half of one), so the neighbour
   // levels' mixing ratios and the lower interface's flux come from the
   // neighbouring lanes; lanes at a chunk edge load or compute their own
@@ -1358,33 +1373,34 @@ __global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64)
   const bool edge_p1 = l + 1 >= NZT || lr + 1 > 15, edge_p2 = l + 2 >= NZT || lr + 2 > 15;
   const int lw0 = 2 * wave + (lane >> 5), iz0 = chunk * NZT + lw0;  // this half's first level in phase B
   const bool live0 = 2 * wave < NZT && lw0 < NZT && iz0 < Nz;
-  // this level's tracer density and DSS accumulator, one tracer ahead
-  double Trs_n = 0, o_n = 0;
-  if (valid && ntr > 0) {
-    Trs_n = U[5 * vs + ui];
-    if (!first) o_n = F[5 * vs + ui];
-  }
-  for (int tr = 0; tr < ntr; ++tr) {
+  const bool hm1 = valid && has_lo && edge_m1, hm2 = valid && iz >= 2 && edge_m2;
+  const bool hp1 = valid && has_hi && edge_p1, hp2 = valid && iz + 2 <= Nz - 1 && edge_p2;
+  // (no lane of a chunk of at least 3 levels has a halo level on both sides)
+  const double rho1 = hm1 ? rho_m : rho_p, rho2 = hm2 ? rho_mm : rho_pp;
+  // this level's tracer density and the halo levels', one tracer ahead
+  double Trs_n = 0, q1n = 0, q2n = 0;
+  auto load = [&](int tr) {
     const double *Tr = U + (size_t)(5 + tr) * vs;
-    double *Ft = F + (size_t)(5 + tr) * vs;
+    if (valid) Trs_n = Tr[ui];
+    if (hm1 || hp1) q1n = Tr[hm1 ? ui - 1 : ui + 1];
+    if (hm2 || hp2) q2n = Tr[hm2 ? ui - 2 : ui + 2];
+  };
+  if (ntr > 0) load(0);
+  for (int tr = 0; tr < ntr; ++tr) {
     // phase B's bounds of the first level pair, loaded ahead of phase A
     double qMin0 = 0, qMax0 = 0;
     if (live0) bounds(tr, iz0, qMin0, qMax0);
-    const double Trs = Trs_n, o = o_n;
-    if (valid && tr + 1 < ntr) {
-      Trs_n = Tr[vs + ui];
-      if (!first) o_n = Ft[vs + ui];
-    }
+    const double Trs = Trs_n, q1 = q1n, q2 = q2n;
+    if (tr + 1 < ntr) load(tr + 1);
     double c = 0, f = 0;
     if (valid) c = Trs / rho;
     double cm = dpp_from_below<1>(c), cmm = dpp_from_below<2>(c);
     double cp = dpp_from_above<1>(c), cpp = dpp_from_above<2>(c);
-    if (valid) {
-      if (has_lo && edge_m1) cm = Tr[ui - 1] / rho_m;
-      if (iz >= 2 && edge_m2) cmm = Tr[ui - 2] / rho_mm;
-      if (has_hi && edge_p1) cp = Tr[ui + 1] / rho_p;
-      if (iz + 2 <= Nz - 1 && edge_p2) cpp = Tr[ui + 2] / rho_pp;
-    }
+    const double c1 = q1 / rho1, c2 = q2 / rho2;
+    if (hm1) cm = c1;
+    if (hm2) cmm = c2;
+    if (hp1) cp = c1;
+    if (hp2) cpp = c2;
     // clamped levels (the reference's max/min)
     if (!has_lo) cm = c;
     if (iz < 2) cmm = cm;
@@ -1393,17 +1409,9 @@ __global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64)
     // upwind vertical flux through the upper interface; the lower one is the
     // upper flux of the level below (the unlimited kernel's fluxes)
     double Fup = 0;
-    if (valid && has_hi) {
-      double cFL, cFR;
-      recu4_apply(cm, c, cp, cpp, Wup, cFL, cFR);
-      Fup = 0.25 * ((fabs(wup) + wup) * cFL + (-fabs(wup) + wup) * cFR);
-    }
+    if (valid && has_hi) Fup = recu4_flux(cm, c, cp, cpp, Wup, wup);
     double Flo = dpp_from_below<1>(Fup);
-    if (valid && has_lo && edge_m1) {
-      double cFL, cFR;
-      recu4_apply(cmm, cm, c, has_hi ? cp : c, Wlo, cFL, cFR);
-      Flo = 0.25 * ((fabs(wlo) + wlo) * cFL + (-fabs(wlo) + wlo) * cFR);
-    }
+    if (valid && has_lo && edge_m1) Flo = recu4_flux(cmm, cm, c, has_hi ? cp : c, Wlo, wlo);
     if (valid) {
       if (has_lo) f += Flo / Ms;
       if (has_hi) f += -Fup / Ms;
@@ -1484,11 +1492,35 @@ __global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64)
     __syncthreads();  // (C) the clipped q of every node
     if (valid) {
       f += (wQ[l * NN + node] * RhoS - Trs) * Js / dtau / Ms;
-      Ft[ui] = first ? f : o + f;
+      E2[tr * a.ecs + ((size_t)e * NN + node) * Nz + iz] = f;
     }
     // the next tracer writes tile 2, wS and wT after barrier (A), and wQ
     // after (B), which every lane reaches only after reading them here
   }
+}
+
+// The sum of a global point's element copies E, in colour order.
+__device__ __forceinline__ double copies_sum(const KArgs &a, const double *__restrict__ E, unsigned ip) {
+  const unsigned g = ip / (unsigned)a.Nz, iz = ip - g * (unsigned)a.Nz;
+  const int *cp = a.gcpy + (size_t)g * a.cpw;
+  const int c0 = cp[0], c1 = cp[1];
+  double v = E[(size_t)c0 * a.Nz + iz];
+  if (c1 >= 0) {
+    double y = E[(size_t)c1 * a.Nz + iz];
+    for (int q = 2; q < a.cpw && cp[q] >= 0; ++q) {
+      v += y;
+      y = E[(size_t)cp[q] * a.Nz + iz];
+    }
+    v += y;
+  }
+  return v;
+}
+
+// F of the tracers from their element copies, for callers that want F and
+// for the microphysics; tracer blockIdx.y
+__global__ void k_tr_dss(KArgs a, const double *__restrict__ E, double *__restrict__ F, unsigned ng) {
+  for (unsigned ip = blockIdx.x * blockDim.x + threadIdx.x; ip < ng; ip += gridDim.x * blockDim.x)
+    F[(size_t)blockIdx.y * ng + ip] = copies_sum(a, E + blockIdx.y * a.ecs, ip);
 }
 
 // SchurSolveBKernel! for the tracers (SchurSolve.jl:106-109): k = fac v
@@ -1499,13 +1531,18 @@ __global__ void k_tr_scale(const double *__restrict__ v, double *__restrict__ k,
 
 // Rosenbrock stage arithmetic of the tracers (k = fac v, SchurSolve.jl:106-109):
 // v = fV + sum_j cf[j] k_j; k = fac v; V = Vn + sum_j av[j] k_j (+ av[STAGE] k).
-// Stage 0 reads V and stores it as Vn.
+// Stage 0 reads V and stores it as Vn.  fV is summed here from the element
+// copies E, unless it is given (the microphysics adds to the sums).
+// Tracer blockIdx.y; ng points each.
 template <int STAGE>
-__global__ void k_rw_tr(const double *__restrict__ fV, const double *__restrict__ k0, const double *__restrict__ k1,
-                        double cf0, double cf1, double av0, double av1, double av2, double fac, double *__restrict__ V,
-                        double *__restrict__ Vn, double *__restrict__ kout, size_t n) {
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-    double v = fV[i];
+__global__ void k_rw_tr(KArgs a, const double *__restrict__ E, const double *__restrict__ fV,
+                        const double *__restrict__ k0, const double *__restrict__ k1, double cf0, double cf1,
+                        double av0, double av1, double av2, double fac, double *__restrict__ V,
+                        double *__restrict__ Vn, double *__restrict__ kout, unsigned ng) {
+  const size_t off = (size_t)blockIdx.y * ng;
+  for (unsigned ip = blockIdx.x * blockDim.x + threadIdx.x; ip < ng; ip += gridDim.x * blockDim.x) {
+    const size_t i = off + ip;
+    double v = fV ? fV[i] : copies_sum(a, E + blockIdx.y * a.ecs, ip);
     double kp0 = 0, kp1 = 0;
     if (STAGE > 0) {
       kp0 = k0[i];

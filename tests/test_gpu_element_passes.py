@@ -211,3 +211,35 @@ def test_prepare_theta(pkg, torch_cuda, scale):
     bad[0, :3] = True
     assert torch.equal(torch.isnan(th), torch.isnan(want)) and torch.isnan(th[bad]).all()
     assert float(((th - want) / want)[~bad].abs().max()) <= 1e-14
+
+
+@pytest.mark.parametrize("limited", [False, True])
+@pytest.mark.parametrize("metric", ["compact", "full"])
+@pytest.mark.parametrize("p,nz,chunk,ntr", [(4, 3, 8, 1), (4, 9, 8, 3), (4, 17, 16, 2), (3, 8, 8, 2), (3, 25, 8, 1)])
+def test_tracer_passes(pkg, oracle_mod, torch_cuda, monkeypatch, p, nz, chunk, ntr, metric, limited):
+    """The tracers' element copies, halo levels and upwind fluxes, with equal
+    and with general layer volumes, in steps (and in the plain transport's
+    tendency and caches)."""
+    torch, host = torch_cuda, pkg.host
+    if metric == "full":
+        monkeypatch.setenv("CGD_METRIC", "full")
+    print(f"tracers p={p} nz={nz} chunk={chunk} NumTr={ntr} {metric} limited={limited}", flush=True)
+    disc, phys, dev, orc = setup(pkg, oracle_mod, 2, p, nz, H=512.0 * nz, NumTr=ntr, horlimit=limited)
+    FE, Metric, Global, Cache, JCache = dev
+    host.init_context(FE, Metric, phys, Global).set_launch_shape(chunk_levels=chunk)
+    U0 = noisy_state(pkg, disc, 9)
+    q = 0.01 * (1.0 + 0.5 * np.random.default_rng(9).random((ntr,) + U0[0].shape))
+    U0 = np.concatenate([U0, q * U0[0:1]], axis=0)
+    if not limited:
+        F, T1 = tendency(torch, host, phys, dev, U0)
+        Fo, T1o = orc.fcn(U0.copy(), orc.prepare(U0.copy()))
+        for v in range(5 + ntr):
+            assert rel_l2(F[v], Fo[v]) <= TOL, f"F{v + 1} {rel_l2(F[v], Fo[v]):.3e}"
+            assert rel_l2(T1[v], T1o[v]) <= TOL, f"Temp1[{v}] {rel_l2(T1[v], T1o[v]):.3e}"
+    V = torch.as_tensor(U0, device="cuda").clone()
+    host.TimeStepper(V, 100.0, 2, FE, Metric, phys, Cache, JCache, Global)
+    torch.cuda.synchronize()
+    Vo = U0.copy()
+    orc.rw_step(Vo, 100.0, 2)
+    for v in range(5 + ntr):
+        assert rel_l2(V[v].cpu().numpy(), Vo[v]) <= TOL, f"V{v + 1} {rel_l2(V[v].cpu().numpy(), Vo[v]):.3e}"
