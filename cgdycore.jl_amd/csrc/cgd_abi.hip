@@ -64,6 +64,8 @@ struct cgd_ctx {
   // or 32 for two columns per wavefront when Nz <= 32) and workgroup size
   int colw = 64, colblock = 256;
   int col1 = 0;    // pass 1 over whole columns (k_fcn1c), until its chunk height is set
+  // k_fcn1 and k_fcn2r in chunks of 16 levels, until their chunk heights are set
+  int p16 = 0, r16 = 0;
   int items1 = 1;  // pass-1 work items (element, level chunk) per workgroup: 1 or 2
   // one persistent launch per RW stage (k_stage_persist): on/off, its grid
   // (workgroups resident at once), the grid barrier's state and wait bound
@@ -91,10 +93,10 @@ struct cgd_ctx {
 // two sets of 7 tiles and the per-node horizontal metric
 // FP32 element kernels: an FP64 region for the theta hyperviscosity after
 // the R-typed LDS (pass 1: D, DW and three tiles; pass 2: DW and three tiles)
-template <typename R> static size_t lds_fcn1(const cgd_ctx *c) {
-  const size_t r = sizeof(R) * (2 * c->NN + 9 * c->NN * c->nzt1);
+template <typename R> static size_t lds_fcn1(const cgd_ctx *c, int nzt1) {
+  const size_t r = sizeof(R) * (2 * c->NN + 9 * c->NN * nzt1);
   if (std::is_same<R, double>::value) return r;
-  return (r + 7) / 8 * 8 + sizeof(double) * (2 * c->NN + 3 * c->NN * c->nzt1);
+  return (r + 7) / 8 * 8 + sizeof(double) * (2 * c->NN + 3 * c->NN * nzt1);
 }
 template <typename R> static size_t lds_fcn2(const cgd_ctx *c) {
   // + the horizontal metric: 12 values per node (compact layout), 10 per point
@@ -109,10 +111,18 @@ template <typename R> static size_t lds_fcn2(const cgd_ctx *c) {
 // k_fcn1c: three tiles of whole columns, one of them FP64
 static size_t lds_fcn1c(const cgd_ctx *c, size_t r) { return (size_t)c->NN * 64 * (sizeof(double) + 2 * r); }
 
+// the chunk heights of pass 1 and, for the tendency in type R, of pass 2
+static int cache_nzt(const cgd_ctx *c) { return c->p16 && !c->persistent ? 16 : c->nzt1; }
+template <typename R> static int tend_nzt(const cgd_ctx *c) {
+  return std::is_same<R, double>::value && c->r16 && !c->persistent ? 16 : c->nzt;
+}
+template <typename R> static int tend_nchunk(const cgd_ctx *c) {
+  return (c->Nz + tend_nzt<R>(c) - 1) / tend_nzt<R>(c);
+}
 // k_fcn2r: D, DW, 12 tiles, four tiles with the level below, its sums, the
 // horizontal metric and 1/(2 M)
-static size_t lds_fcn2r(const cgd_ctx *c) {
-  return sizeof(double) * (2 * c->NN + 12 * c->NN * c->nzt + 4 * c->NN * (c->nzt + 1) + 7 * c->NN);
+static size_t lds_fcn2r(const cgd_ctx *c, int nzt) {
+  return sizeof(double) * (2 * c->NN + 12 * c->NN * nzt + 4 * c->NN * (nzt + 1) + 7 * c->NN);
 }
 
 static int fail(cgd_ctx *c, int code, const std::string &msg) {
@@ -733,6 +743,16 @@ static int ctx_build(cgd_ctx *c, const cgd_desc *ds, int nmem, hipStream_t st) {
   // instead of 190 (ne = 30), at Nz = 40 the idle lanes make it 1 % slower
   // than the chunks, so it is taken from three quarters of a wavefront on.
   c->col1 = c->cm && Nz >= 48 && Nz <= 64;
+  // 16 levels per workgroup where that pads no more levels than 8 do (nz = 40,
+  // padded to 48: pass 1 15 %, pass 2 25 % slower) and leaves the chip a few
+  // rounds of workgroups: 128-byte pieces of the columns, and in pass 2 half
+  // the halo levels.  Pass 1, 32 grids of 32 levels: a step 1.5 % faster; where
+  // it can't take whole columns.  Pass 2 at nz = 64: 502 -> 487 us (ne = 30),
+  // 1900 -> 1856 (ne = 60); at nz = 32 no faster (the ensemble 0.4 % slower),
+  // so from 48 levels on.
+  const bool tall = c->N == 5 && !(((Nz + 7) / 8) & 1) && (size_t)NF * ((Nz + 15) / 16) >= 4096;
+  c->p16 = tall && c->cm && !c->col1;
+  c->r16 = tall && Nz >= 48 && c->reg && !c->smooth;
   c->ok = true;
   return CGD_OK;
 }
@@ -847,20 +867,23 @@ extern "C" int cgd_profile_read(cgd_ctx *c, int which, double *total_ms, long lo
 // template dispatch on (N, chunk height, metric layout); R is the tendency
 // type (double, or float in the mixed-precision mode)
 template <int N, int NZT, bool CM, typename R>
-static void fcn1_t(cgd_ctx *c, int nitems, hipStream_t st, const R *UR, R *E, const double *U64, double *Eth) {
+static void fcn1_t(cgd_ctx *c, hipStream_t st, const R *UR, R *E, const double *U64, double *Eth) {
+  const int nchunk = (c->Nz + NZT - 1) / NZT, nitems = c->NF * nchunk;
+  const dim3 b((N * N * NZT + 63) / 64 * 64);
+  const size_t lds = lds_fcn1<R>(c, NZT);
   if (c->items1 == 2)
-    hipLaunchKernelGGL((k_fcn1<N, NZT, CM, R, 2>), dim3((nitems + 1) / 2), dim3(c->block1), lds_fcn1<R>(c), st,
-                       c->ka, c->nchunk1, nitems, UR, E, U64, Eth);
+    hipLaunchKernelGGL((k_fcn1<N, NZT, CM, R, 2>), dim3((nitems + 1) / 2), b, lds, st, c->ka, nchunk, nitems, UR, E,
+                       U64, Eth);
   else
-    hipLaunchKernelGGL((k_fcn1<N, NZT, CM, R, 1>), dim3(nitems), dim3(c->block1), lds_fcn1<R>(c), st, c->ka,
-                       c->nchunk1, nitems, UR, E, U64, Eth);
+    hipLaunchKernelGGL((k_fcn1<N, NZT, CM, R, 1>), dim3(nitems), b, lds, st, c->ka, nchunk, nitems, UR, E, U64, Eth);
 }
 template <int N, int NZT, bool CM, typename R>
 static void fcn2_t(cgd_ctx *c, dim3 g, hipStream_t st, const double *U, const R *UR, const R *E1, const double *P,
                    R *E2, const double *E1th, double *Cout) {
   if constexpr (std::is_same<R, double>::value && CM) {
     if (c->reg && !c->smooth) {
-      hipLaunchKernelGGL((k_fcn2r<N, NZT>), g, dim3(c->block), lds_fcn2r(c), st, c->ka, c->nchunk, U, E1, P, E2,
+      hipLaunchKernelGGL((k_fcn2r<N, NZT>), g, dim3((N * N * NZT + 63) / 64 * 64), lds_fcn2r(c, NZT), st, c->ka,
+                         tend_nchunk<R>(c), U, E1, P, E2,
                          c->d_f4x, Cout);
       return;
     }
@@ -910,19 +933,19 @@ static void tr2lim_t(cgd_ctx *c, int nitems, hipStream_t st, const double *U) {
 }
 
 template <typename R>
-static void launch_fcn1(cgd_ctx *c, int nitems, hipStream_t st, const R *UR, R *E, const double *U64, double *Eth) {
+static void launch_fcn1(cgd_ctx *c, hipStream_t st, const R *UR, R *E, const double *U64, double *Eth) {
   if (c->col1) {
     const size_t lds = lds_fcn1c(c, sizeof(R));
     if (c->N == 5) hipLaunchKernelGGL((k_fcn1c<5, R>), dim3(c->NF), dim3(320), lds, st, c->ka, UR, E, U64, Eth);
     else hipLaunchKernelGGL((k_fcn1c<4, R>), dim3(c->NF), dim3(256), lds, st, c->ka, UR, E, U64, Eth);
     return;
   }
-  CGD_DISPATCH(fcn1_t, R, c->nzt1, nitems, st, UR, E, U64, Eth);
+  CGD_DISPATCH(fcn1_t, R, cache_nzt(c), st, UR, E, U64, Eth);
 }
 template <typename R>
 static void launch_fcn2(cgd_ctx *c, dim3 g, hipStream_t st, const double *U, const R *UR, const R *E1,
                         const double *P, R *E2, const double *E1th, double *Cout) {
-  CGD_DISPATCH(fcn2_t, R, c->nzt, g, st, U, UR, E1, P, E2, E1th, Cout);
+  CGD_DISPATCH(fcn2_t, R, tend_nzt<R>(c), g, st, U, UR, E1, P, E2, E1th, Cout);
 }
 
 extern "C" int cgd_prepare(cgd_ctx *c, const double *U, double *AuxG, void *stream) {
@@ -958,7 +981,7 @@ static int run_fcn(cgd_ctx *c, R *F, const double *U, const R *UR, R *Temp1, con
   double *const E1th = e1_theta<R>(c);
   prof_begin(c, st, 0);
   int launches = 1;
-  launch_fcn1<R>(c, c->NF * c->nchunk1, st, UR, E1, U, E1th);
+  launch_fcn1<R>(c, st, UR, E1, U, E1th);
   HIPCHK(c, hipGetLastError());
   // the tracers run in FP64 in both modes: their tendencies and caches are
   // components 6.. of the FP64 F and Temp1 (the mixed mode's FP32 dynamics
@@ -973,7 +996,7 @@ static int run_fcn(cgd_ctx *c, R *F, const double *U, const R *UR, R *Temp1, con
   if ((r = prof_end(c, st, 0, launches))) return r;
   prof_begin(c, st, 1);
   launches = 0;
-  launch_fcn2<R>(c, dim3(c->NF * c->nchunk), st, U, UR, E1, AuxG, E2, E1th, want_f ? T1d : nullptr);
+  launch_fcn2<R>(c, dim3(c->NF * tend_nchunk<R>(c)), st, U, UR, E1, AuxG, E2, E1th, want_f ? T1d : nullptr);
   HIPCHK(c, hipGetLastError());
   ++launches;
   {
@@ -1006,10 +1029,10 @@ static int run_fcn(cgd_ctx *c, R *F, const double *U, const R *UR, R *Temp1, con
     const R *F4x = reinterpret_cast<const R *>(c->d_f4x);
     if (has_hooks(c))
       hipLaunchKernelGGL((k_dss<R, true>), g, dim3(256), 0, st, c->ka, c->hooks, U, AuxG, E2, F4x, F, Fd,
-                         c->nchunk, c->nzt);
+                         tend_nchunk<R>(c), tend_nzt<R>(c));
     else
       hipLaunchKernelGGL((k_dss<R, false>), g, dim3(256), 0, st, c->ka, c->hooks, U, AuxG, E2, F4x, F, Fd,
-                         c->nchunk, c->nzt);
+                         tend_nchunk<R>(c), tend_nzt<R>(c));
     HIPCHK(c, hipGetLastError());
     ++launches;
   }
@@ -1111,7 +1134,7 @@ template <int N, typename R, int W> static const void *persist_fn(const cgd_ctx 
   return reinterpret_cast<const void *>(&k_stage_persist<N, true, R, W, false>);
 }
 template <typename R> static size_t lds_persist(const cgd_ctx *c) {
-  return std::max(lds_fcn1<R>(c), std::is_same<R, double>::value && c->reg ? lds_fcn2r(c) : lds_fcn2<R>(c));
+  return std::max(lds_fcn1<R>(c, c->nzt1), std::is_same<R, double>::value && c->reg ? lds_fcn2r(c, c->nzt) : lds_fcn2<R>(c));
 }
 
 // The grid: every workgroup resident at once (the kernel's occupancy per CU
@@ -1209,8 +1232,8 @@ static int rw_step_fused(cgd_ctx *c, double *V, double dt, const cgd_rw_work *w,
     rw.k = is < 2 ? kR[is] : nullptr;  // k_3 is consumed in registers
     rw.P = (is < 2 || more) ? w->AuxG : nullptr;
     rw.F4x = reinterpret_cast<const R *>(c->d_f4x);
-    rw.nchunk = c->nchunk;
-    rw.nzt = c->nzt;
+    rw.nchunk = tend_nchunk<R>(c);
+    rw.nzt = tend_nzt<R>(c);
     rw.fac = dt * gamma;
     rw.invfac = 1.0 / rw.fac;
     rw.invfac2 = rw.invfac / rw.fac;
@@ -1405,7 +1428,8 @@ extern "C" int cgd_set_launch_shape(cgd_ctx *c, const cgd_launch_shape *shape) {
                 "-1; a persistent launch takes chunk heights 8, pass1_items 1 and col_block = 64 * ceil(N*N*8 / 64)");
   graph_free(c);  // a captured graph keeps the old shapes
   apply_shape(c, sh);
-  if (shape->pass1_chunk_levels) c->col1 = 0;
+  if (shape->pass1_chunk_levels) c->col1 = c->p16 = 0;
+  if (shape->chunk_levels) c->r16 = 0;
   return CGD_OK;
 }
 

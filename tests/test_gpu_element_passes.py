@@ -243,3 +243,28 @@ def test_tracer_passes(pkg, oracle_mod, torch_cuda, monkeypatch, p, nz, chunk, n
     orc.rw_step(Vo, 100.0, 2)
     for v in range(5 + ntr):
         assert rel_l2(V[v].cpu().numpy(), Vo[v]) <= TOL, f"V{v + 1} {rel_l2(V[v].cpu().numpy(), Vo[v]):.3e}"
+
+
+@pytest.mark.parametrize("nz", [44, 48, 60, 77])
+def test_taller_chunks(pkg, torch_cuda, nz):
+    """Both passes in chunks of 16 levels, which the context takes by itself on
+    grids that fill the chip, against 8 (44 and 60: a ragged last chunk)."""
+    torch, host = torch_cuda, pkg.host
+    print(f"taller chunks nz={nz}", flush=True)
+    disc = pkg.discretization.build(16, 4, nz, 512.0 * nz)
+    phys = pkg.discretization.Phys()
+    dev = host.device_setup(disc, phys, device="cuda")
+    FE, Metric, Global, Cache, JCache = dev
+    ctx = host.init_context(FE, Metric, phys, Global)
+    U0 = noisy_state(pkg, disc, 10)
+    out = []
+    for shape in ({}, {"chunk_levels": 8, "pass1_chunk_levels": 8}):
+        ctx.set_launch_shape(**shape)
+        F, T1 = tendency(torch, host, phys, dev, U0)
+        V = torch.as_tensor(U0, device="cuda").clone()
+        host.TimeStepper(V, 100.0, 2, FE, Metric, phys, Cache, JCache, Global)
+        torch.cuda.synchronize()
+        out.append((F, T1, V.cpu().numpy()))
+    for x, y in zip(*out):
+        for v in range(5):
+            assert rel_l2(x[v], y[v]) <= TOL, f"{v + 1} {rel_l2(x[v], y[v]):.3e}"
