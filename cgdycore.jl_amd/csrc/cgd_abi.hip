@@ -356,9 +356,9 @@ static int validate_desc(cgd_ctx *c, const cgd_desc *d, const std::string &who) 
 // concatenated: member m's elements and global nodes follow those of members
 // 0..m-1, so the state of the batch is one (Nz, sum NumG, 5) array.  Each
 // member is coloured on its own and colour k of the batch is the union of
-// the members' colour k, so one launch per colour covers every member and
-// each node accumulates its element contributions in the order a context of
-// its member alone uses: a member's results are bit-identical either way.
+// the members' colour k, so each node sums its element contributions in the
+// order a context of its member alone uses: a member's results are
+// bit-identical either way.
 static int ctx_build(cgd_ctx *c, const cgd_desc *ds, int nmem, hipStream_t st) {
   int r;
   for (int m = 0; m < nmem; ++m) {
@@ -744,14 +744,17 @@ static int ctx_build(cgd_ctx *c, const cgd_desc *ds, int nmem, hipStream_t st) {
   // than the chunks, so it is taken from three quarters of a wavefront on.
   c->col1 = c->cm && Nz >= 48 && Nz <= 64;
   // 16 levels per workgroup where that pads no more levels than 8 do (nz = 40,
-  // padded to 48: pass 1 15 %, pass 2 25 % slower) and leaves the chip a few
-  // rounds of workgroups: 128-byte pieces of the columns, and in pass 2 half
-  // the halo levels.  Pass 1, 32 grids of 32 levels: a step 1.5 % faster; where
-  // it can't take whole columns.  Pass 2 at nz = 64: 502 -> 487 us (ne = 30),
-  // 1900 -> 1856 (ne = 60); at nz = 32 no faster (the ensemble 0.4 % slower),
-  // so from 48 levels on.
-  const bool tall = c->N == 5 && !(((Nz + 7) / 8) & 1) && (size_t)NF * ((Nz + 15) / 16) >= 4096;
-  c->p16 = tall && c->cm && !c->col1;
+  // padded to 48: pass 1 15 %, pass 2 25 % slower): 128-byte pieces of the
+  // columns, and in pass 2 half the halo levels.
+  // Pass 1, where it can't take whole columns and the grid leaves the chip a few
+  // rounds of workgroups (the height changes no bit there): a step of 32 grids
+  // of 32 levels 1.5 % faster.
+  // Pass 2, whose rounding depends on the height, so that the rule must not
+  // depend on the grid's size (a grid in a batch and alone agree to the bit):
+  // nz = 64: 502 -> 487 us (ne = 30), 1900 -> 1856 (ne = 60), a step at ne <= 16
+  // within 1.5 % either way; at nz = 32 no faster, so from 48 levels on.
+  const bool tall = c->N == 5 && !(((Nz + 7) / 8) & 1);
+  c->p16 = tall && c->cm && !c->col1 && (size_t)NF * ((Nz + 15) / 16) >= 4096;
   c->r16 = tall && Nz >= 48 && c->reg && !c->smooth;
   c->ok = true;
   return CGD_OK;
@@ -1118,7 +1121,7 @@ static void launch_stage(cgd_ctx *c, int is, const RWStage<R> &rw, hipStream_t s
 // the passes), N = 4 or 5, and stage workgroups of the element tile's size.
 static bool persist_supported(const cgd_ctx *c, std::string *why) {
   const char *w = nullptr;
-  if (c->Nz > 64) w = "Nz > 64 (the composed step)";
+  if (c->Nz > 64) w = "Nz > 64";
   else if (c->N != 4 && c->N != 5) w = "N must be 4 or 5";
   else if (!c->cm) w = "the metric is not in the compact layout";
   else if (c->ntr > 0) w = "tracers";

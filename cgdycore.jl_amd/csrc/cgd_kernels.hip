@@ -15,11 +15,11 @@
 // tile[f][node][level]; vertical neighbours come from the neighbouring
 // lanes by DPP row shifts, with one global load at each chunk edge.
 //
-// DSS: the dynamics' element passes write each element's contributions to
-// an array of its own, X[c][e*NN + node][iz], all elements in one launch,
-// and the consumer of a field sums a node's copies in colour order (a
-// fixed order, no atomics).  The tracer kernels accumulate in place, one
-// launch per element colour (no two elements of a colour share a node).
+// DSS: the element passes write each element's contributions to an array of
+// its own, X[c][e*NN + node][iz], all elements in one launch, and the consumer
+// of a field sums a node's copies in colour order (a fixed order, no atomics).
+// The adjoint's kernels accumulate in place, one launch per element colour
+// (no two elements of a colour share a node).
 #include <hip/hip_runtime.h>
 
 #include <stdint.h>
@@ -46,7 +46,7 @@ struct KArgs {
   double DWm[CGD_NMAX * CGD_NMAX]; // DW[i*N + k]
   float Df[CGD_NMAX * CGD_NMAX], DWf[CGD_NMAX * CGD_NMAX];  // both in FP32 (mixed precision)
   const int *glob;                 // [e][NN]: 0-based node | bit 31 set on the node's first copy (colour order)
-  const int *clist;                // elements by colour (the tracer and adjoint kernels' launch order)
+  const int *clist;                // elements by colour (the adjoint kernels' launch order)
   const int *cpy;                  // [e][NN][cpw]: the node's copies e'*NN + node' in colour order, then -1
   const int *gcpy;                 // [NumG][cpw]: the same per global node
   int cpw;                         // a multiple of 2, at least 4
@@ -1261,7 +1261,7 @@ __device__ __forceinline__ double half_tree_sum(double x) {
 }
 
 // DivRhoTrUpwind3LimKernel! (HorLimiterKernel.jl:24-196) for all tracers,
-// one launch per colour, one thread per (node, level) of an element and
+// one thread per (node, level) of an element and
 // level chunk: the upwind vertical flux through both interfaces of the
 // layer (as k_tr2), then the limited horizontal transport: the predicted
 // rho*q and rho after dtau, the mixing ratio clipped to the bounds of the

@@ -48,14 +48,14 @@ enum {
  * gravity, the horizontal pressure gradient, the theta hyperviscosity (from
  * the FP64 state, with an FP64 cache), the column Jacobian and Schur solve
  * and the Rosenbrock stage arithmetic stay FP64, as does the state V.
- * The fV, Temp1 and k work buffers then hold FP32 data (the FP32 tendency
- * and an FP32 copy of the stage state in fV, the FP32 cache in Temp1 with
- * the FP64 theta cache at the offset of component 4 in doubles, the stage
+ * The fV and k work buffers then hold FP32 data (an FP32 copy of the stage
+ * state and, with physics hooks, the FP32 tendency in fV; the stage
  * increments, solved in FP64, stored in FP32 in k).  Tracers
  * (NumTr > 0, with HorLimit, the moist state and microphysics) stay FP64 in
- * this mode: their tendencies, caches and increments are components 6.. of
- * the same buffers, beyond the FP32 data.  The other entry points compute in
- * FP64 in either mode. */
+ * this mode: their increments (and tendencies, with microphysics) are
+ * components 6.. of the same buffers, beyond the FP32 data.  Columns of more
+ * than 64 levels step in FP64, and the other entry points compute in FP64 in
+ * either mode. */
 enum { CGD_FP64 = 0, CGD_MIXED = 1 };
 
 typedef struct {
@@ -145,9 +145,9 @@ int cgd_ctx_create(const cgd_desc *desc, cgd_ctx **ctx, void *stream);
  * hyperviscosity.  The batch's arrays concatenate the members along NumG:
  * U, V, F, ... are (Nz, sum_m NumG_m, 5) with member m's nodes at
  * NumG_0 + ... + NumG_{m-1} onward (and likewise k, AuxG, Temp1, the J
- * blocks).  Each member is coloured on its own and one launch per colour
- * covers all members, so a member's results are bit-identical to those of
- * a context built for it alone with the same launch shape.  No reference
+ * blocks).  Each member is coloured on its own and a node's contributions are
+ * summed in its member's colour order, so a member's results are bit-identical
+ * to those of a context built for it alone with the same launch shape.  No reference
  * counterpart (the reference steps one grid per process; batch variants of
  * the calls above, src/GPU/FcnGPU.jl:552 and src/Integration/RosenbrockSchur.jl:1). */
 int cgd_ctx_create_batch(const cgd_desc *members, int nmem, cgd_ctx **ctx, void *stream);
@@ -190,9 +190,9 @@ int cgd_schur(cgd_ctx *ctx, double *k, double *v, const double *JRhoW, const dou
  * reference's Cache.Vn, Cache.fV, Cache.k, Cache.AuxG, Cache.Temp1 and the
  * JCache blocks; all are caller owned.  V is advanced by one step exactly as
  * the reference's sequence of calls would; the work buffers are scratch.
- * For Nz <= 64 the stage kernel recomputes the frozen Jacobian from Vn
- * instead of storing it, so JRhoW..JRhoThW, tri, fV and k[:,:,:,3] are left
- * unwritten, AuxG[:,:,1] holds the pressure of the last stage state and
+ * The stage kernel recomputes the frozen Jacobian from Vn
+ * instead of storing it, so JRhoW..JRhoThW, tri, Temp1, k[:,:,:,3] and (without
+ * physics hooks) fV are left unwritten, AuxG[:,:,1] holds the pressure of the last stage state and
  * AuxG[:,:,2:4] are neither read nor written (AuxG[:,:,4] must be zero, as
  * for State = Dry). */
 typedef struct {
@@ -209,7 +209,8 @@ int cgd_rw_step(cgd_ctx *ctx, double *V, double dt, const cgd_rw_work *work, voi
 int cgd_rw_run(cgd_ctx *ctx, double *V, double dt, const cgd_rw_work *work, int nsteps, void *stream);
 
 /* The schedule and layout cgd_ctx_create chose: the number of element
- * colours (DSS launches per pass), the level chunk height of the element
+ * colours (the order in which a node's contributions are summed), the level
+ * chunk height of the element
  * kernels, and whether the metric is stored in the compact layout (every
  * component except the terrain row dXdxI[3,1:2,:] identical across levels,
  * so stored once per element node).  No reference counterpart. */
@@ -217,12 +218,15 @@ int cgd_ctx_info(const cgd_ctx *ctx, int *ncolor, int *chunk_levels, int *compac
 
 /* Launch shapes (no reference counterpart; the reference fixes its
  * workgroup shapes by NumberThreadGPU, src/DyCore/GlobalVariables.jl:240).
- * In cgd_set_launch_shape a field of 0 keeps the current value.  The
+ * In cgd_set_launch_shape a field of 0 keeps the current value.  Until a chunk
+ * height is set, the library may take whole columns or 16 levels instead of
+ * the 8 it reports, by a rule on N, Nz and the metric; a height that is set
+ * (8 included) is the one that runs.  The
  * workgroup sizes and pass1_items change no bit; the pass-2 chunk height
  * (chunk-interface w sums) and 32-lane columns (the compiler's fused
  * multiply-adds) change rounding only, within the FP64 parity bound.
  * persistent = 1 runs each RW stage of cgd_rw_step as ONE launch (both
- * tendency passes over every colour, then the column stage) whose
+ * tendency passes, then the column stage) whose
  * workgroups stay resident and meet at grid-wide barriers where the
  * separate launches have kernel boundaries; the results are bit-identical
  * to the separate launches.  It takes the dry dynamics with the compact

@@ -247,8 +247,8 @@ def test_tracer_passes(pkg, oracle_mod, torch_cuda, monkeypatch, p, nz, chunk, n
 
 @pytest.mark.parametrize("nz", [44, 48, 60, 77])
 def test_taller_chunks(pkg, torch_cuda, nz):
-    """Both passes in chunks of 16 levels, which the context takes by itself on
-    grids that fill the chip, against 8 (44 and 60: a ragged last chunk)."""
+    """Both passes in chunks of 16 levels, which the context takes by itself,
+    against 8 (44 and 60: a ragged last chunk)."""
     torch, host = torch_cuda, pkg.host
     print(f"taller chunks nz={nz}", flush=True)
     disc = pkg.discretization.build(16, 4, nz, 512.0 * nz)
@@ -268,3 +268,5 @@ def test_taller_chunks(pkg, torch_cuda, nz):
     for x, y in zip(*out):
         for v in range(5):
             assert rel_l2(x[v], y[v]) <= TOL, f"{v + 1} {rel_l2(x[v], y[v]):.3e}"
+    if nz < 48 or nz > 64:  # no columns: pass 1's chunk height changes no bit
+        assert np.array_equal(out[0][1], out[1][1])
