@@ -1504,6 +1504,7 @@ __device__ __forceinline__ double copies_sum(const KArgs &a, const double *__res
   const unsigned g = ip / (unsigned)a.Nz, iz = ip - g * (unsigned)a.Nz;
   const int *cp = a.gcpy + (size_t)g * a.cpw;
   const int c0 = cp[0], c1 = cp[1];
+  if (c0 < 0) return 0.0;  // a node of no element
   double v = E[(size_t)c0 * a.Nz + iz];
   if (c1 >= 0) {
     double y = E[(size_t)c1 * a.Nz + iz];
