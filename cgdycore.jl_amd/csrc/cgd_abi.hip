@@ -1057,6 +1057,12 @@ extern "C" int cgd_set_dtau(cgd_ctx *c, double dtau) {
   return CGD_OK;
 }
 
+// whether the J blocks take 16-byte accesses
+static bool aligned16(const double *a, const double *b, const double *d, const double *e) {
+  return ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b) | reinterpret_cast<uintptr_t>(d) |
+           reinterpret_cast<uintptr_t>(e)) & 15) == 0;
+}
+
 extern "C" int cgd_jac(cgd_ctx *c, double *JRhoW, double *JWRho, double *JWRhoTh, double *JRhoThW, const double *U,
                        const double *AuxG, void *stream) {
   int r = check(c);
@@ -1064,7 +1070,8 @@ extern "C" int cgd_jac(cgd_ctx *c, double *JRhoW, double *JWRho, double *JWRhoTh
   if (!JRhoW || !JWRho || !JWRhoTh || !JRhoThW || !U || !AuxG) return fail(c, CGD_ERR_ARG, "cgd_jac: null array");
   const size_t n = (size_t)c->NumG * (c->Nz - 1);
   const size_t ng = (size_t)c->NumG * c->Nz;
-  hipLaunchKernelGGL(k_jac, dim3(grid_for(n, 256)), dim3(256), 0, S(stream), c->ka, U, AuxG + 3 * ng, c->dz,
+  const auto kernel = aligned16(JRhoW, JWRho, JWRhoTh, JRhoThW) ? k_jac<true> : k_jac<false>;
+  hipLaunchKernelGGL(kernel, dim3(grid_for(n, 256)), dim3(256), 0, S(stream), c->ka, U, AuxG + 3 * ng, c->dz,
                      JRhoW, JWRho, JWRhoTh, JRhoThW);
   HIPCHK(c, hipGetLastError());
   return CGD_OK;
@@ -1087,8 +1094,9 @@ extern "C" int cgd_schur(cgd_ctx *c, double *k, double *v, const double *JRhoW, 
   prof_begin(c, st, 2);
   const double invfac = 1.0 / fac, invfac2 = invfac / fac;
   if (c->Nz <= 64)
-    hipLaunchKernelGGL(k_schur_col, dim3((c->NumG + 3) / 4), dim3(256), 0, st, c->ka, k, v, JRhoW, JWRho, JWRhoTh,
-                       JRhoThW, tri, fac, invfac2, comp_tri, c->thomas);
+    hipLaunchKernelGGL((aligned16(JRhoW, JWRho, JWRhoTh, JRhoThW) ? k_schur_col<true> : k_schur_col<false>),
+                       dim3((c->NumG + 3) / 4), dim3(256), 0, st, c->ka, k, v, JRhoW, JWRho, JWRhoTh, JRhoThW, tri,
+                       fac, invfac2, comp_tri, c->thomas);
   else
     launch_tall(c->Nz, [&](auto w) {
       constexpr int W = decltype(w)::value;

@@ -270,3 +270,33 @@ def test_taller_chunks(pkg, torch_cuda, nz):
             assert rel_l2(x[v], y[v]) <= TOL, f"{v + 1} {rel_l2(x[v], y[v]):.3e}"
     if nz < 48 or nz > 64:  # no columns: pass 1's chunk height changes no bit
         assert np.array_equal(out[0][1], out[1][1])
+
+
+@pytest.mark.parametrize("nz", [3, 33, 64])
+def test_column_calls_alignment(pkg, torch_cuda, nz):
+    """The Jacobian and the column solve on J blocks that take 16-byte
+    accesses and on ones that do not: the same bits."""
+    torch, host = torch_cuda, pkg.host
+    print(f"column alignment nz={nz}", flush=True)
+    disc = pkg.discretization.build(2, 3, nz, 30000.0)
+    phys = pkg.discretization.Phys()
+    FE, Metric, Global, Cache, JCache = host.device_setup(disc, phys, device="cuda")
+    U = torch.as_tensor(pkg.state.jet_state(disc, seed=11), device="cuda")
+    eq = host.CompressibleShallow()
+    names = ("JRhoW", "JWRho", "JWRhoTh", "JRhoThW")
+    out = []
+    for shift in (0, 1):
+        for name in names:
+            J = getattr(JCache, name)
+            view = torch.zeros(J.numel() + 2, dtype=J.dtype, device="cuda")[shift:shift + J.numel()].view(J.shape)
+            assert view.data_ptr() % 16 == 8 * shift
+            setattr(JCache, name, view)
+        host.FcnPrepareGPU(U, FE, Metric, phys, Cache, None, Global, None, eq)
+        host.JacSchurGPU(JCache, U, FE, Metric, phys, Cache, Global, None, eq)
+        v = torch.as_tensor(np.random.default_rng(11).standard_normal(tuple(U.shape)), device="cuda")
+        k = torch.zeros_like(v)
+        JCache.CompTri = True
+        host.SchurSolveGPU(k, v, JCache, 150.0, Cache, Global)
+        torch.cuda.synchronize()
+        out.append([getattr(JCache, n).cpu() for n in names] + [JCache.tri.cpu(), k.cpu(), v.cpu()])
+    assert all(torch.equal(x, y) for x, y in zip(*out))
