@@ -389,6 +389,16 @@ template <typename R, typename... D> __device__ __forceinline__ void pin(R &x, D
   pin(y...);
 }
 
+// Between LDS stores of some lanes of a wavefront and their first reads by other
+// lanes of the same one: the hardware keeps a wavefront's LDS accesses in
+// order, and this keeps the compiler from moving a read above a store that the
+// reading lane does not make.  No instruction, LDS only.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 // ------------------------------------------------------------------------
 // Pass 1: HyperViscKernel! (src/GPU/ViscKernel.jl:1-84).
 // Grid: one workgroup per ITEMS consecutive work items, an
