@@ -17,8 +17,12 @@ struct cgd_ctx {
   cgd_desc desc{};
   KArgs ka{};
   int N = 0, NN = 0, Nz = 0, NF = 0, NumG = 0;
-  int nzt = 0, nchunk = 0, block = 0;     // pass 2 (and the chunk-interface side sums)
-  int nzt1 = 0, nchunk1 = 0, block1 = 0;  // pass 1
+  // levels per workgroup of pass 2 and of pass 1 (64: whole columns, k_fcn1c)
+  // as cgd_get_launch_shape reports them for separate launches, and the ones
+  // the context chose: nzt is then 16 levels in FP64 where r16 (k_fcn2r) is set
+  int nzt = 0, nzt1 = 0;
+  int base_nzt = 8, rule_nzt = 0, rule_nzt1 = 0;
+  int r16 = 0;
   int thomas = 0;  // column solve: 0 = cyclic reduction, 1 = serial Thomas (CGD_THOMAS=1)
   int ntr = 0;     // tracers (components 5..4+ntr of the state arrays, 0-based)
   int ncolor = 0;
@@ -63,9 +67,6 @@ struct cgd_ctx {
   // column launch shape of the fused stage kernel: lanes per column (64,
   // or 32 for two columns per wavefront when Nz <= 32) and workgroup size
   int colw = 64, colblock = 256;
-  int col1 = 0;    // pass 1 over whole columns (k_fcn1c), until its chunk height is set
-  // k_fcn1 and k_fcn2r in chunks of 16 levels, until their chunk heights are set
-  int p16 = 0, r16 = 0;
   int items1 = 1;  // pass-1 work items (element, level chunk) per workgroup: 1 or 2
   // one persistent launch per RW stage (k_stage_persist): on/off, its grid
   // (workgroups resident at once), the grid barrier's state and wait bound
@@ -98,27 +99,37 @@ template <typename R> static size_t lds_fcn1(const cgd_ctx *c, int nzt1) {
   if (std::is_same<R, double>::value) return r;
   return (r + 7) / 8 * 8 + sizeof(double) * (2 * c->NN + 3 * c->NN * nzt1);
 }
-template <typename R> static size_t lds_fcn2(const cgd_ctx *c) {
+template <typename R> static size_t lds_fcn2(const cgd_ctx *c, int nzt) {
   // + the horizontal metric: 12 values per node (compact layout), 10 per point
   // (full layout, FP64)
-  const size_t hm = c->cm || !std::is_same<R, double>::value ? 12 * c->NN : 10 * c->NN * c->nzt;
-  const size_t r = sizeof(R) * (2 * c->NN + 14 * c->NN * c->nzt + hm);
-  const size_t base = sizeof(double) * (c->NN + c->NN * c->nzt);
+  const size_t hm = c->cm || !std::is_same<R, double>::value ? 12 * c->NN : 10 * c->NN * nzt;
+  const size_t r = sizeof(R) * (2 * c->NN + 14 * c->NN * nzt + hm);
+  const size_t base = sizeof(double) * (c->NN + c->NN * nzt);
   if (std::is_same<R, double>::value) return base + r;
-  return base + (r + 7) / 8 * 8 + sizeof(double) * (c->NN + 3 * c->NN * c->nzt);
+  return base + (r + 7) / 8 * 8 + sizeof(double) * (c->NN + 3 * c->NN * nzt);
 }
 
+// pass 1 can take whole columns
+static bool columns_ok(const cgd_ctx *c) { return c->cm && c->Nz <= 64; }
 // k_fcn1c: three tiles of whole columns, one of them FP64
 static size_t lds_fcn1c(const cgd_ctx *c, size_t r) { return (size_t)c->NN * 64 * (sizeof(double) + 2 * r); }
 
-// the chunk heights of pass 1 and, for the tendency in type R, of pass 2
-static int cache_nzt(const cgd_ctx *c) { return c->p16 && !c->persistent ? 16 : c->nzt1; }
+// The heights that run.  A persistent launch has chunks of 8 levels.  A height
+// that is the context's own choice stands for all of that choice: in pass 2
+// the FP64 and the FP32 tendency's, each by its rule, and base_nzt for the
+// tracers' kernels; any other is the height of all of them.
+static int cache_nzt(const cgd_ctx *c) { return c->persistent ? 8 : c->nzt1; }
 template <typename R> static int tend_nzt(const cgd_ctx *c) {
-  return std::is_same<R, double>::value && c->r16 && !c->persistent ? 16 : c->nzt;
+  if (c->persistent) return 8;
+  if (c->nzt != c->rule_nzt) return c->nzt;
+  return std::is_same<R, double>::value && c->r16 ? 16 : c->base_nzt;
 }
-template <typename R> static int tend_nchunk(const cgd_ctx *c) {
-  return (c->Nz + tend_nzt<R>(c) - 1) / tend_nzt<R>(c);
-}
+static int tr_cache_nzt(const cgd_ctx *c) { return c->nzt1 == c->rule_nzt1 || c->nzt1 == 64 ? c->base_nzt : c->nzt1; }
+static int tr_tend_nzt(const cgd_ctx *c) { return c->nzt == c->rule_nzt ? c->base_nzt : c->nzt; }
+static int nchunks(const cgd_ctx *c, int nzt) { return (c->Nz + nzt - 1) / nzt; }
+// threads of an element tile of nzt levels
+static int tile_block(const cgd_ctx *c, int nzt) { return (c->NN * nzt + 63) / 64 * 64; }
+
 // k_fcn2r: D, DW, 12 tiles, four tiles with the level below, its sums, the
 // horizontal metric and 1/(2 M)
 static size_t lds_fcn2r(const cgd_ctx *c, int nzt) {
@@ -304,7 +315,7 @@ extern "C" int cgd_ctx_info(const cgd_ctx *c, int *ncolor, int *chunk_levels, in
   if (!c) return CGD_ERR_ARG;
   if (!c->ok) return CGD_ERR_STATE;
   if (ncolor) *ncolor = c->ncolor;
-  if (chunk_levels) *chunk_levels = c->nzt;
+  if (chunk_levels) *chunk_levels = c->persistent ? 8 : c->nzt;
   if (compact_metric) *compact_metric = c->cm;
   return CGD_OK;
 }
@@ -423,16 +434,13 @@ static int ctx_build(cgd_ctx *c, const cgd_desc *ds, int nmem, hipStream_t st) {
   // wavefronts better but straddle cache lines); CGD_NZT=16 overrides, and
   // cgd_set_launch_shape / cgd_autotune change it later.
   {
-    int nzt = 8;
+    c->base_nzt = 8;
     if (const char *ev = getenv("CGD_NZT")) {
       const int o = atoi(ev);
-      if (o == 16 && c->N == 5) nzt = o;
+      if (o == 16 && c->N == 5) c->base_nzt = o;
     }
-    c->nzt = c->nzt1 = nzt;
-    c->nchunk = c->nchunk1 = (Nz + nzt - 1) / nzt;
     if (const char *ev = getenv("CGD_THOMAS")) c->thomas = atoi(ev) != 0;
   }
-  c->block = c->block1 = ((NN * c->nzt + 63) / 64) * 64;
   c->colw = 64;
   c->colblock = 256;
   c->items1 = 1;
@@ -688,7 +696,6 @@ static int ctx_build(cgd_ctx *c, const cgd_desc *ds, int nmem, hipStream_t st) {
   KArgs &a = c->ka;
   a.Nz = Nz;
   a.NumG = NumG;
-  a.nzt = c->nzt;
   a.Grav = d->Grav;
   a.Omega = d->Omega;
   a.Rd = d->Rd;
@@ -742,7 +749,7 @@ static int ctx_build(cgd_ctx *c, const cgd_desc *ds, int nmem, hipStream_t st) {
   // Pass 1 over whole columns has a lane per level: at Nz = 64 it takes 127 us
   // instead of 190 (ne = 30), at Nz = 40 the idle lanes make it 1 % slower
   // than the chunks, so it is taken from three quarters of a wavefront on.
-  c->col1 = c->cm && Nz >= 48 && Nz <= 64;
+  const bool col1 = columns_ok(c) && Nz >= 48;
   // 16 levels per workgroup where that pads no more levels than 8 do (nz = 40,
   // padded to 48: pass 1 15 %, pass 2 25 % slower): 128-byte pieces of the
   // columns, and in pass 2 half the halo levels.
@@ -754,8 +761,10 @@ static int ctx_build(cgd_ctx *c, const cgd_desc *ds, int nmem, hipStream_t st) {
   // nz = 64: 502 -> 487 us (ne = 30), 1900 -> 1856 (ne = 60), a step at ne <= 16
   // within 1.5 % either way; at nz = 32 no faster, so from 48 levels on.
   const bool tall = c->N == 5 && !(((Nz + 7) / 8) & 1);
-  c->p16 = tall && c->cm && !c->col1 && (size_t)NF * ((Nz + 15) / 16) >= 4096;
+  const bool p16 = tall && c->cm && !col1 && (size_t)NF * ((Nz + 15) / 16) >= 4096;
   c->r16 = tall && Nz >= 48 && c->reg && !c->smooth;
+  c->nzt = c->rule_nzt = c->r16 && !(c->mixed && Nz <= 64) ? 16 : c->base_nzt;  // that of the steps' tendency
+  c->nzt1 = c->rule_nzt1 = col1 ? 64 : p16 ? 16 : c->base_nzt;
   c->ok = true;
   return CGD_OK;
 }
@@ -872,7 +881,7 @@ extern "C" int cgd_profile_read(cgd_ctx *c, int which, double *total_ms, long lo
 template <int N, int NZT, bool CM, typename R>
 static void fcn1_t(cgd_ctx *c, hipStream_t st, const R *UR, R *E, const double *U64, double *Eth) {
   const int nchunk = (c->Nz + NZT - 1) / NZT, nitems = c->NF * nchunk;
-  const dim3 b((N * N * NZT + 63) / 64 * 64);
+  const dim3 b(tile_block(c, NZT));
   const size_t lds = lds_fcn1<R>(c, NZT);
   if (c->items1 == 2)
     hipLaunchKernelGGL((k_fcn1<N, NZT, CM, R, 2>), dim3((nitems + 1) / 2), b, lds, st, c->ka, nchunk, nitems, UR, E,
@@ -881,25 +890,25 @@ static void fcn1_t(cgd_ctx *c, hipStream_t st, const R *UR, R *E, const double *
     hipLaunchKernelGGL((k_fcn1<N, NZT, CM, R, 1>), dim3(nitems), b, lds, st, c->ka, nchunk, nitems, UR, E, U64, Eth);
 }
 template <int N, int NZT, bool CM, typename R>
-static void fcn2_t(cgd_ctx *c, dim3 g, hipStream_t st, const double *U, const R *UR, const R *E1, const double *P,
-                   R *E2, const double *E1th, double *Cout) {
+static void fcn2_t(cgd_ctx *c, hipStream_t st, const double *U, const R *UR, const R *E1, const double *P, R *E2,
+                   const double *E1th, double *Cout) {
+  const int nchunk = nchunks(c, NZT);
+  const dim3 g(c->NF * nchunk), b(tile_block(c, NZT));
   if constexpr (std::is_same<R, double>::value && CM) {
     if (c->reg && !c->smooth) {
-      hipLaunchKernelGGL((k_fcn2r<N, NZT>), g, dim3((N * N * NZT + 63) / 64 * 64), lds_fcn2r(c, NZT), st, c->ka,
-                         tend_nchunk<R>(c), U, E1, P, E2,
-                         c->d_f4x, Cout);
+      hipLaunchKernelGGL((k_fcn2r<N, NZT>), g, b, lds_fcn2r(c, NZT), st, c->ka, nchunk, U, E1, P, E2, c->d_f4x, Cout);
       return;
     }
   }
+  const size_t lds = lds_fcn2<R>(c, NZT);
+  R *const F4x = reinterpret_cast<R *>(c->d_f4x);
   if constexpr (std::is_same<R, double>::value) {
     if (c->smooth) {  // kink-smoothed upwind flux (FP64 only)
-      hipLaunchKernelGGL((k_fcn2<N, NZT, CM, R, true>), g, dim3(c->block), lds_fcn2<R>(c), st, c->ka, c->nchunk, U,
-                         UR, E1, P, E2, reinterpret_cast<R *>(c->d_f4x), E1th, Cout);
+      hipLaunchKernelGGL((k_fcn2<N, NZT, CM, R, true>), g, b, lds, st, c->ka, nchunk, U, UR, E1, P, E2, F4x, E1th, Cout);
       return;
     }
   }
-  hipLaunchKernelGGL((k_fcn2<N, NZT, CM, R, false>), g, dim3(c->block), lds_fcn2<R>(c), st, c->ka, c->nchunk, U,
-                     UR, E1, P, E2, reinterpret_cast<R *>(c->d_f4x), E1th, Cout);
+  hipLaunchKernelGGL((k_fcn2<N, NZT, CM, R, false>), g, b, lds, st, c->ka, nchunk, U, UR, E1, P, E2, F4x, E1th, Cout);
 }
 #define CGD_DISPATCH(FN, R, NZTV, ...)                             \
   do {                                                             \
@@ -916,28 +925,31 @@ static void fcn2_t(cgd_ctx *c, dim3 g, hipStream_t st, const double *U, const R 
   } while (0)
 // the tracers' element copies: components 5.. of d_e1 and d_e2, FP64 in both modes
 template <int N, int NZT, bool CM, typename R>
-static void tr1_t(cgd_ctx *c, int nitems, hipStream_t st, const double *U) {
+static void tr1_t(cgd_ctx *c, hipStream_t st, const double *U) {
   const size_t lds = sizeof(double) * (2 * c->NN + 3 * c->NN * NZT);
-  hipLaunchKernelGGL((k_tr1<N, NZT, CM>), dim3(nitems), dim3(c->block1), lds, st, c->ka, c->nchunk1, c->ntr, U,
-                     c->d_e1 + 5 * c->ka.ecs);
+  const int nchunk = nchunks(c, NZT);
+  hipLaunchKernelGGL((k_tr1<N, NZT, CM>), dim3(c->NF * nchunk), dim3(tile_block(c, NZT)), lds, st, c->ka, nchunk,
+                     c->ntr, U, c->d_e1 + 5 * c->ka.ecs);
 }
 template <int N, int NZT, bool CM, typename R>
-static void tr2_t(cgd_ctx *c, int nitems, hipStream_t st, const double *U, double *Cout) {
+static void tr2_t(cgd_ctx *c, hipStream_t st, const double *U, double *Cout) {
   const size_t lds = sizeof(double) * (2 * c->NN + 10 * c->NN * NZT);
-  hipLaunchKernelGGL((k_tr2<N, NZT, CM>), dim3(nitems), dim3(c->block), lds, st, c->ka, c->nchunk, c->ntr, U,
-                     c->d_e1 + 5 * c->ka.ecs, Cout, c->d_e2 + 5 * c->ka.ecs);
+  const int nchunk = nchunks(c, NZT);
+  hipLaunchKernelGGL((k_tr2<N, NZT, CM>), dim3(c->NF * nchunk), dim3(tile_block(c, NZT)), lds, st, c->ka, nchunk,
+                     c->ntr, U, c->d_e1 + 5 * c->ka.ecs, Cout, c->d_e2 + 5 * c->ka.ecs);
 }
 
 template <int N, int NZT, bool CM, typename R>
-static void tr2lim_t(cgd_ctx *c, int nitems, hipStream_t st, const double *U) {
+static void tr2lim_t(cgd_ctx *c, hipStream_t st, const double *U) {
   const size_t lds = sizeof(double) * (c->NN + 7 * c->NN * NZT);
-  hipLaunchKernelGGL((k_tr2_lim<N, NZT, CM>), dim3(nitems), dim3(c->block), lds, st, c->ka, c->nchunk, c->ntr, U,
-                     c->d_stencil, c->NF, c->d_qmin, c->d_qmax, c->dtau, c->d_e2 + 5 * c->ka.ecs);
+  const int nchunk = nchunks(c, NZT);
+  hipLaunchKernelGGL((k_tr2_lim<N, NZT, CM>), dim3(c->NF * nchunk), dim3(tile_block(c, NZT)), lds, st, c->ka, nchunk,
+                     c->ntr, U, c->d_stencil, c->NF, c->d_qmin, c->d_qmax, c->dtau, c->d_e2 + 5 * c->ka.ecs);
 }
 
 template <typename R>
 static void launch_fcn1(cgd_ctx *c, hipStream_t st, const R *UR, R *E, const double *U64, double *Eth) {
-  if (c->col1) {
+  if (cache_nzt(c) == 64) {
     const size_t lds = lds_fcn1c(c, sizeof(R));
     if (c->N == 5) hipLaunchKernelGGL((k_fcn1c<5, R>), dim3(c->NF), dim3(320), lds, st, c->ka, UR, E, U64, Eth);
     else hipLaunchKernelGGL((k_fcn1c<4, R>), dim3(c->NF), dim3(256), lds, st, c->ka, UR, E, U64, Eth);
@@ -946,9 +958,9 @@ static void launch_fcn1(cgd_ctx *c, hipStream_t st, const R *UR, R *E, const dou
   CGD_DISPATCH(fcn1_t, R, cache_nzt(c), st, UR, E, U64, Eth);
 }
 template <typename R>
-static void launch_fcn2(cgd_ctx *c, dim3 g, hipStream_t st, const double *U, const R *UR, const R *E1,
-                        const double *P, R *E2, const double *E1th, double *Cout) {
-  CGD_DISPATCH(fcn2_t, R, tend_nzt<R>(c), g, st, U, UR, E1, P, E2, E1th, Cout);
+static void launch_fcn2(cgd_ctx *c, hipStream_t st, const double *U, const R *UR, const R *E1, const double *P, R *E2,
+                        const double *E1th, double *Cout) {
+  CGD_DISPATCH(fcn2_t, R, tend_nzt<R>(c), st, U, UR, E1, P, E2, E1th, Cout);
 }
 
 extern "C" int cgd_prepare(cgd_ctx *c, const double *U, double *AuxG, void *stream) {
@@ -992,14 +1004,14 @@ static int run_fcn(cgd_ctx *c, R *F, const double *U, const R *UR, R *Temp1, con
   double *const Fd = reinterpret_cast<double *>(F);
   double *const T1d = reinterpret_cast<double *>(Temp1);
   if (c->ntr > 0 && !c->horlimit) {  // HorLimit: no tracer hyperviscosity (FcnGPU.jl:747-751)
-    CGD_DISPATCH(tr1_t, double, c->nzt1, c->NF * c->nchunk1, st, U);
+    CGD_DISPATCH(tr1_t, double, tr_cache_nzt(c), st, U);
     HIPCHK(c, hipGetLastError());
     ++launches;
   }
   if ((r = prof_end(c, st, 0, launches))) return r;
   prof_begin(c, st, 1);
   launches = 0;
-  launch_fcn2<R>(c, dim3(c->NF * tend_nchunk<R>(c)), st, U, UR, E1, AuxG, E2, E1th, want_f ? T1d : nullptr);
+  launch_fcn2<R>(c, st, U, UR, E1, AuxG, E2, E1th, want_f ? T1d : nullptr);
   HIPCHK(c, hipGetLastError());
   ++launches;
   {
@@ -1011,11 +1023,11 @@ static int run_fcn(cgd_ctx *c, R *F, const double *U, const R *UR, R *Temp1, con
                          c->d_qmin, c->d_qmax);
       HIPCHK(c, hipGetLastError());
       ++launches;
-      CGD_DISPATCH(tr2lim_t, double, c->nzt, c->NF * c->nchunk, st, U);
+      CGD_DISPATCH(tr2lim_t, double, tr_tend_nzt(c), st, U);
       HIPCHK(c, hipGetLastError());
       ++launches;
     } else if (c->ntr > 0) {
-      CGD_DISPATCH(tr2_t, double, c->nzt, c->NF * c->nchunk, st, U, want_f ? T1d : nullptr);
+      CGD_DISPATCH(tr2_t, double, tr_tend_nzt(c), st, U, want_f ? T1d : nullptr);
       HIPCHK(c, hipGetLastError());
       ++launches;
     }
@@ -1032,10 +1044,10 @@ static int run_fcn(cgd_ctx *c, R *F, const double *U, const R *UR, R *Temp1, con
     const R *F4x = reinterpret_cast<const R *>(c->d_f4x);
     if (has_hooks(c))
       hipLaunchKernelGGL((k_dss<R, true>), g, dim3(256), 0, st, c->ka, c->hooks, U, AuxG, E2, F4x, F, Fd,
-                         tend_nchunk<R>(c), tend_nzt<R>(c));
+                         nchunks(c, tend_nzt<R>(c)), tend_nzt<R>(c));
     else
       hipLaunchKernelGGL((k_dss<R, false>), g, dim3(256), 0, st, c->ka, c->hooks, U, AuxG, E2, F4x, F, Fd,
-                         tend_nchunk<R>(c), tend_nzt<R>(c));
+                         nchunks(c, tend_nzt<R>(c)), tend_nzt<R>(c));
     HIPCHK(c, hipGetLastError());
     ++launches;
   }
@@ -1145,7 +1157,7 @@ template <int N, typename R, int W> static const void *persist_fn(const cgd_ctx 
   return reinterpret_cast<const void *>(&k_stage_persist<N, true, R, W, false>);
 }
 template <typename R> static size_t lds_persist(const cgd_ctx *c) {
-  return std::max(lds_fcn1<R>(c, c->nzt1), std::is_same<R, double>::value && c->reg ? lds_fcn2r(c, c->nzt) : lds_fcn2<R>(c));
+  return std::max(lds_fcn1<R>(c, 8), std::is_same<R, double>::value && c->reg ? lds_fcn2r(c, 8) : lds_fcn2<R>(c, 8));
 }
 
 // The grid: every workgroup resident at once (the kernel's occupancy per CU
@@ -1154,12 +1166,12 @@ template <typename R, int W> static int persist_grid(cgd_ctx *c, int &G) {
   const void *fn = c->N == 5 ? persist_fn<5, R, W>(c) : persist_fn<4, R, W>(c);
   const size_t lds = lds_persist<R>(c);
   int per_cu = 0, dev = 0, ncu = 0;
-  HIPCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, c->block, lds));
+  HIPCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, tile_block(c, 8), lds));
   HIPCHK(c, hipGetDevice(&dev));
   HIPCHK(c, hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
   if (per_cu < 1) return fail(c, CGD_ERR_UNSUPPORTED, "persistent stage launch: the kernel does not fit a CU");
   int need = (c->NumG + c->colblock / c->colw - 1) / (c->colblock / c->colw);
-  need = std::max(need, c->NF * std::max(c->nchunk, c->nchunk1));
+  need = std::max(need, c->NF * nchunks(c, 8));
   G = std::max(1, std::min(per_cu * ncu, need));
   return CGD_OK;
 }
@@ -1171,8 +1183,7 @@ static int launch_persist(cgd_ctx *c, int is, const RWStage<R> &rw, const double
   if (!c->pgrid && (r = persist_grid<R, W>(c, c->pgrid))) return r;
   StagePersist<R> p{};
   p.nf = c->NF;
-  p.nchunk1 = c->nchunk1;
-  p.nchunk = c->nchunk;
+  p.nchunk1 = p.nchunk = nchunks(c, 8);
   p.UR = UR;
   p.T1 = reinterpret_cast<R *>(c->d_e1);
   p.U = U;
@@ -1187,7 +1198,7 @@ static int launch_persist(cgd_ctx *c, int is, const RWStage<R> &rw, const double
   const void *fn = c->N == 5 ? persist_fn<5, R, W>(c) : persist_fn<4, R, W>(c);
   RWStage<R> rws = rw;
   void *args[] = {&c->ka, &p, &rws, &is};
-  HIPCHK(c, hipLaunchKernel(fn, dim3(c->pgrid), dim3(c->block), args, lds, st));
+  HIPCHK(c, hipLaunchKernel(fn, dim3(c->pgrid), dim3(tile_block(c, 8)), args, lds, st));
   HIPCHK(c, hipGetLastError());
   return CGD_OK;
 }
@@ -1243,7 +1254,7 @@ static int rw_step_fused(cgd_ctx *c, double *V, double dt, const cgd_rw_work *w,
     rw.k = is < 2 ? kR[is] : nullptr;  // k_3 is consumed in registers
     rw.P = (is < 2 || more) ? w->AuxG : nullptr;
     rw.F4x = reinterpret_cast<const R *>(c->d_f4x);
-    rw.nchunk = tend_nchunk<R>(c);
+    rw.nchunk = nchunks(c, tend_nzt<R>(c));
     rw.nzt = tend_nzt<R>(c);
     rw.fac = dt * gamma;
     rw.invfac = 1.0 / rw.fac;
@@ -1381,21 +1392,22 @@ static void graph_free(cgd_ctx *c) {
 // element tile's size (256 threads for N = 5, 128 for N = 4).
 static bool shape_ok(const cgd_ctx *c, const cgd_launch_shape &sh) {
   auto chunk_ok = [&](int z) { return z == 8 || (z == 16 && c->N == 5); };
-  if (!chunk_ok(sh.chunk_levels) || !chunk_ok(sh.pass1_chunk_levels)) return false;
+  if (!chunk_ok(sh.chunk_levels)) return false;
+  if (!chunk_ok(sh.pass1_chunk_levels) && !(sh.pass1_chunk_levels == 64 && columns_ok(c))) return false;
   if (!(sh.pass1_items == 1 || sh.pass1_items == 2)) return false;
   if (!(sh.col_lanes == 64 || (sh.col_lanes == 32 && c->Nz <= 32 && !c->thomas))) return false;
   if (!(sh.col_block >= 64 && sh.col_block <= 256 && sh.col_block % 64 == 0)) return false;
   if (sh.persistent != 1 && sh.persistent != -1) return false;
   if (sh.persistent == 1)
     return persist_supported(c, nullptr) && sh.chunk_levels == 8 && sh.pass1_chunk_levels == 8 &&
-           sh.pass1_items == 1 && sh.col_block == (c->NN * 8 + 63) / 64 * 64;
+           sh.pass1_items == 1 && sh.col_block == tile_block(c, 8);
   return true;
 }
 
 static cgd_launch_shape current_shape(const cgd_ctx *c) {
   cgd_launch_shape sh;
-  sh.chunk_levels = c->nzt;
-  sh.pass1_chunk_levels = c->nzt1;
+  sh.chunk_levels = c->persistent ? 8 : c->nzt;
+  sh.pass1_chunk_levels = c->persistent ? 8 : c->nzt1;
   sh.pass1_items = c->items1;
   sh.col_lanes = c->colw;
   sh.col_block = c->colblock;
@@ -1405,12 +1417,7 @@ static cgd_launch_shape current_shape(const cgd_ctx *c) {
 
 static void apply_shape(cgd_ctx *c, const cgd_launch_shape &sh) {
   c->nzt = sh.chunk_levels;
-  c->nchunk = (c->Nz + c->nzt - 1) / c->nzt;
-  c->block = ((c->NN * c->nzt + 63) / 64) * 64;
-  c->ka.nzt = c->nzt;
   c->nzt1 = sh.pass1_chunk_levels;
-  c->nchunk1 = (c->Nz + c->nzt1 - 1) / c->nzt1;
-  c->block1 = ((c->NN * c->nzt1 + 63) / 64) * 64;
   c->items1 = sh.pass1_items;
   c->colw = sh.col_lanes;
   c->colblock = sh.col_block;
@@ -1423,6 +1430,11 @@ extern "C" int cgd_set_launch_shape(cgd_ctx *c, const cgd_launch_shape *shape) {
   if (r) return r;
   if (!shape) return fail(c, CGD_ERR_ARG, "cgd_set_launch_shape: null shape");
   cgd_launch_shape sh = current_shape(c);
+  // a persistent launch takes 8 levels in place of the heights the context
+  // chose, which stand again when it is turned off, but not of set ones
+  const bool pers = shape->persistent ? shape->persistent == 1 : c->persistent;
+  sh.chunk_levels = pers && c->nzt == c->rule_nzt ? 8 : c->nzt;
+  sh.pass1_chunk_levels = pers && c->nzt1 == c->rule_nzt1 ? 8 : c->nzt1;
   if (shape->chunk_levels) sh.chunk_levels = shape->chunk_levels;
   if (shape->pass1_chunk_levels) sh.pass1_chunk_levels = shape->pass1_chunk_levels;
   if (shape->pass1_items) sh.pass1_items = shape->pass1_items;
@@ -1434,13 +1446,15 @@ extern "C" int cgd_set_launch_shape(cgd_ctx *c, const cgd_launch_shape *shape) {
     return fail(c, CGD_ERR_UNSUPPORTED, "persistent stage launch: not for " + why);
   if (!shape_ok(c, sh))
     return fail(c, CGD_ERR_ARG,
-                "launch shape: chunk heights must be 8 (or 16 for N = 5), pass1_items 1 or 2, col_lanes 64 (or 32 "
+                "launch shape: chunk heights must be 8 (or 16 for N = 5; 64 in pass 1, whole columns, for the compact "
+                "metric and Nz <= 64), pass1_items 1 or 2, col_lanes 64 (or 32 "
                 "when Nz <= 32 without the Thomas solve), col_block a multiple of 64 in [64, 256], persistent 1 or "
                 "-1; a persistent launch takes chunk heights 8, pass1_items 1 and col_block = 64 * ceil(N*N*8 / 64)");
   graph_free(c);  // a captured graph keeps the old shapes
+  const int nzt = c->nzt, nzt1 = c->nzt1;
   apply_shape(c, sh);
-  if (shape->pass1_chunk_levels) c->col1 = c->p16 = 0;
-  if (shape->chunk_levels) c->r16 = 0;
+  if (!shape->chunk_levels) c->nzt = nzt;
+  if (!shape->pass1_chunk_levels) c->nzt1 = nzt1;
   return CGD_OK;
 }
 
@@ -1519,7 +1533,14 @@ extern "C" int cgd_autotune(cgd_ctx *c, double *V, double dt, const cgd_rw_work 
   double *Vsave = nullptr;
   hipEvent_t e0 = nullptr, e1 = nullptr;
   cgd_launch_shape best = current_shape(c);
+  const cgd_launch_shape entry = best;
+  const int entry_nzt = c->nzt, entry_nzt1 = c->nzt1;
   double bms = 1e300;
+  auto same = [](const cgd_launch_shape &x, const cgd_launch_shape &y) {
+    return x.chunk_levels == y.chunk_levels && x.pass1_chunk_levels == y.pass1_chunk_levels &&
+           x.pass1_items == y.pass1_items && x.col_lanes == y.col_lanes && x.col_block == y.col_block &&
+           x.persistent == y.persistent;
+  };
   auto run = [&]() -> int {
     HIPCHK(c, hipMalloc(&Vsave, n5 * sizeof(double)));
     HIPCHK(c, hipEventCreate(&e0));
@@ -1551,12 +1572,6 @@ extern "C" int cgd_autotune(cgd_ctx *c, double *V, double dt, const cgd_rw_work 
     // The shape the context had keeps its place unless another is faster by
     // more than 1 %: short timings rank shapes within that margin in either
     // order, and a switch on noise has cost more over long runs than it won.
-    const cgd_launch_shape entry = best;
-    auto same = [](const cgd_launch_shape &x, const cgd_launch_shape &y) {
-      return x.chunk_levels == y.chunk_levels && x.pass1_chunk_levels == y.pass1_chunk_levels &&
-             x.pass1_items == y.pass1_items && x.col_lanes == y.col_lanes && x.col_block == y.col_block &&
-             x.persistent == y.persistent;
-    };
     auto pick = [&](const std::vector<cgd_launch_shape> &cand, const cgd_launch_shape &keep) -> int {
       std::vector<double> tmin(cand.size(), 1e300);
       for (int sweep = 0; sweep < 2; ++sweep)
@@ -1578,24 +1593,22 @@ extern "C" int cgd_autotune(cgd_ctx *c, double *V, double dt, const cgd_rw_work 
       return CGD_OK;
     };
     // the element kernels' shapes jointly (both passes' chunk heights and
-    // the pass-1 items), then the column shape with the best of them
+    // the pass-1 items, which whole columns have none of), then the column
+    // shape with the best of them
     int rr;
     std::vector<cgd_launch_shape> cand;
     best.persistent = -1;  // the element and column sweeps time separate launches
+    const cgd_launch_shape ek = best;
     for (int z2 : {8, 16})
-      for (int z1 : {8, 16})
+      for (int z1 : {8, 16, 64})
         for (int it : {1, 2}) {
-          cgd_launch_shape sh = best;
+          cgd_launch_shape sh = ek;
           sh.chunk_levels = z2;
           sh.pass1_chunk_levels = z1;
           sh.pass1_items = it;
-          if (shape_ok(c, sh)) cand.push_back(sh);
+          if (shape_ok(c, sh) && (same(sh, ek) || z1 != 64 || it == 1)) cand.push_back(sh);
         }
-    {
-      cgd_launch_shape ek = entry;
-      ek.persistent = -1;
-      if ((rr = pick(cand, ek))) return rr;
-    }
+    if ((rr = pick(cand, ek))) return rr;
     const cgd_launch_shape b1 = best;
     cand.clear();
     for (int l : {64, 32})
@@ -1641,6 +1654,10 @@ extern "C" int cgd_autotune(cgd_ctx *c, double *V, double dt, const cgd_rw_work 
   if (e0) (void)hipEventDestroy(e0);
   if (e1) (void)hipEventDestroy(e1);
   apply_shape(c, best);
+  if (same(best, entry)) {  // (a persistent launch keeps the heights it stands in for)
+    c->nzt = entry_nzt;
+    c->nzt1 = entry_nzt1;
+  }
   c->prof = prof;
   if (r) return r;
   if (chosen) *chosen = best;

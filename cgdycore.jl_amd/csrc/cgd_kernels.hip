@@ -38,7 +38,7 @@
 #define CGD_NMETN 12 // compact layout: components stored once per element node
 
 struct KArgs {
-  int Nz, NumG, nzt;
+  int Nz, NumG;
   double Grav, Omega, Rd, Cpd, p0, kappa;
   double Rd_p0, eos_y, dpd_y;      // Rd/p0, 1/(1-kappa), kappa/(1-kappa)
   double Rd_Cpd;                   // Rd/Cpd

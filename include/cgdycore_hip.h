@@ -218,11 +218,15 @@ int cgd_ctx_info(const cgd_ctx *ctx, int *ncolor, int *chunk_levels, int *compac
 
 /* Launch shapes (no reference counterpart; the reference fixes its
  * workgroup shapes by NumberThreadGPU, src/DyCore/GlobalVariables.jl:240).
- * In cgd_set_launch_shape a field of 0 keeps the current value.  Until a chunk
- * height is set, the library may take whole columns or 16 levels instead of
- * the 8 it reports, by a rule on N, Nz and the metric; a height that is set
- * (8 included) is the one that runs.  The
- * workgroup sizes and pass1_items change no bit; the pass-2 chunk height
+ * In cgd_set_launch_shape a field of 0 keeps the current value.  A context
+ * starts with heights chosen by a rule on N, Nz, the metric and the size of
+ * the grid.  cgd_get_launch_shape reports the heights that run (chunk_levels:
+ * those of cgd_rw_step's tendency), and setting the reported shape, on this
+ * context or on another one for the same inputs, changes nothing.  A height
+ * that equals the chosen one stands for the whole choice (in the mixed mode
+ * the FP64 tendency of cgd_fcn may have another height than the steps', and
+ * tracers keep 8 levels); any other is the height of all of a pass's kernels.
+ * The workgroup sizes and pass1_items change no bit; the pass-2 chunk height
  * (chunk-interface w sums) and 32-lane columns (the compiler's fused
  * multiply-adds) change rounding only, within the FP64 parity bound.
  * persistent = 1 runs each RW stage of cgd_rw_step as ONE launch (both
@@ -232,13 +236,14 @@ int cgd_ctx_info(const cgd_ctx *ctx, int *ncolor, int *chunk_levels, int *compac
  * to the separate launches.  It takes the dry dynamics with the compact
  * metric (no tracers, hooks or kink smoothing), N = 4 or 5, Nz <= 64, chunk
  * heights 8, pass1_items 1 and col_block = 64*ceil(8*N*N/64); otherwise
- * CGD_ERR_UNSUPPORTED.  A barrier wait is bounded (250 ms): should the
+ * CGD_ERR_UNSUPPORTED.  Heights that the context chose give way to 8 while
+ * persistent is 1 and stand again afterwards; set heights must be 8.  A barrier wait is bounded (250 ms): should the
  * workgroups not all be resident (another process on the device), the
  * launch ends and cgd_check reports it.
  * Setting a shape drops a captured step graph. */
 typedef struct {
   int chunk_levels;       /* levels per workgroup of the fused tendency pass: 8, or 16 for N = 5 */
-  int pass1_chunk_levels; /* the same for the first (hyperviscosity) pass */
+  int pass1_chunk_levels; /* the same for the first (hyperviscosity) pass; 64: whole columns (compact metric, Nz <= 64) */
   int pass1_items;        /* (element, chunk) items per pass-1 workgroup: 1 or 2 (loads of both in flight) */
   int col_lanes;          /* lanes per column in the stage kernel: 64, or 32 (two columns per wavefront, Nz <= 32) */
   int col_block;          /* threads per stage workgroup: 64, 128, 192 or 256 */
@@ -255,7 +260,8 @@ int cgd_check(cgd_ctx *ctx, void *stream);
 /* Autotuner: times cgd_rw_step per candidate launch shape on the caller's V
  * and work buffers (per shape the fastest of three timings of reps steps,
  * over two sweeps through the candidates) and keeps the fastest: the
- * element-kernel shapes jointly (both chunk heights and pass1_items), then
+ * element-kernel shapes jointly (both chunk heights, whole columns of pass 1 and
+ * pass1_items), then
  * the column shape with the best of them, then separate launches against
  * one persistent launch per stage where the configuration allows it.  The context's shape on entry is
  * kept unless a candidate beats it by more than 1 %.  V, all components,

@@ -1,0 +1,159 @@
+"""Which kernels run: the shape that a context reports, sets and tunes names
+them (GPU, through the C ABI).  The kernels are read off torch's profiler.
+
+The layers are 512 m thick, so that the metric has the same bits at all levels
+(the compact layout, regular) at the level counts used here.
+"""
+import re
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def torch_cuda():
+    import torch
+
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    return torch
+
+
+def kernels_of(torch, fn):
+    """The names, without arguments, of the kernels that fn launches."""
+    from torch.profiler import ProfilerActivity, profile
+
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as prof:
+        fn()
+        torch.cuda.synchronize()
+    names = {re.sub(r"^void |\(.*", "", e.key) for e in prof.key_averages()}
+    return {n for n in names if n.startswith("k_")}
+
+
+class Case:
+    def __init__(self, pkg, torch, ne, p, nz, precision="fp64", ntr=0, thickness=512.0):
+        self.host, self.torch = pkg.host, torch
+        disc = pkg.discretization.build(ne, p, nz, thickness * nz)
+        self.phys = pkg.discretization.Phys()
+        self.dev = pkg.host.device_setup(disc, self.phys, device="cuda", precision=precision, NumTr=ntr)
+        self.ctx = pkg.host.init_context(self.dev[0], self.dev[1], self.phys, self.dev[2])
+        U0 = pkg.state.jet_state(disc, seed=1)
+        U0 = np.concatenate([U0] + [0.01 * (t + 1) * U0[0:1] for t in range(ntr)], axis=0)
+        self.U0 = torch.as_tensor(U0, device="cuda")
+
+    def step(self, n=1):
+        FE, Metric, Global, Cache, JCache = self.dev
+        V = self.U0.clone()
+        self.host.TimeStepper(V, 100.0, n, FE, Metric, self.phys, Cache, JCache, Global)
+        self.torch.cuda.synchronize()
+        return V
+
+    def kernels(self):
+        return {k for k in kernels_of(self.torch, self.step) if k.startswith(("k_fcn", "k_tr1", "k_tr2", "k_stage"))}
+
+
+def heights(shape):
+    return shape["chunk_levels"], shape["pass1_chunk_levels"]
+
+
+@pytest.mark.parametrize("ne,p,nz,precision,ntr,shape,names", [
+    (3, 4, 64, "fp64", 0, (16, 64), {"k_fcn1c<5, double>", "k_fcn2r<5, 16>"}),
+    (3, 4, 62, "fp64", 1, (16, 64), {"k_fcn1c<5, double>", "k_fcn2r<5, 16>", "k_tr1<5, 8, true>", "k_tr2<5, 8, true>"}),
+    (3, 4, 64, "mixed", 0, (8, 64), {"k_fcn1c<5, float>", "k_fcn2<5, 8, true, float, false>"}),
+    (3, 3, 48, "fp64", 0, (8, 64), {"k_fcn1c<4, double>", "k_fcn2r<4, 8>"}),
+    (19, 4, 32, "fp64", 0, (8, 16), {"k_fcn1<5, 16, true, double, 1>", "k_fcn2r<5, 8>"}),
+    (3, 4, 32, "fp64", 0, (8, 8), {"k_fcn1<5, 8, true, double, 1>", "k_fcn2r<5, 8>"}),
+    (3, 4, 72, "fp64", 0, (8, 8), {"k_fcn1<5, 8, true, double, 1>", "k_fcn2r<5, 8>"}),
+    (3, 4, 80, "mixed", 0, (16, 8), {"k_fcn1<5, 8, true, double, 1>", "k_fcn2r<5, 16>"}),
+    (3, 4, 50, "fp64", 0, (8, 8), {"k_fcn1<5, 8, false, double, 1>", "k_fcn2<5, 8, false, double, false>"}),
+])
+def test_shape_names_what_runs(pkg, torch_cuda, ne, p, nz, precision, ntr, shape, names):
+    """The reported heights are those of the kernels that run; setting the
+    reported shape, here or on a fresh context, changes neither; a height
+    that is set runs, and the reported shape brings the first ones back."""
+    print(f"shape ne={ne} p={p} nz={nz} {precision} NumTr={ntr}", flush=True)
+    c = Case(pkg, torch_cuda, ne, p, nz, precision, ntr)
+    first = c.ctx.launch_shape()
+    assert heights(first) == shape and c.ctx.info()[1] == shape[0]
+    assert c.kernels() == names
+    V = c.step(2)
+    c.ctx.set_launch_shape(**first)
+    assert c.ctx.launch_shape() == first and c.kernels() == names
+    assert torch_cuda.equal(c.step(2), V)
+    c.ctx.set_launch_shape(chunk_levels=8, pass1_chunk_levels=8)
+    if shape != (8, 8):
+        assert heights(c.ctx.launch_shape()) == (8, 8)
+        ran = c.kernels()
+        assert ran != names and not any(k.startswith("k_fcn1c") or ", 16" in k for k in ran)
+    c.ctx.set_launch_shape(**first)
+    assert c.ctx.launch_shape() == first and c.kernels() == names
+    d = Case(pkg, torch_cuda, ne, p, nz, precision, ntr)
+    d.ctx.set_launch_shape(**first)
+    assert d.ctx.launch_shape() == first and d.kernels() == names
+    assert torch_cuda.equal(d.step(2), V)
+
+
+def test_columns_refused(pkg, torch_cuda, monkeypatch):
+    """Whole columns need the compact metric and at most 64 levels."""
+    print("columns refused", flush=True)
+    for nz, metric, ok in ((64, "", True), (20, "", True), (72, "", False), (20, "full", False)):
+        monkeypatch.setenv("CGD_METRIC", metric)
+        c = Case(pkg, torch_cuda, 2, 4, nz)
+        if ok:
+            V = c.step(2)
+            c.ctx.set_launch_shape(pass1_chunk_levels=64)
+            assert "k_fcn1c<5, double>" in c.kernels()
+            assert torch_cuda.equal(c.step(2), V)
+        else:
+            with pytest.raises(pkg.host.CGDError):
+                c.ctx.set_launch_shape(pass1_chunk_levels=64)
+        with pytest.raises(pkg.host.CGDError):
+            c.ctx.set_launch_shape(chunk_levels=64)
+
+
+@pytest.mark.parametrize("ne,nz,precision", [(3, 64, "fp64"), (19, 32, "fp64"), (3, 64, "mixed")])
+def test_autotune_runs_its_candidates(pkg, torch_cuda, ne, nz, precision):
+    """Every height that the context admits is timed, and the chosen shape is
+    the one that runs, here and set on a fresh context."""
+    print(f"autotune candidates ne={ne} nz={nz} {precision}", flush=True)
+    c = Case(pkg, torch_cuda, ne, 4, nz, precision)
+    FE, Metric, Global, Cache, JCache = c.dev
+    got = {}
+    V = c.U0.clone()
+    ran = kernels_of(torch_cuda, lambda: got.update(s=c.ctx.autotune(V, 100.0, Cache, JCache, reps=1)))
+    R = "float" if precision == "mixed" else "double"
+    for z in (8, 16):
+        assert f"k_fcn1<5, {z}, true, {R}, 1>" in ran and f"k_fcn1<5, {z}, true, {R}, 2>" in ran
+        assert (f"k_fcn2<5, {z}, true, float, false>" if R == "float" else f"k_fcn2r<5, {z}>") in ran
+    assert f"k_fcn1c<5, {R}>" in ran
+    shape = got["s"][0]
+    assert c.ctx.launch_shape() == shape and torch_cuda.equal(V, c.U0)
+    names, V = c.kernels(), c.step(2)
+    d = Case(pkg, torch_cuda, ne, 4, nz, precision)
+    d.ctx.set_launch_shape(**shape)
+    assert d.ctx.launch_shape() == shape and d.kernels() == names
+    assert torch_cuda.equal(d.step(2), V)
+
+
+def test_persistent_stands_in_for_the_chosen_heights(pkg, torch_cuda):
+    """A persistent launch has chunks of 8 levels; the heights that the context
+    chose stand again when it is turned off, and set ones are refused."""
+    print("persistent heights", flush=True)
+    c = Case(pkg, torch_cuda, 3, 4, 64)
+    first = c.ctx.launch_shape()
+    c.ctx.set_launch_shape(persistent=1)
+    assert heights(c.ctx.launch_shape()) == (8, 8) and c.ctx.info()[1] == 8
+    assert c.kernels() == {"k_stage_persist<5, true, double, 64, true>"}
+    c.ctx.check_device()
+    c.ctx.set_launch_shape(persistent=-1)
+    assert c.ctx.launch_shape() == first
+    with pytest.raises(pkg.host.CGDError):
+        c.ctx.set_launch_shape(persistent=1, chunk_levels=16)
+    c = Case(pkg, torch_cuda, 3, 4, 32)
+    c.ctx.set_launch_shape(chunk_levels=16)
+    with pytest.raises(pkg.host.CGDError):
+        c.ctx.set_launch_shape(persistent=1)
+    assert c.ctx.launch_shape()["chunk_levels"] == 16
