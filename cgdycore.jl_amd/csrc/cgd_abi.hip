@@ -315,7 +315,7 @@ extern "C" int cgd_ctx_info(const cgd_ctx *c, int *ncolor, int *chunk_levels, in
   if (!c) return CGD_ERR_ARG;
   if (!c->ok) return CGD_ERR_STATE;
   if (ncolor) *ncolor = c->ncolor;
-  if (chunk_levels) *chunk_levels = c->persistent ? 8 : c->nzt;
+  if (chunk_levels) *chunk_levels = c->persistent ? 8 : tr_tend_nzt(c);
   if (compact_metric) *compact_metric = c->cm;
   return CGD_OK;
 }

@@ -210,8 +210,9 @@ int cgd_rw_run(cgd_ctx *ctx, double *V, double dt, const cgd_rw_work *work, int 
 
 /* The schedule and layout cgd_ctx_create chose: the number of element
  * colours (the order in which a node's contributions are summed), the level
- * chunk height of the element
- * kernels, and whether the metric is stored in the compact layout (every
+ * chunk height of the element kernels before the context's own choice of
+ * another one for some of them (which cgd_get_launch_shape reports), and
+ * whether the metric is stored in the compact layout (every
  * component except the terrain row dXdxI[3,1:2,:] identical across levels,
  * so stored once per element node).  No reference counterpart. */
 int cgd_ctx_info(const cgd_ctx *ctx, int *ncolor, int *chunk_levels, int *compact_metric);
