@@ -124,6 +124,10 @@ template <typename R> static int tend_nzt(const cgd_ctx *c) {
   if (c->nzt != c->rule_nzt) return c->nzt;
   return std::is_same<R, double>::value && c->r16 ? 16 : c->base_nzt;
 }
+// the levels between the interfaces whose w terms pass 2 leaves in d_f4x
+template <typename R> static int f4_nzt(const cgd_ctx *c) {
+  return std::is_same<R, double>::value && c->reg && !c->smooth ? 8 : tend_nzt<R>(c);
+}
 static int tr_cache_nzt(const cgd_ctx *c) { return c->nzt1 == c->rule_nzt1 || c->nzt1 == 64 ? c->base_nzt : c->nzt1; }
 static int tr_tend_nzt(const cgd_ctx *c) { return c->nzt == c->rule_nzt ? c->base_nzt : c->nzt; }
 static int nchunks(const cgd_ctx *c, int nzt) { return (c->Nz + nzt - 1) / nzt; }
@@ -756,10 +760,10 @@ static int ctx_build(cgd_ctx *c, const cgd_desc *ds, int nmem, hipStream_t st) {
   // Pass 1, where it can't take whole columns and the grid leaves the chip a few
   // rounds of workgroups (the height changes no bit there): a step of 32 grids
   // of 32 levels 1.5 % faster.
-  // Pass 2, whose rounding depends on the height, so that the rule must not
-  // depend on the grid's size (a grid in a batch and alone agree to the bit):
+  // Pass 2 on a regular metric, where the height changes no bit either:
   // nz = 64: 502 -> 487 us (ne = 30), 1900 -> 1856 (ne = 60), a step at ne <= 16
-  // within 1.5 % either way; at nz = 32 no faster, so from 48 levels on.
+  // within 1.5 % either way; a step at ne = 30 2 % faster at nz = 48, no slower
+  // at 62; at nz = 32 no faster, so from 48 levels on.
   const bool tall = c->N == 5 && !(((Nz + 7) / 8) & 1);
   const bool p16 = tall && c->cm && !col1 && (size_t)NF * ((Nz + 15) / 16) >= 4096;
   c->r16 = tall && Nz >= 48 && c->reg && !c->smooth;
@@ -1044,10 +1048,10 @@ static int run_fcn(cgd_ctx *c, R *F, const double *U, const R *UR, R *Temp1, con
     const R *F4x = reinterpret_cast<const R *>(c->d_f4x);
     if (has_hooks(c))
       hipLaunchKernelGGL((k_dss<R, true>), g, dim3(256), 0, st, c->ka, c->hooks, U, AuxG, E2, F4x, F, Fd,
-                         nchunks(c, tend_nzt<R>(c)), tend_nzt<R>(c));
+                         nchunks(c, f4_nzt<R>(c)), f4_nzt<R>(c));
     else
       hipLaunchKernelGGL((k_dss<R, false>), g, dim3(256), 0, st, c->ka, c->hooks, U, AuxG, E2, F4x, F, Fd,
-                         nchunks(c, tend_nzt<R>(c)), tend_nzt<R>(c));
+                         nchunks(c, f4_nzt<R>(c)), f4_nzt<R>(c));
     HIPCHK(c, hipGetLastError());
     ++launches;
   }
@@ -1254,8 +1258,8 @@ static int rw_step_fused(cgd_ctx *c, double *V, double dt, const cgd_rw_work *w,
     rw.k = is < 2 ? kR[is] : nullptr;  // k_3 is consumed in registers
     rw.P = (is < 2 || more) ? w->AuxG : nullptr;
     rw.F4x = reinterpret_cast<const R *>(c->d_f4x);
-    rw.nchunk = nchunks(c, tend_nzt<R>(c));
-    rw.nzt = tend_nzt<R>(c);
+    rw.nchunk = nchunks(c, f4_nzt<R>(c));
+    rw.nzt = f4_nzt<R>(c);
     rw.fac = dt * gamma;
     rw.invfac = 1.0 / rw.fac;
     rw.invfac2 = rw.invfac / rw.fac;

@@ -227,14 +227,16 @@ int cgd_ctx_info(const cgd_ctx *ctx, int *ncolor, int *chunk_levels, int *compac
  * that equals the chosen one stands for the whole choice (in the mixed mode
  * the FP64 tendency of cgd_fcn may have another height than the steps', and
  * tracers keep 8 levels); any other is the height of all of a pass's kernels.
- * The workgroup sizes and pass1_items change no bit; the pass-2 chunk height
- * (chunk-interface w sums) and 32-lane columns (the compiler's fused
+ * The workgroup sizes, pass 1's height and pass1_items change no bit; the pass-2
+ * chunk height (chunk-interface w sums; in FP64 not on the regular metric of
+ * flat uniform layers) and 32-lane columns (the compiler's fused
  * multiply-adds) change rounding only, within the FP64 parity bound.
  * persistent = 1 runs each RW stage of cgd_rw_step as ONE launch (both
  * tendency passes, then the column stage) whose
  * workgroups stay resident and meet at grid-wide barriers where the
- * separate launches have kernel boundaries; the results are bit-identical
- * to the separate launches.  It takes the dry dynamics with the compact
+ * separate launches have kernel boundaries; the results in FP64 are
+ * bit-identical to the separate launches with heights of 8 (on a regular
+ * metric with any heights).  It takes the dry dynamics with the compact
  * metric (no tracers, hooks or kink smoothing), N = 4 or 5, Nz <= 64, chunk
  * heights 8, pass1_items 1 and col_block = 64*ceil(8*N*N/64); otherwise
  * CGD_ERR_UNSUPPORTED.  Heights that the context chose give way to 8 while

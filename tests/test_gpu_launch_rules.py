@@ -157,3 +157,40 @@ def test_persistent_stands_in_for_the_chosen_heights(pkg, torch_cuda):
     with pytest.raises(pkg.host.CGDError):
         c.ctx.set_launch_shape(persistent=1)
     assert c.ctx.launch_shape()["chunk_levels"] == 16
+
+
+@pytest.mark.parametrize("p,nz", [(4, 64), (4, 62), (4, 57), (4, 48), (4, 20), (3, 48)])
+def test_heights_change_no_bit_of_a_regular_metric(pkg, torch_cuda, p, nz):
+    """On a regular metric the tendency and the steps have the same bits at
+    every height, and in persistent launches whichever heights the separate
+    ones have (57, 62, 20: ragged last chunks)."""
+    torch = torch_cuda
+    print(f"heights p={p} nz={nz}", flush=True)
+    c = Case(pkg, torch, 3, p, nz)
+    FE, Metric, Global, Cache, JCache = c.dev
+    eq = pkg.host.CompressibleShallow()
+    U = c.U0 + torch.randn(c.U0.shape, generator=torch.Generator("cuda").manual_seed(1), device="cuda",
+                           dtype=c.U0.dtype) * torch.tensor([0.0, 3.0, 3.0, 0.3, 0.0], device="cuda")[:, None, None]
+    U[3, :, -1] = 0.0
+    c.U0 = U
+
+    def results():
+        F = torch.empty_like(U)
+        pkg.host.FcnPrepareGPU(U, FE, Metric, c.phys, Cache, None, Global, None, eq)
+        pkg.host.FcnGPU(F, U, FE, Metric, c.phys, Cache, None, Global, None, eq)
+        return F, Cache.Temp1[:5].clone(), c.step(3)
+
+    want = results()
+    assert all(bool(torch.isfinite(x).all()) for x in want)
+    heights_ = [(8, 8)] + ([(16, 16), (8, 16), (16, 8)] if p == 4 else []) + [(8, 64)]
+    for z2, z1 in heights_:
+        c.ctx.set_launch_shape(chunk_levels=z2, pass1_chunk_levels=z1)
+        for v, (x, y) in enumerate(zip(results(), want)):
+            assert torch.equal(x, y), f"heights {z2}, {z1}, result {v}"
+    d = Case(pkg, torch, 3, p, nz)
+    d.U0 = U
+    d.ctx.set_launch_shape(persistent=1, col_block=((p + 1) ** 2 * 8 + 63) // 64 * 64)
+    assert torch.equal(d.step(3), want[2])
+    d.ctx.check_device()
+    d.ctx.set_launch_shape(persistent=-1)
+    assert torch.equal(d.step(3), want[2])
