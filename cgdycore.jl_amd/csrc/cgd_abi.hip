@@ -1117,7 +1117,7 @@ extern "C" int cgd_schur(cgd_ctx *c, double *k, double *v, const double *JRhoW, 
     launch_tall(c->Nz, [&](auto w) {
       constexpr int W = decltype(w)::value;
       hipLaunchKernelGGL(k_schur_tall<W>, dim3(c->NumG), dim3(W), 0, st, c->ka, k, v, JRhoW, JWRho, JWRhoTh, JRhoThW,
-                         tri, fac, invfac2, comp_tri);
+                         tri, fac, invfac2, comp_tri, c->thomas);
     });
   HIPCHK(c, hipGetLastError());
   if (c->ntr > 0) {
