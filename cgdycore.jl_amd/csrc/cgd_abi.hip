@@ -503,16 +503,10 @@ static int ctx_build(cgd_ctx *c, const cgd_desc *ds, int nmem, hipStream_t st) {
       for (int i = 0; i < NN; ++i) ccopy[fp[g32[(size_t)e * NN + i]]++] = e * NN + i;
     }
   }
-  // the same as fixed-width lists (an even number of entries, -1 past the
-  // last copy), per global node and per element node
+  // width of the fixed-width lists of the same (an even number)
   int mult = 4;
   for (int gn = 0; gn < NumG; ++gn) mult = std::max(mult, cptr[gn + 1] - cptr[gn]);
   const int cpw = (mult + 1) / 2 * 2;
-  std::vector<int> gcpy((size_t)NumG * cpw, -1), cpy((size_t)NF * NN * cpw, -1);
-  for (int gn = 0; gn < NumG; ++gn)
-    std::copy(ccopy.begin() + cptr[gn], ccopy.begin() + cptr[gn + 1], gcpy.begin() + (size_t)gn * cpw);
-  for (size_t i = 0; i < g32.size(); ++i)
-    std::copy_n(gcpy.begin() + (size_t)g32[i] * cpw, cpw, cpy.begin() + i * cpw);
   // numbering, bit 31 marking the first copy of each node
   std::vector<int> gslot = g32;
   for (int gn = 0; gn < NumG; ++gn)
@@ -552,8 +546,8 @@ static int ctx_build(cgd_ctx *c, const cgd_desc *ds, int nmem, hipStream_t st) {
   const int nchunk_max = (Nz + 7) / 8;
   HIPCHK(c, hipMalloc(&c->d_glob, gslot.size() * sizeof(int)));
   HIPCHK(c, hipMalloc(&c->d_clist, (size_t)NF * sizeof(int)));
-  HIPCHK(c, hipMalloc(&c->d_cpy, cpy.size() * sizeof(int)));
-  HIPCHK(c, hipMalloc(&c->d_gcpy, gcpy.size() * sizeof(int)));
+  HIPCHK(c, hipMalloc(&c->d_cpy, (size_t)NF * NN * cpw * sizeof(int)));
+  HIPCHK(c, hipMalloc(&c->d_gcpy, (size_t)NumG * cpw * sizeof(int)));
   HIPCHK(c, hipMalloc(&c->d_e1, npt * (5 + c->ntr) * sizeof(double)));
   HIPCHK(c, hipMalloc(&c->d_e2, npt * (5 + c->ntr) * sizeof(double)));
   HIPCHK(c, hipMalloc(&c->d_met, npt * CGD_NMET * sizeof(double)));
@@ -567,8 +561,9 @@ static int ctx_build(cgd_ctx *c, const cgd_desc *ds, int nmem, hipStream_t st) {
   HIPCHK(c, hipMemcpyAsync(c->d_ncopy, ccopy.data(), ccopy.size() * sizeof(int), hipMemcpyHostToDevice, st));
   HIPCHK(c, hipMemcpyAsync(c->d_glob, gslot.data(), gslot.size() * sizeof(int), hipMemcpyHostToDevice, st));
   HIPCHK(c, hipMemcpyAsync(c->d_clist, elist.data(), elist.size() * sizeof(int), hipMemcpyHostToDevice, st));
-  HIPCHK(c, hipMemcpyAsync(c->d_cpy, cpy.data(), cpy.size() * sizeof(int), hipMemcpyHostToDevice, st));
-  HIPCHK(c, hipMemcpyAsync(c->d_gcpy, gcpy.data(), gcpy.size() * sizeof(int), hipMemcpyHostToDevice, st));
+  hipLaunchKernelGGL(k_copy_lists, dim3(grid_for((size_t)NumG + (size_t)NF * NN, 256)), dim3(256), 0, st, c->d_nptr,
+                     c->d_ncopy, c->d_glob, NumG, NF * NN, cpw, c->d_gcpy, c->d_cpy);
+  HIPCHK(c, hipGetLastError());
   HIPCHK(c, hipMemcpyAsync(c->d_kvis, kvis.data(), kvis.size() * sizeof(double), hipMemcpyHostToDevice, st));
   if (c->horlimit) {
     const size_t nb = (size_t)c->ntr * NF * Nz;

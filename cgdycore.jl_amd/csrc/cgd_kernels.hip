@@ -2550,6 +2550,22 @@ __global__ void k_relayout_metric(const double *__restrict__ dXdxI, const double
   }
 }
 
+// The copies of each node, the list of global node g being
+// ncopy[nptr[g] .. nptr[g+1]), as fixed-width lists: gcpy[NumG][cpw] per global
+// node, cpy[NF*NN][cpw] per element node, -1 past the last copy.
+__global__ void k_copy_lists(const int *__restrict__ nptr, const int *__restrict__ ncopy, const int *__restrict__ glob,
+                             int NumG, int ne, int cpw, int *__restrict__ gcpy, int *__restrict__ cpy) {
+  const size_t n = (size_t)NumG + ne;
+  for (size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x; q < n; q += (size_t)gridDim.x * blockDim.x) {
+    const bool elem = q >= (size_t)NumG;
+    const size_t i = elem ? q - NumG : q;
+    const int g = elem ? glob[i] & 0x7fffffff : (int)q;
+    int *out = (elem ? cpy : gcpy) + i * cpw;
+    const int c0 = nptr[g], c1 = nptr[g + 1];
+    for (int r = 0; r < cpw; ++r) out[r] = c0 + r < c1 ? ncopy[c0 + r] : -1;
+  }
+}
+
 // Whether a compact metric is regular (cgd_pass2r_body.inc): flag[0] is set
 // to 1 where it is not.  metn: [NF][12][NN]; met: [NF][5][NN][Nz]; M:
 // [2][NumG][Nz].  Where it is, iMn[g] = 1 / (M1 + M2) (ms: that, per point).
