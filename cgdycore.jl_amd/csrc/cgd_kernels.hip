@@ -997,7 +997,7 @@ __global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64) __attribute__((a
     k_tr2(KArgs a, int nchunk, int ntr, const double *__restrict__ U, const double *__restrict__ E1,
           double *__restrict__ Cout, double *__restrict__ E2) {
   constexpr int NN = N * N;
-  static_assert(NZT >= 3 && NZT <= 16, "chunk heights 3..16 (the DPP neighbour reach is 2)");
+  static_assert(NZT >= 4 && NZT <= 16 && 64 % NZT == 0, "chunk heights 4, 8 or 16 (halo levels share registers)");
   extern __shared__ double smem[];
   double *Ds = smem, *DWs = Ds + NN;
   // fields 0, 1: uc, vc (all tracers); 2..5 and 6..9: C, c, and the
@@ -1066,7 +1066,7 @@ __global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64) __attribute__((a
   const bool hm1 = valid && has_lo && edge_m1, hm2 = valid && iz >= 2 && edge_m2;
   const bool hp1 = valid && has_hi && edge_p1, hp2 = valid && iz + 2 <= Nz - 1 && edge_p2;
   // (the lanes' lower and upper halo levels share registers: with chunks of at
-  // least 3 levels no lane has both)
+  // least 4 levels no lane has both: in one of 3 the middle one would)
   double hrho = 1, hu = 0, hv = 0, hw = 0, h31 = 0, h32 = 0, h33 = 0, hJ = 1, hrho2 = 1, hJ2 = 1;
   if (hm1 || hp1) {
     const unsigned uh = hm1 ? ui - 1 : ui + 1;
@@ -1293,6 +1293,7 @@ __global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64)
               double *__restrict__ E2) {
   constexpr int NN = N * N;
   static_assert(NN <= 32, "a 32-lane half of a wavefront holds the nodes of an element level");
+  static_assert(NZT >= 4 && NZT <= 16 && 64 % NZT == 0, "chunk heights 4, 8 or 16 (halo levels share registers)");
   extern __shared__ double smem[];
   double *Ds = smem;
   // tiles 0, 1: uc, vc; 2: c.  Then per (level, node), node fastest: J,
@@ -1385,7 +1386,7 @@ __global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64)
   const bool live0 = 2 * wave < NZT && lw0 < NZT && iz0 < Nz;
   const bool hm1 = valid && has_lo && edge_m1, hm2 = valid && iz >= 2 && edge_m2;
   const bool hp1 = valid && has_hi && edge_p1, hp2 = valid && iz + 2 <= Nz - 1 && edge_p2;
-  // (no lane of a chunk of at least 3 levels has a halo level on both sides)
+  // (no lane of a chunk of at least 4 levels has a halo level on both sides)
   const double rho1 = hm1 ? rho_m : rho_p, rho2 = hm2 ? rho_mm : rho_pp;
   // this level's tracer density and the halo levels', one tracer ahead
   double Trs_n = 0, q1n = 0, q2n = 0;
