@@ -74,6 +74,10 @@ struct cgd_ctx {
   int pgrid = 0;
   GridBar *d_bar = nullptr;
   long long bar_ticks = 0;
+  // the stream of the last call that used the context's own arrays (order_streams)
+  hipStream_t last = nullptr;
+  bool used = false;
+  hipEvent_t ev_last = nullptr;
   // captured step graph (cgd_rw_graph_create)
   hipStream_t gstream = nullptr;
   hipGraph_t graph = nullptr;
@@ -796,6 +800,7 @@ extern "C" int cgd_ctx_destroy(cgd_ctx *c) {
   // without touching the HIP runtime
   graph_free(c);
   if (c->gstream) (void)hipStreamDestroy(c->gstream);
+  if (c->ev_last) (void)hipEventDestroy(c->ev_last);
   for (void *p : {(void *)c->d_stencil, (void *)c->d_qmin, (void *)c->d_qmax})
     if (p) (void)hipFree(p);
   for (void *p : {(void *)c->d_glob, (void *)c->d_clist, (void *)c->d_cpy, (void *)c->d_gcpy,
@@ -973,6 +978,32 @@ extern "C" int cgd_prepare(cgd_ctx *c, const double *U, double *AuxG, void *stre
   return CGD_OK;
 }
 
+// Tendencies and steps use arrays of the context (the element copies, the
+// chunk-interface terms, the limiter's bounds): a call on another stream than
+// the last one waits for what that stream holds by then.  On one stream this
+// is a comparison.  Calls that are being captured are ordered by the capture's
+// owner; a last stream that no longer takes an event is waited for.
+static int order_streams(cgd_ctx *c, hipStream_t st) {
+  if (c->used && st == c->last) return CGD_OK;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  HIPCHK(c, hipStreamIsCapturing(st, &cap));
+  if (cap != hipStreamCaptureStatusNone) return CGD_OK;
+  if (c->used) {
+    if (!c->ev_last) HIPCHK(c, hipEventCreateWithFlags(&c->ev_last, hipEventDisableTiming));
+    hipError_t e = hipStreamIsCapturing(c->last, &cap);
+    if (e == hipSuccess && cap == hipStreamCaptureStatusNone) e = hipEventRecord(c->ev_last, c->last);
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      HIPCHK(c, hipDeviceSynchronize());
+    } else if (cap == hipStreamCaptureStatusNone) {
+      HIPCHK(c, hipStreamWaitEvent(st, c->ev_last, 0));
+    }
+  }
+  c->last = st;
+  c->used = true;
+  return CGD_OK;
+}
+
 static bool has_hooks(const cgd_ctx *c) { return c->hooks.forcing || c->hooks.damping || c->hooks.micro; }
 
 // The element copies of the pass-1 cache (FP32 mode: four FP32 components,
@@ -990,7 +1021,8 @@ template <typename R> static double *e1_theta(cgd_ctx *c) {
 template <typename R>
 static int run_fcn(cgd_ctx *c, R *F, const double *U, const R *UR, R *Temp1, const double *AuxG, hipStream_t st,
                    bool want_f) {
-  int r;
+  int r = order_streams(c, st);
+  if (r) return r;
   R *const E1 = reinterpret_cast<R *>(c->d_e1), *const E2 = reinterpret_cast<R *>(c->d_e2);
   double *const E1th = e1_theta<R>(c);
   prof_begin(c, st, 0);
@@ -1346,6 +1378,7 @@ static int rw_run(cgd_ctx *c, double *V, double dt, const cgd_rw_work *w, int ns
   if (!(dt > 0.0)) return fail(c, CGD_ERR_ARG, "cgd_rw_step: dt must be positive");
   if (nsteps < 1) return fail(c, CGD_ERR_ARG, "cgd_rw_run: nsteps must be positive");
   hipStream_t st = S(stream);
+  if ((r = order_streams(c, st))) return r;
   c->dtau = dt;  // Global.TimeStepper.dtauStage = dt (RosenbrockSchur.jl:9)
   // SSP-Knoth: a = alpha/Gamma, c = -inv(Gamma), m = Gamma'\b, gamma = 1
   const double A[3][3] = {{0, 0, 0}, {1.0, 0, 0}, {0.25, 0.25, 0}};
@@ -1514,6 +1547,7 @@ extern "C" int cgd_rw_graph_launch(cgd_ctx *c, void *stream) {
   int r = check(c);
   if (r) return r;
   if (!c->gexec) return fail(c, CGD_ERR_STATE, "cgd_rw_graph_launch: no captured step graph");
+  if ((r = order_streams(c, S(stream)))) return r;
   HIPCHK(c, hipGraphLaunch(c->gexec, S(stream)));
   return CGD_OK;
 }

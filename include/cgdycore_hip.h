@@ -23,7 +23,11 @@
  * cgd_rw_graph_launch) allocate nothing; only the set-up calls
  * (cgd_ctx_create*, cgd_autotune, cgd_rw_graph_create, cgd_profile_enable)
  * do.  A context is not thread-safe; calls on one context must be issued
- * from one host thread.
+ * from one host thread.  Tendencies and steps use arrays of the context:
+ * on several streams they run one after the other, in the order of the calls
+ * (a call waits for the work that the stream of the last one holds by then).
+ * Calls that a caller captures into graphs of its own are not ordered so;
+ * their replays must not overlap others of the context.
  */
 #ifndef CGDYCORE_HIP_H
 #define CGDYCORE_HIP_H
