@@ -151,7 +151,11 @@ int cgd_ctx_create(const cgd_desc *desc, cgd_ctx **ctx, void *stream);
  * NumG_0 + ... + NumG_{m-1} onward (and likewise k, AuxG, Temp1, the J
  * blocks).  Each member is coloured on its own and a node's contributions are
  * summed in its member's colour order, so a member's results are bit-identical
- * to those of a context built for it alone with the same launch shape.  No reference
+ * to those of a context built for it alone with the same launch shape, where the
+ * members' metrics are of one kind: all on flat uniform layers with the same
+ * bits at all levels, or none.  Otherwise the whole batch takes the kernels of
+ * the general metric, and a member has the bits of its own context with
+ * CGD_METRIC=full, which differ from its default ones by rounding.  No reference
  * counterpart (the reference steps one grid per process; batch variants of
  * the calls above, src/GPU/FcnGPU.jl:552 and src/Integration/RosenbrockSchur.jl:1). */
 int cgd_ctx_create_batch(const cgd_desc *members, int nmem, cgd_ctx **ctx, void *stream);
@@ -218,7 +222,8 @@ int cgd_rw_run(cgd_ctx *ctx, double *V, double dt, const cgd_rw_work *work, int 
  * another one for some of them (which cgd_get_launch_shape reports), and
  * whether the metric is stored in the compact layout (every
  * component except the terrain row dXdxI[3,1:2,:] identical across levels,
- * so stored once per element node).  No reference counterpart. */
+ * so stored once per element node; of a batch: that of every member).  The
+ * kernels of the layouts agree to rounding.  No reference counterpart. */
 int cgd_ctx_info(const cgd_ctx *ctx, int *ncolor, int *chunk_levels, int *compact_metric);
 
 /* Launch shapes (no reference counterpart; the reference fixes its
