@@ -194,3 +194,67 @@ def test_heights_change_no_bit_of_a_regular_metric(pkg, torch_cuda, p, nz):
     d.ctx.check_device()
     d.ctx.set_launch_shape(persistent=-1)
     assert torch.equal(d.step(3), want[2])
+
+
+def rel_l2(a, b):
+    return float(np.linalg.norm(np.ravel(a - b)) / np.linalg.norm(np.ravel(b)))
+
+
+@pytest.mark.parametrize("p,nz", [(4, 48), (4, 57), (4, 63), (3, 48), (3, 61)])
+def test_columns_against_the_oracle(pkg, oracle_mod, torch_cuda, p, nz):
+    """Pass 1 over whole columns of fewer levels than lanes: the caches and
+    tendencies in FP64 to 1e-12 relative L2 (a few dozen terms of 1.1e-16 each,
+    cancellation of up to 1e2), the mixed mode's steps to that mode's 1e-5."""
+    torch, host = torch_cuda, pkg.host
+    print(f"columns against the oracle p={p} nz={nz}", flush=True)
+    disc = pkg.discretization.build(2, p, nz, 512.0 * nz)
+    phys = pkg.discretization.Phys()
+    hd = host.hyperdiffusion_for(2)
+    orc = oracle_mod.Oracle(disc, phys, (hd, hd, hd))
+    c = Case(pkg, torch, 2, p, nz)
+    assert f"k_fcn1c<{p + 1}, double>" in c.kernels()
+    rng = np.random.default_rng(4)
+    U0 = c.U0.cpu().numpy()
+    U0[1:4] += np.array([5.0, 5.0, 0.5])[:, None, None] * rng.standard_normal(U0[1:4].shape)
+    U0[3][:, -1] = 0.0
+    FE, Metric, Global, Cache, _ = c.dev
+    U = torch.as_tensor(U0, device="cuda")
+    F = torch.empty_like(U)
+    eq = host.CompressibleShallow()
+    host.FcnPrepareGPU(U, FE, Metric, phys, Cache, None, Global, None, eq)
+    host.FcnGPU(F, U, FE, Metric, phys, Cache, None, Global, None, eq)
+    torch.cuda.synchronize()
+    Fo, T1o = orc.fcn(U0.copy(), orc.prepare(U0.copy()))
+    for v in range(5):
+        assert rel_l2(Cache.Temp1[v].cpu().numpy(), T1o[v]) <= 1e-12, f"Temp1[{v}]"
+        assert rel_l2(F[v].cpu().numpy(), Fo[v]) <= 1e-12, f"F{v + 1}"
+    m = Case(pkg, torch, 2, p, nz, "mixed")
+    assert f"k_fcn1c<{p + 1}, float>" in m.kernels()
+    Vo = m.U0.cpu().numpy().copy()
+    orc.rw_step(Vo, 100.0, 2)
+    V = m.step(2).cpu().numpy()
+    for v in range(5):
+        assert rel_l2(V[v], Vo[v]) <= 1e-5, f"mixed V{v + 1}"
+
+
+@pytest.mark.parametrize("nz,precision", [(70, "fp64"), (130, "fp64"), (70, "mixed")])
+def test_hooks_above_64_levels(pkg, oracle_mod, torch_cuda, nz, precision):
+    """Forcing and damping in the fused stage of columns taller than a
+    wavefront (FP64 in either mode), to 1e-12 relative L2 of the oracle."""
+    torch, host = torch_cuda, pkg.host
+    print(f"hooks above 64 levels nz={nz} {precision}", flush=True)
+    damping = (30000.0, 12000.0, 0.05)
+    disc = pkg.discretization.build(2, 3, nz, 30000.0)
+    phys = pkg.discretization.Phys()
+    FE, Metric, Global, Cache, JCache = host.device_setup(disc, phys, device="cuda", damping=damping, forcing=True,
+                                                          precision=precision)
+    hd = host.hyperdiffusion_for(2)
+    orc = oracle_mod.Oracle(disc, phys, (hd, hd, hd), damping=damping, forcing=host.held_suarez_param())
+    U0 = pkg.state.jet_state(disc, seed=6)
+    V = torch.as_tensor(U0, device="cuda").clone()
+    host.TimeStepper(V, 100.0, 2, FE, Metric, phys, Cache, JCache, Global)
+    torch.cuda.synchronize()
+    Vo = U0.copy()
+    orc.rw_step(Vo, 100.0, 2)
+    for v in range(5):
+        assert rel_l2(V[v].cpu().numpy(), Vo[v]) <= 1e-12, f"V{v + 1}"
