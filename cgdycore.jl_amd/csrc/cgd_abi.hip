@@ -118,11 +118,12 @@ static bool columns_ok(const cgd_ctx *c) { return c->cm && c->Nz <= 64; }
 // k_fcn1c: three tiles of whole columns, one of them FP64
 static size_t lds_fcn1c(const cgd_ctx *c, size_t r) { return (size_t)c->NN * 64 * (sizeof(double) + 2 * r); }
 
-// The heights that run.  A persistent launch has chunks of 8 levels.  A height
-// that is the context's own choice stands for all of that choice: in pass 2
-// the FP64 and the FP32 tendency's, each by its rule, and base_nzt for the
-// tracers' kernels; any other is the height of all of them.
-static int cache_nzt(const cgd_ctx *c) { return c->persistent ? 8 : c->nzt1; }
+// The heights that separate launches run (a persistent one has chunks of 8
+// levels, and so has pass 2 of a tendency called beside it).  A height that is
+// the context's own choice stands for all of that choice: in pass 2 the FP64
+// and the FP32 tendency's, each by its rule, and base_nzt for the tracers'
+// kernels; any other is the height of all of them.
+static int cache_nzt(const cgd_ctx *c) { return c->nzt1; }
 template <typename R> static int tend_nzt(const cgd_ctx *c) {
   if (c->persistent) return 8;
   if (c->nzt != c->rule_nzt) return c->nzt;

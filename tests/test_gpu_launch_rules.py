@@ -147,6 +147,11 @@ def test_persistent_stands_in_for_the_chosen_heights(pkg, torch_cuda):
     c.ctx.set_launch_shape(persistent=1)
     assert heights(c.ctx.launch_shape()) == (8, 8) and c.ctx.info()[1] == 8
     assert c.kernels() == {"k_stage_persist<5, true, double, 64, true>"}
+    FE, Metric, Global, Cache, _ = c.dev
+    F = torch_cuda.empty_like(c.U0)
+    fcn = lambda: pkg.host.FcnGPU(F, c.U0, FE, Metric, c.phys, Cache, None, Global, None,  # noqa: E731
+                                  pkg.host.CompressibleShallow())
+    assert "k_fcn1c<5, double>" in kernels_of(torch_cuda, fcn)  # a separate tendency
     c.ctx.check_device()
     c.ctx.set_launch_shape(persistent=-1)
     assert c.ctx.launch_shape() == first
