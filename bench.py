@@ -601,14 +601,16 @@ def main():
     Ne = sb["Ne"]
     ms_per_step = wall / args.steps * 1e3
     mpts = Ne * args.steps / wall / 1e6
-    # dominant kernel: fused tendency pass (k_fcn2r), 3 evaluations per step
+    # dominant kernel: fused tendency pass (k_fcn2r; k_fcn2 where the metric
+    # is not the same at all levels), 3 evaluations per step
+    kern = "k_fcn2r" if ctx.info()[2] else "k_fcn2"
     n_eval = 3 * args.steps
     p2_eval_s = p2_ms / 1e3 / n_eval
     achieved = sb["pass2"] / p2_eval_s / 1e9
     workload = f"rw_step_fp64_ne{args.ne}_p{args.p}_nz{args.nz}" + (f"_tr{args.ntr}" if args.ntr else "") + (
         "_lim" if args.horlimit else "")
-    traffic = measured_traffic("k_fcn2r", workload, sb["pass2"])
-    roofline = {"bound": "hbm", "kernel": "k_fcn2r (fused tendency pass)", "achieved": round(achieved, 1),
+    traffic = measured_traffic(kern, workload, sb["pass2"])
+    roofline = {"bound": "hbm", "kernel": f"{kern} (fused tendency pass)", "achieved": round(achieved, 1),
                 "peak": PEAK_HBM_GBS, "unit": "GB/s", "frac": round(achieved / PEAK_HBM_GBS, 4),
                 "traffic": traffic,
                 "algorithmic_bytes_per_eval": sb["pass2"], "launches_per_eval": p2_launch // max(n_eval, 1),
@@ -616,8 +618,8 @@ def main():
                 "step_roofline_frac": round(sb["step"] / (wall / args.steps) / 1e9 / PEAK_HBM_GBS, 4),
                 "pass_ms_per_step": {k: round(v[0] / nb, 4) for k, v in passes.items()}}
     # the committed kernel-trace summary of this workload: the same fraction
-    # from rocprofv3's average dispatch duration of the kernel
-    tr = trace_average("k_fcn2r", workload)
+    # from rocprofv3's average dispatch duration of the kernel at this height
+    tr = trace_average(f"{kern}<{args.p + 1}, {shape['chunk_levels']}", workload)
     if tr is not None:
         per_eval = roofline["launches_per_eval"] or 1
         roofline["trace"] = dict(tr, file=f"profiles/kernels_{workload}.json",

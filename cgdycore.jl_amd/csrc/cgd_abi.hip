@@ -750,20 +750,24 @@ static int ctx_build(cgd_ctx *c, const cgd_desc *ds, int nmem, hipStream_t st) {
     HIPCHK(c, hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev));
     c->bar_ticks = (long long)std::max(khz, 1000) * 250;  // 250 ms
   }
-  // Pass 1 over whole columns has a lane per level: at Nz = 64 it takes 127 us
-  // instead of 190 (ne = 30), at Nz = 40 the idle lanes make it 1 % slower
-  // than the chunks, so it is taken from three quarters of a wavefront on.
+  // Pass 1 over whole columns has a lane per level, so that it pays where most
+  // lanes have one.  Kernel times at ne = 30, p = 4, columns against 8-level
+  // chunks: nz = 64 115 against 178 us, 61 119 and 190, 57 118 and 184, 48 104
+  // and 131; nz = 32 94 and 88 (a step 1.1 % slower).  The steps at 48..64 gain
+  // 2 to 6 %.  (44 and 40 would gain too, 3.4 and 1.4 %; the line lies where it
+  // was drawn before they were timed.)
   const bool col1 = columns_ok(c) && Nz >= 48;
   // 16 levels per workgroup where that pads no more levels than 8 do (nz = 40,
   // padded to 48: pass 1 15 %, pass 2 25 % slower): 128-byte pieces of the
   // columns, and in pass 2 half the halo levels.
   // Pass 1, where it can't take whole columns and the grid leaves the chip a few
   // rounds of workgroups (the height changes no bit there): a step of 32 grids
-  // of 32 levels 1.5 % faster.
+  // of 32 levels 1.5 % faster, steps at ne = 20..45, nz = 9..32 0 to 2 %.
   // Pass 2 on a regular metric, where the height changes no bit either:
-  // nz = 64: 502 -> 487 us (ne = 30), 1900 -> 1856 (ne = 60), a step at ne <= 16
-  // within 1.5 % either way; a step at ne = 30 2 % faster at nz = 48, no slower
-  // at 62; at nz = 32 no faster, so from 48 levels on.
+  // steps with 16 against 8 levels, nz = 64: ne = 60 9.78 and 9.88 ms, ne = 30
+  // 2.451 and 2.498, ne = 16 0.725 and 0.720; ne = 30, nz = 48 1.959 and 1.999,
+  // 57 and 61 equal; ne = 20, nz = 80 1.623 and 1.634; at nz = 32 the kernel is no
+  // faster, so from 48 levels on.
   const bool tall = c->N == 5 && !(((Nz + 7) / 8) & 1);
   const bool p16 = tall && c->cm && !col1 && (size_t)NF * ((Nz + 15) / 16) >= 4096;
   c->r16 = tall && Nz >= 48 && c->reg && !c->smooth;
@@ -1016,7 +1020,8 @@ template <typename R> static double *e1_theta(cgd_ctx *c) {
 // Both tendency passes.  The dynamics' tendency ends as element copies in
 // d_e2; with want_f (cgd_fcn; U = UR, R = double) and wherever physics hooks
 // add to it, it is summed into F, and with want_f the cache into Temp1.
-// The tracers' tendencies and caches are summed in F and Temp1 either way.
+// The tracers' likewise (into F for the microphysics too; the steps sum them
+// in k_rw_tr).
 // U is the FP64 state; UR the state the R-typed terms read (U itself, or
 // its FP32 shadow).
 template <typename R>
@@ -1239,7 +1244,7 @@ static int launch_persist(cgd_ctx *c, int is, const RWStage<R> &rw, const double
 // tendency passes and one column kernel (Jacobian, tri, stage terms, Schur
 // solve, next state and its pressure; the first also stores Vn = V).  With
 // R = float (mixed precision) the FP32 tendency and its FP32 state shadow
-// share the fV work buffer and the FP32 cache sits in Temp1.
+// share the fV work buffer (the tendency only where hooks need its sums).
 template <typename R>
 static int rw_step_fused(cgd_ctx *c, double *V, double dt, const cgd_rw_work *w, hipStream_t st, double *const k[3],
                          const double A[3][3], const double Cc[3][3], const double Mw[3], double gamma, bool begin,

@@ -407,7 +407,7 @@ __device__ __forceinline__ void wave_lds_fence() {
 // twice the memory requests in flight (the kernel is latency-bound: its
 // waves mostly wait on memory).  nitems = elements x nchunk.
 // R is the arithmetic and storage type of the state it reads (U: the state,
-// or its FP32 shadow), of Temp1 and of the LDS tiles: double, or float in
+// or its FP32 shadow), of the cache it writes and of the LDS tiles: double, or float in
 // the mixed-precision mode.
 template <typename R> struct Pass1In {
   R S11, S12, S21, S22, Js, iMs;
@@ -607,9 +607,8 @@ __global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64) k_fcn1(KArgs a, 
 // element, one wavefront per row J of its nodes, lane = level, so a lane
 // holds the N nodes of its row.
 // - Every load and store is one node's column, a whole run of 8 Nz bytes; the
-//   chunked kernel's 64-byte pieces are what bounds it (724 us at ne = 60,
-//   nz = 64, all of it loads and stores); the same bytes in columns take
-//   450 us, this kernel 503 us.
+//   chunked kernel's 64-byte pieces are what bounds it: 711 us at ne = 60,
+//   nz = 64 in 8-level chunks, 669 in 16-level ones, 466 in columns.
 // - The derivatives along the row need no LDS, and the node's metric, the
 //   derivative matrices and the addresses are uniform (scalar registers);
 //   only the derivatives across the rows exchange values through LDS.
