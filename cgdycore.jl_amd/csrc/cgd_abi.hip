@@ -1126,10 +1126,14 @@ extern "C" int cgd_jac(cgd_ctx *c, double *JRhoW, double *JWRho, double *JWRhoTh
   return CGD_OK;
 }
 
-// f(std::integral_constant<int, W>) for the workgroup of a tall column
-template <typename F> static void launch_tall(int Nz, F f) {
-  if (Nz <= 128) f(std::integral_constant<int, 128>{});
-  else f(std::integral_constant<int, 256>{});
+// f(W, Thomas) as integral constants, W the workgroup of a tall column
+template <typename F> static void launch_tall(const cgd_ctx *c, F f) {
+  auto w = [&](auto th) {
+    if (c->Nz <= 128) f(std::integral_constant<int, 128>{}, th);
+    else f(std::integral_constant<int, 256>{}, th);
+  };
+  if (c->thomas) w(std::true_type{});
+  else w(std::false_type{});
 }
 
 extern "C" int cgd_schur(cgd_ctx *c, double *k, double *v, const double *JRhoW, const double *JWRho,
@@ -1147,10 +1151,11 @@ extern "C" int cgd_schur(cgd_ctx *c, double *k, double *v, const double *JRhoW, 
                        dim3((c->NumG + 3) / 4), dim3(256), 0, st, c->ka, k, v, JRhoW, JWRho, JWRhoTh, JRhoThW, tri,
                        fac, invfac2, comp_tri, c->thomas);
   else
-    launch_tall(c->Nz, [&](auto w) {
+    launch_tall(c, [&](auto w, auto th) {
       constexpr int W = decltype(w)::value;
-      hipLaunchKernelGGL(k_schur_tall<W>, dim3(c->NumG), dim3(W), 0, st, c->ka, k, v, JRhoW, JWRho, JWRhoTh, JRhoThW,
-                         tri, fac, invfac2, comp_tri, c->thomas);
+      constexpr bool TH = decltype(th)::value;
+      hipLaunchKernelGGL((k_schur_tall<W, TH>), dim3(c->NumG), dim3(W), 0, st, c->ka, k, v, JRhoW, JWRho, JWRhoTh,
+                         JRhoThW, tri, fac, invfac2, comp_tri);
     });
   HIPCHK(c, hipGetLastError());
   if (c->ntr > 0) {
@@ -1308,12 +1313,13 @@ static int rw_step_fused(cgd_ctx *c, double *V, double dt, const cgd_rw_work *w,
     prof_begin(c, st, 2);
     if (c->Nz > 64) {
       if constexpr (std::is_same<R, double>::value)
-        launch_tall(c->Nz, [&](auto w) {
+        launch_tall(c, [&](auto w, auto th) {
           constexpr int W = decltype(w)::value;
+          constexpr bool TH = decltype(th)::value;
           const dim3 g(c->NumG), b(W);
-          if (is == 0) hipLaunchKernelGGL((k_rw_stage_tall<0, W>), g, b, 0, st, c->ka, rw);
-          else if (is == 1) hipLaunchKernelGGL((k_rw_stage_tall<1, W>), g, b, 0, st, c->ka, rw);
-          else hipLaunchKernelGGL((k_rw_stage_tall<2, W>), g, b, 0, st, c->ka, rw);
+          if (is == 0) hipLaunchKernelGGL((k_rw_stage_tall<0, W, TH>), g, b, 0, st, c->ka, rw);
+          else if (is == 1) hipLaunchKernelGGL((k_rw_stage_tall<1, W, TH>), g, b, 0, st, c->ka, rw);
+          else hipLaunchKernelGGL((k_rw_stage_tall<2, W, TH>), g, b, 0, st, c->ka, rw);
         });
     } else if (c->colw == 32) launch_stage<R, 32>(c, is, rw, st);
     else launch_stage<R, 64>(c, is, rw, st);

@@ -2039,14 +2039,14 @@ __device__ __forceinline__ void sub_product(double &s, double &lo, double a, dou
 // rounding errors.  The reduction's rounding grows with the height, as the
 // layers get thin against fac: against an extended-precision solve it is ten
 // times that of the elimination in order, refined it is smaller than that.
-// With thomas, triSolve!'s recurrence in its order instead, by one thread in
-// LDS, as the Thomas branch of col_solve.
-template <int W>
-__device__ __forceinline__ double tall_solve(TallX<W> &X, double t0, double t1, double t2, double rhs, int n,
-                                             int thomas) {
+// With TH, triSolve!'s recurrence in its order instead, by one thread in LDS,
+// as the Thomas branch of col_solve (kernels of their own: as a branch it made
+// the stages 1 % slower).
+template <int W, bool TH>
+__device__ __forceinline__ double tall_solve(TallX<W> &X, double t0, double t1, double t2, double rhs, int n) {
   constexpr int S = W == 128 ? 7 : 8;
   static_assert(W == 1 << S, "one level per thread");
-  if (thomas) {
+  if constexpr (TH) {
     X.put(t0, t1, t2, rhs);
     double *p0 = X.q + X.ph * 4 * W, *p1 = p0 + W, *p2 = p1 + W, *pb = p2 + W;
     if (X.i == 0) {
@@ -2123,12 +2123,12 @@ __device__ __forceinline__ void tall_tri(TallX<W> &X, const JacBlocks &J, double
 }
 
 // SchurSolveGPU! (as k_schur_col)
-template <int W>
+template <int W, bool TH>
 __global__ void __launch_bounds__(W)
     k_schur_tall(KArgs a, double *__restrict__ k, double *__restrict__ v, const double *__restrict__ JRhoW,
                  const double *__restrict__ JWRho, const double *__restrict__ JWRhoTh,
                  const double *__restrict__ JRhoThW, double *__restrict__ tri, double fac, double invfac2,
-                 int comp_tri, int thomas) {
+                 int comp_tri) {
   __shared__ double lds[8 * W];
   TallX<W> X{lds, (int)threadIdx.x, 0};
   const int Nz = a.Nz, n = Nz - 1, i = X.i;
@@ -2167,7 +2167,7 @@ __global__ void __launch_bounds__(W)
     v4 = v4 / fac + J.wr1 * v1 + J.wr0 * v1p + J.wt1 * v5 + J.wt0 * v5p;
     v[c0 + 3 * vs] = v4;
   }
-  const double k4 = tall_solve(X, t0, t1, t2, v4, n, thomas);
+  const double k4 = tall_solve<W, TH>(X, t0, t1, t2, v4, n);
   X.put(k4, J.rw1, J.tw1, 0.0);
   const double k4m = X.get(0, -1, 0.0), rw1m = X.get(1, -1, 0.0), tw1m = X.get(2, -1, 0.0);
   if (lev) {
@@ -2190,7 +2190,7 @@ __global__ void __launch_bounds__(W)
 }
 
 // The Rosenbrock stage (as k_rw_stage), FP64
-template <int STAGE, int W>
+template <int STAGE, int W, bool TH>
 __global__ void __launch_bounds__(W) k_rw_stage_tall(KArgs a, RWStage<double> rw) {
   __shared__ double lds[8 * W];
   TallX<W> X{lds, (int)threadIdx.x, 0};
@@ -2247,7 +2247,7 @@ __global__ void __launch_bounds__(W) k_rw_stage_tall(KArgs a, RWStage<double> rw
   double rhs = 0.0;
   if (row)
     rhs = v[3] * rw.invfac + J.wr1 * v[0] + J.wr0 * X.get(0, 1, 0.0) + J.wt1 * v[4] + J.wt0 * X.get(1, 1, 0.0);
-  const double k4 = tall_solve(X, t0, t1, t2, rhs, n, rw.thomas);
+  const double k4 = tall_solve<W, TH>(X, t0, t1, t2, rhs, n);
   X.put(k4, J.rw1, J.tw1, 0.0);
   if (!lev) return;
   if (row) {
