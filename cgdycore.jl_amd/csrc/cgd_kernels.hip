@@ -1723,10 +1723,8 @@ __device__ __forceinline__ void col_tri(double jrw0, double jrw1, double jwr0, d
 
 // A J block's two entries of one interface: one 16-byte access where the
 // caller's arrays are aligned for it (A16), so that a wavefront's access is one
-// run instead of two of every other word.  With the solution stored and the J
-// blocks read past the cache (nothing here reads them again) k_schur_col takes
-// 184 us instead of 204 for 86402 columns of 64 levels, k_jac 94 instead of 97
-// (its stores past the cache: 107, and the solve that follows 172).
+// run instead of two of every other word: k_jac 94 us instead of 97 for 86402
+// columns of 64 levels.
 typedef double dbl2 __attribute__((ext_vector_type(2)));
 template <bool A16> __device__ __forceinline__ void store_pair(double *p, double x, double y) {
   if constexpr (A16) {
@@ -1736,9 +1734,25 @@ template <bool A16> __device__ __forceinline__ void store_pair(double *p, double
     p[1] = y;
   }
 }
-template <bool A16> __device__ __forceinline__ void load_pair(const double *p, double &x, double &y) {
+// NT: past the cache, for what nothing here reads again.  k_schur_col streams so
+// where the call is larger than the last-level cache (256 MB): 24 words a point,
+// 86402 columns of 64 levels 184 us instead of 204.  Where its arrays stay in the
+// cache from the call before it, a stream loses them: 24578 columns 60 us instead
+// of 50, 13826 34 instead of 28.
+template <bool NT> __device__ __forceinline__ double load_nt(const double *p) {
+  if constexpr (NT) return __builtin_nontemporal_load(p);
+  else return *p;
+}
+template <bool NT> __device__ __forceinline__ void store_nt(double x, double *p) {
+  if constexpr (NT) __builtin_nontemporal_store(x, p);
+  else *p = x;
+}
+template <bool A16, bool NT> __device__ __forceinline__ void load_pair(const double *p, double &x, double &y) {
   if constexpr (A16) {
-    const dbl2 v = __builtin_nontemporal_load(reinterpret_cast<const dbl2 *>(p));
+    const dbl2 *q = reinterpret_cast<const dbl2 *>(p);
+    dbl2 v;
+    if constexpr (NT) v = __builtin_nontemporal_load(q);
+    else v = *q;
     x = v.x;
     y = v.y;
   } else {
@@ -1755,7 +1769,7 @@ template <bool A16> __device__ __forceinline__ void load_pair(const double *p, d
 // solved by parallel cyclic reduction (default) or, with thomas != 0, by
 // the Thomas recurrence of triSolve! run wave-serially in the reference's
 // operation order (one useful lane per step, about 2.5x slower).
-template <bool A16>
+template <bool A16, bool NT>
 __global__ void __launch_bounds__(256) k_schur_col(KArgs a, double *__restrict__ k, double *__restrict__ v,
                                                    const double *__restrict__ JRhoW, const double *__restrict__ JWRho,
                                                    const double *__restrict__ JWRhoTh,
@@ -1771,10 +1785,10 @@ __global__ void __launch_bounds__(256) k_schur_col(KArgs a, double *__restrict__
   const size_t jb = (ig * (size_t)n + i) * 2, tb = (ig * (size_t)n + i) * 3;
   double jrw0 = 0, jrw1 = 0, jwr0 = 0, jwr1 = 0, jwt0 = 0, jwt1 = 0, jtw0 = 0, jtw1 = 0;
   if (row) {
-    load_pair<A16>(JRhoW + jb, jrw0, jrw1);
-    load_pair<A16>(JWRho + jb, jwr0, jwr1);
-    load_pair<A16>(JWRhoTh + jb, jwt0, jwt1);
-    load_pair<A16>(JRhoThW + jb, jtw0, jtw1);
+    load_pair<A16, NT>(JRhoW + jb, jrw0, jrw1);
+    load_pair<A16, NT>(JWRho + jb, jwr0, jwr1);
+    load_pair<A16, NT>(JWRhoTh + jb, jwt0, jwt1);
+    load_pair<A16, NT>(JRhoThW + jb, jtw0, jtw1);
   }
   double t0, t1, t2;
   if (comp_tri) {
@@ -1797,8 +1811,8 @@ __global__ void __launch_bounds__(256) k_schur_col(KArgs a, double *__restrict__
   double v1 = 0, v2 = 0, v3 = 0, v4 = 0, v5 = 0;
   if (lev) {
     v1 = v[c0 + i];
-    v2 = __builtin_nontemporal_load(&v[c0 + i + vs]);
-    v3 = __builtin_nontemporal_load(&v[c0 + i + 2 * vs]);
+    v2 = load_nt<NT>(&v[c0 + i + vs]);
+    v3 = load_nt<NT>(&v[c0 + i + 2 * vs]);
     v4 = v[c0 + i + 3 * vs];
     v5 = v[c0 + i + 4 * vs];
   }
@@ -1822,13 +1836,13 @@ __global__ void __launch_bounds__(256) k_schur_col(KArgs a, double *__restrict__
       v1 += jrw0 * k4 + jrw1m * k4m;
       v5 += jtw0 * k4 + jtw1m * k4m;
     }
-    __builtin_nontemporal_store(fac * v1, &k[c0 + i]);
-    __builtin_nontemporal_store(fac * v2, &k[c0 + i + vs]);
-    __builtin_nontemporal_store(fac * v3, &k[c0 + i + 2 * vs]);
-    __builtin_nontemporal_store(k4, &k[c0 + i + 3 * vs]);
-    __builtin_nontemporal_store(fac * v5, &k[c0 + i + 4 * vs]);
-    __builtin_nontemporal_store(v1, &v[c0 + i]);
-    __builtin_nontemporal_store(v5, &v[c0 + i + 4 * vs]);
+    store_nt<NT>(fac * v1, &k[c0 + i]);
+    store_nt<NT>(fac * v2, &k[c0 + i + vs]);
+    store_nt<NT>(fac * v3, &k[c0 + i + 2 * vs]);
+    store_nt<NT>(k4, &k[c0 + i + 3 * vs]);
+    store_nt<NT>(fac * v5, &k[c0 + i + 4 * vs]);
+    store_nt<NT>(v1, &v[c0 + i]);
+    store_nt<NT>(v5, &v[c0 + i + 4 * vs]);
   }
 }
 

@@ -263,3 +263,43 @@ def test_hooks_above_64_levels(pkg, oracle_mod, torch_cuda, nz, precision):
     orc.rw_step(Vo, 100.0, 2)
     for v in range(5):
         assert rel_l2(V[v].cpu().numpy(), Vo[v]) <= 1e-12, f"V{v + 1}"
+
+
+@pytest.mark.parametrize("shift", [0, 1])
+def test_column_solve_streams_on_large_grids(pkg, torch_cuda, shift):
+    """The column solve of 2^21 points and more streams past the cache; its
+    columns are those of a small grid with the same inputs, to the bit, with
+    J blocks that take 16-byte accesses and without."""
+    torch, host = torch_cuda, pkg.host
+    print(f"column streams shift={shift}", flush=True)
+    phys = pkg.discretization.Phys()
+    gen = torch.Generator("cuda").manual_seed(5)
+    solves, inputs = [], None
+    for ne in (25, 3):
+        FE, Metric, Global, Cache, JCache, _ = host.device_build(ne, 3, 64, 30000.0)
+        ctx = host.init_context(FE, Metric, phys, Global)
+        g, nz = Global.NumG, Global.Nz
+        assert (g * nz >= 1 << 21) == (ne == 25)
+        if inputs is None:
+            blocks = [1e-3 * torch.randn((g, nz - 1, 2), generator=gen, device="cuda", dtype=torch.float64)
+                      for _ in range(4)]
+            inputs = blocks, torch.randn((5, g, nz), generator=gen, device="cuda", dtype=torch.float64)
+        for name, J in zip(("JRhoW", "JWRho", "JWRhoTh", "JRhoThW"), inputs[0]):
+            buf = torch.zeros(J[:g].numel() + 1, device="cuda", dtype=torch.float64)[shift:]
+            setattr(JCache, name, buf[:J[:g].numel()].view(g, nz - 1, 2).copy_(J[:g]))
+        v = inputs[1][:, :g].clone()  # the solve overwrites its right-hand side
+        k = torch.zeros_like(v)
+        JCache.CompTri = True
+
+        def solve():
+            host.SchurSolveGPU(k, v, JCache, 1.0, Cache, Global)
+
+        names = kernels_of(torch, solve)
+        want = f"k_schur_col<{'false' if shift else 'true'}, {'true' if ne == 25 else 'false'}>"
+        assert names == {want}
+        solves.append((k, v, JCache.tri))
+        ctx.close()
+    small = solves[1][0].shape[1]
+    assert torch.isfinite(solves[0][0]).all()
+    assert torch.equal(solves[0][0][:, :small], solves[1][0]) and torch.equal(solves[0][1][:, :small], solves[1][1])
+    assert torch.equal(solves[0][2][:small], solves[1][2])
