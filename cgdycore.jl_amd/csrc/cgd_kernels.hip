@@ -773,8 +773,13 @@ __device__ __forceinline__ void fcn2_block(int item, const KArgs &a, int nchunk,
 #undef CGD_ITEM
 }
 
+// Waves per SIMD: what fits without spills, 4 in FP64 and 5 in FP32.  The kink-
+// smoothed flux (SM) takes 142 registers in the full layout: at 4 waves it
+// spilled 14 (2400 elements of 45 levels 376 us, 337 at 3 waves).  In the compact
+// layout 3 waves also hold the early halo levels and copies, 154 registers: 5400
+// elements of 64 levels 1009 us with 16 spilled at 4 waves, 897 at 3.
 template <int N, int NZT, bool CM, typename R, bool SM>
-__global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64) __attribute__((amdgpu_waves_per_eu(std::is_same<R, float>::value ? 5 : 4))) k_fcn2(KArgs a, int nchunk,
+__global__ void __launch_bounds__((N * N * NZT + 63) / 64 * 64) __attribute__((amdgpu_waves_per_eu(std::is_same<R, float>::value ? 5 : SM ? 3 : 4))) k_fcn2(KArgs a, int nchunk,
                                                const double *__restrict__ U, const R *__restrict__ UR,
                                                const R *__restrict__ C, const double *__restrict__ P,
                                                R *__restrict__ F, R *__restrict__ F4x,
